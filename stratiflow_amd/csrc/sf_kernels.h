@@ -114,9 +114,27 @@ template <typename T>
 hipError_t launch_x_c2r(const XTArgs<T>& a, int N1, int N2, hipStream_t s);
 template <typename T>
 hipError_t launch_x_r2c(const XTArgs<T>& a, int N1, int N2, hipStream_t s);
+// FP64 inner products (sf_fields.hip): one launch for up to DOT_MAX pairs,
+// results and then the sequence number of the call in pinned host memory
+constexpr int DOT_MAX = 4;
+constexpr int DOT_BLOCKS = 1024;  // blocks (partial sums) per pair
+struct DotResult {
+    double val[DOT_MAX];
+    unsigned long long seq;
+};
 template <typename T>
-hipError_t launch_dot(const cx<T>* a, const cx<T>* b, int A1, int A2, int N3, const T* w, double* partial,
-                      double* out, int slot, hipStream_t s);
+struct DotArgs {
+    const cx<T>* a[DOT_MAX];
+    const cx<T>* b[DOT_MAX];
+    const T* w[DOT_MAX];  // vertical weights of each pair
+    unsigned n, A1, N3;   // n = A1*A2*N3 values per field
+    double* partial;      // DOT_MAX * DOT_BLOCKS values
+    unsigned* ticket;     // zero between launches
+    DotResult* host;
+    unsigned long long seq;
+};
+template <typename T>
+hipError_t launch_dot(const DotArgs<T>& a, int pairs, hipStream_t s);
 template <typename T>
 hipError_t launch_maxabs(const T* f, size_t n, int N3, const T* add, double* partial, double* out, int slot,
                          hipStream_t s);
@@ -201,7 +219,7 @@ void fft_twiddles_plan(int n, int r1f, double* re, double* im);
 bool yfwd_tiles(int N2, int A1, int precision);
 int fft_first_radix(int n, int r1f);
 int max_rows_per_lane();
-// blocks (and so partial sums) of the two-pass FP64 reductions (dot, max-abs)
+// blocks (and so partial maxima) of the two-pass max-abs reduction
 int max_reduction_blocks();
 // modes per block of the modal kernels for M rows per lane
 int modal_modes_per_block(int M, int precision);

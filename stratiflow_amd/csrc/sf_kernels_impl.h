@@ -1641,67 +1641,9 @@ hipError_t launch_x_r2c(const XTArgs<T>& a, int N1, int N2, hipStream_t s) {
     }
 }
 
-// ---------------------------------------------------------------------------
-// FP64 inner product, InnerProd (Integration.h:117-146):
-//   sum_z w_z sum_modes c_m Re(a conj b),  c = 1 for mode (0,0), 2 otherwise.
-// Deterministic two-pass reduction.
-// ---------------------------------------------------------------------------
-constexpr int DOT_BLOCKS = 1024;
-
-template <typename T>
-__global__ __launch_bounds__(BS) void k_dot_partial(const cx<T>* __restrict__ a, const cx<T>* __restrict__ b,
-                                                    size_t n, int N3, int A1, const T* __restrict__ w,
-                                                    double* __restrict__ partial) {
-    __shared__ double red[BS];
-    double acc = 0;
-    for (size_t e = size_t(blockIdx.x) * BS + threadIdx.x; e < n; e += size_t(gridDim.x) * BS) {
-        const size_t rowz = e / size_t(A1);  // [ja][z][j1]
-        const int j1 = int(e - rowz * size_t(A1));
-        const int z = int(rowz % size_t(N3));
-        const bool m00 = (j1 == 0) && (rowz < size_t(N3));  // ja == 0 and j1 == 0
-        const cx<T> x = a[e], y = b[e];
-        const double re = double(x.x) * double(y.x) + double(x.y) * double(y.y);
-        acc += (m00 ? 1.0 : 2.0) * double(w[z]) * re;
-    }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-static __global__ __launch_bounds__(BS) void k_dot_final(const double* __restrict__ partial, int n, double* out, int slot) {
-    __shared__ double red[BS];
-    double acc = 0;
-    for (int i = threadIdx.x; i < n; i += BS) acc += partial[i];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[slot] = red[0];
-}
-
-template <typename T>
-hipError_t launch_dot(const cx<T>* a, const cx<T>* b, int A1, int A2, int N3, const T* w, double* partial,
-                      double* out, int slot, hipStream_t s) {
-    const size_t n = size_t(A1) * size_t(A2) * size_t(N3);
-    int blocks = int((n + BS - 1) / BS);
-    if (blocks > DOT_BLOCKS) blocks = DOT_BLOCKS;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL((k_dot_partial<T>), dim3(blocks), dim3(BS), 0, s, a, b, n, N3, A1, w, partial);
-    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(BS), 0, s, partial, blocks, out, slot);
-    return hipGetLastError();
-}
-
-#ifdef SF_KERNELS_HOST_DEFS
-int max_reduction_blocks() { return DOT_BLOCKS; }
-#endif
-
 // max |f + add[z]| over a nodal field (NodalField::Max, Field.h:771-786)
+constexpr int MAX_BLOCKS = 1024;
+
 template <typename T>
 __global__ __launch_bounds__(BS) void k_maxabs_partial(const T* __restrict__ f, size_t n, int N3,
                                                        const T* __restrict__ add, double* __restrict__ partial) {
@@ -1739,12 +1681,16 @@ template <typename T>
 hipError_t launch_maxabs(const T* f, size_t n, int N3, const T* add, double* partial, double* out, int slot,
                          hipStream_t s) {
     int blocks = int((n + BS - 1) / BS);
-    if (blocks > DOT_BLOCKS) blocks = DOT_BLOCKS;
+    if (blocks > MAX_BLOCKS) blocks = MAX_BLOCKS;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL((k_maxabs_partial<T>), dim3(blocks), dim3(BS), 0, s, f, n, N3, add, partial);
     hipLaunchKernelGGL(k_max_final, dim3(1), dim3(BS), 0, s, partial, blocks, out, slot);
     return hipGetLastError();
 }
+
+#ifdef SF_KERNELS_HOST_DEFS
+int max_reduction_blocks() { return MAX_BLOCKS; }
+#endif
 
 // y = a*x + b*y over n complex values (x may equal y)
 template <typename T>
@@ -1990,7 +1936,6 @@ hipError_t launch_diffprec(const DiffPrecArgs<T>& p, hipStream_t s) {
     template hipError_t launch_yfwd<T>(const YArgs<T>&, int, hipStream_t); \
     template hipError_t launch_x_c2r<T>(const XTArgs<T>&, int, int, hipStream_t); \
     template hipError_t launch_x_r2c<T>(const XTArgs<T>&, int, int, hipStream_t); \
-    template hipError_t launch_dot<T>(const cx<T>*, const cx<T>*, int, int, int, const T*, double*, double*, int, hipStream_t); \
     template hipError_t launch_axpby<T>(cx<T>*, T, const cx<T>*, T, size_t, hipStream_t); \
     template hipError_t launch_maxabs<T>(const T*, size_t, int, const T*, double*, double*, int, hipStream_t); \
     template hipError_t launch_ends<T>(cx<T>*, int, int, int, int, hipStream_t); \
