@@ -159,10 +159,13 @@ struct DiffPrecArgs {
 };
 template <typename T>
 hipError_t launch_diffprec(const DiffPrecArgs<T>& p, hipStream_t s);
-// the advected variant runs ADVPREC_MODES modes per block, each with N3 complex
-// values of LDS, within ADVPREC_LDS bytes
-constexpr int ADVPREC_MODES = 16;
-constexpr size_t ADVPREC_LDS = 64 * 1024;
+// tadv != 0 (sf_precond.hip), for columns of up to advprec_rows levels
+template <typename T>
+constexpr int advprec_rows() {
+    return sizeof(T) == 4 ? 512 : 256;
+}
+template <typename T>
+hipError_t launch_advprec(const DiffPrecArgs<T>& p, hipStream_t s);
 
 // adjoint step (sf_adjoint.hip)
 template <typename T>

@@ -64,3 +64,60 @@ def test_energies_follow_the_queue():
         u1, u3, b = (s.InnerProd(s.state(n), s.state(n)) for n in ("u1", "u3", "b"))
         assert ke == 0.5 * (u1 + u3) and pe == 0.1 * 0.5 * b
     s.close()
+
+
+@pytest.mark.parametrize("shape,prec", [((6, 1, 8, 1), 8), ((24, 1, 64, 1), 4), ((24, 1, 132, 1), 8),
+                                        ((24, 1, 256, 1), 8), ((24, 1, 260, 1), 4), ((24, 1, 384, 1), 4),
+                                        ((24, 1, 448, 1), 4), ((24, 1, 512, 1), 4), ((96, 48, 100, 0), 8),
+                                        ((128, 48, 36, 0), 8), ((128, 48, 64, 0), 4), ((128, 48, 256, 0), 8)])
+@pytest.mark.parametrize("bc", [sf.NEUMANN, sf.DIRICHLET])
+def test_advected_preconditioner(shape, prec, bc):
+    """The wavefront solver for every number of rows per lane, one and eight
+    modes per block, whole and ragged columns and blocks, against dense solves
+    of some modes; within the rounding that the systems' condition allows."""
+    s = solver(shape, prec)
+    N1, N2, N3, dim = shape
+    z, zf = s.vertical_points()
+    dy, dyf = np.ones(N3), np.ones(N3)
+    dy[1:], dyf[:-1] = np.diff(zf), np.diff(z)
+    f, a = random_field(s, bc, 4)
+    out = s.field(sf.MODAL, bc)
+    tnu, delta, tadv, kmax = 0.02, 0.3, 2.0, 9.0
+    print(shape, prec, bc, flush=True)
+    f.diffusion_precondition(out, tnu, delta, kmax, tadv)
+    o = out.download()
+    dirichlet = bc == sf.DIRICHLET
+    U = np.tanh(zf)
+    rng = np.random.default_rng(5)
+    A1 = N1 // 3
+    rows = list(range(N2 // 3)) + list(range(N2 - N2 // 3 + 1, N2)) if dim == 0 else [0]
+    modes = [(j2, j1) for j2 in rows for j1 in range(A1)]
+    picked = {modes[0], modes[-1]} | {modes[i] for i in rng.integers(0, len(modes), 10)}
+    for j2, j1 in picked:
+        kx = 0.44 * j1
+        ky = 2 * np.pi / (LX / 2) * (j2 if j2 <= N2 // 2 else j2 - N2) if dim == 0 else 0.0
+        if kx * kx + ky * ky > kmax * kmax:
+            assert np.array_equal(o[j2, j1], -a[j2, j1])
+            continue
+        A = np.eye(N3, dtype=np.complex128)
+        rhs = -a[j2, j1] / delta
+        ends = [0, 1, N3 - 2, N3 - 1] + ([2] if dirichlet else [])
+        rhs[ends] = 0
+        for j in range(1, N3 - 1):
+            if j in ends:
+                continue
+            if dirichlet:
+                lo, up = 1 / dyf[j - 1] / dy[j], 1 / dyf[j] / dy[j]
+            else:
+                lo, up = 1 / dy[j] / dyf[j], 1 / dy[j + 1] / dyf[j]
+            c = tnu / delta
+            A[j, j - 1], A[j, j + 1] = -c * lo, -c * up
+            A[j, j] = 1 - c * (-lo - up - kx * kx - ky * ky) + 1j * tadv * kx * U[j] / delta
+        if not dirichlet:
+            A[1, 2] = -1
+            A[N3 - 2, N3 - 3], A[N3 - 2, N3 - 2] = 1, -1
+        x = np.linalg.solve(A, rhs)
+        eps = np.finfo(np.float32 if prec == 4 else np.float64).eps
+        tol = 32 * eps * np.linalg.cond(A, np.inf) * np.abs(x).max() + 4 * eps * np.abs(a[j2, j1]).max()
+        assert np.abs(o[j2, j1] - (x - 0.5 * a[j2, j1])).max() <= tol, (j2, j1)
+    s.close()
