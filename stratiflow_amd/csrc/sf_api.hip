@@ -633,12 +633,43 @@ struct Ctx {
         }
     }
 
+    // modal fields src[i] (null: zero) copied to dst[i] (null: none) with the
+    // end conditions ends[i] (null: none) in one launch.  Each copy reads its
+    // source as it was before the call, so no source may be another copy's
+    // destination.
+    void copy_fields(int count, const V* const* src, V* const* dst, const int* ends = nullptr) {
+        CopyArgs<T> a{};
+        a.n = unsigned(nmodal);
+        a.A1 = unsigned(A1);
+        a.N3 = unsigned(N3);
+        int k = 0;
+        for (int i = 0; i < count; ++i) {
+            if (!dst[i]) continue;
+            a.src[k] = src[i];
+            a.dst[k] = dst[i];
+            a.ends[k++] = ends ? ends[i] : COPY_PLAIN;
+        }
+        if (k) check(launch_copy<T>(a, k, stream), "copy");
+    }
+    // whether copying src[i] to dst[i] one after the other is the same as all
+    // at once: no source is another copy's destination
+    static bool independent(int count, const void* const* src, const void* const* dst) {
+        for (int i = 0; i < count; ++i)
+            for (int j = 0; j < count; ++j)
+                if (i != j && src[i] && src[i] == dst[j]) return false;
+        return true;
+    }
+
     void populate_nodal() {
+        const V* from[4] = {nullptr};
+        V* to[4] = {nullptr};
         for (int i = 0; i < 4; ++i) {
             if (i == 1 && !three) continue;
             if (!snap[i]) snap[i] = dalloc<V>(nmodal);
-            SF_HIP(hipMemcpyAsync(snap[i], mf(SF_U1 + i), nmodal * sizeof(V), hipMemcpyDeviceToDevice, stream));
+            from[i] = mf(SF_U1 + i);
+            to[i] = snap[i];
         }
+        copy_fields(4, from, to);
         use_snap = true;
         to_nodal(mf(SF_U1), static_cast<T*>(state[SF_NODAL_U1].d));
         if (three) to_nodal(mf(SF_U2), static_cast<T*>(state[SF_NODAL_U2].d));
@@ -1806,14 +1837,23 @@ int sf_set_linear_background(sf_ctx* ctx, const sf_field* u1, const sf_field* u2
         with_ctx(ctx, [&](auto& C) {
             using T = typename std::remove_reference<decltype(C.h[0])>::type;
             const sf_field* src[4] = {u1, u2, u3, b};
+            const void* from[4];
+            const void* into[4];
+            const cx<T>* s[4];
+            cx<T>* d[4];
             for (int i = 0; i < 4; ++i) {
-                sf_field& d = C.state[SF_U1_TOT + i];
-                if (!src[i]) {
-                    SF_HIP(hipMemsetAsync(d.d, 0, d.n * sizeof(T), C.stream));
-                    continue;
-                }
-                SF_REQUIRE(src[i]->kind == SF_MODAL && src[i]->n == d.n, SF_ERR_ARG, "background must be modal");
-                SF_HIP(hipMemcpyAsync(d.d, src[i]->d, d.n * sizeof(T), hipMemcpyDeviceToDevice, C.stream));
+                const sf_field& st = C.state[SF_U1_TOT + i];
+                SF_REQUIRE(!src[i] || (src[i]->kind == SF_MODAL && src[i]->n == st.n), SF_ERR_ARG,
+                           "background must be modal");
+                from[i] = src[i] ? src[i]->d : nullptr;
+                into[i] = st.d;
+                s[i] = static_cast<const cx<T>*>(from[i]);
+                d[i] = C.mf(SF_U1_TOT + i);
+            }
+            if (C.independent(4, from, into)) {
+                C.copy_fields(4, s, d);
+            } else {
+                for (int i = 0; i < 4; ++i) C.copy_fields(1, s + i, d + i);
             }
         });
     });
@@ -1913,27 +1953,64 @@ int sf_state_bind(sf_ctx* ctx, const sf_field* u1, const sf_field* u2, const sf_
                   const sf_field* p) {
     SF_NULLCHK(ctx);
     const sf_field* src[5] = {u1, u2, u3, b, p};
-    for (int i = 0; i < 5; ++i) {
-        sf_field* st = nullptr;
-        int rc = sf_state_field(ctx, SF_U1 + i, &st);
-        if (rc == SF_OK) rc = src[i] ? sf_field_copy(st, src[i]) : sf_field_zero(st);
-        if (rc != SF_OK) return rc;
-    }
-    return SF_OK;
+    return guarded(ctx, [&]() {
+        with_ctx(ctx, [&](auto& C) {
+            using T = typename std::remove_reference<decltype(C.h[0])>::type;
+            const void* from[5];
+            const void* into[5];
+            for (int i = 0; i < 5; ++i) {
+                const sf_field& st = C.state[SF_U1 + i];
+                SF_REQUIRE(!src[i] || (same_shape(&st, src[i]) && st.bc == src[i]->bc), SF_ERR_ARG,
+                           "field shape/BC mismatch (Field.h:285)");
+                from[i] = src[i] ? src[i]->d : nullptr;
+                into[i] = st.d;
+            }
+            const bool once = C.independent(5, from, into);
+            const cx<T>* s[5];
+            cx<T>* d[5];
+            for (int i = 0; i < 5; ++i) {
+                s[i] = static_cast<const cx<T>*>(from[i]);
+                d[i] = C.mf(SF_U1 + i);
+                if (!once) C.copy_fields(1, s + i, d + i);
+            }
+            if (once) C.copy_fields(5, s, d);
+        });
+    });
 }
 
 int sf_state_fetch(sf_ctx* ctx, sf_field* u1, sf_field* u2, sf_field* u3, sf_field* b, sf_field* p) {
     SF_NULLCHK(ctx);
     sf_field* dst[5] = {u1, u2, u3, b, p};
-    for (int i = 0; i < 5; ++i) {
-        if (!dst[i]) continue;
-        sf_field* st = nullptr;
-        int rc = sf_state_field(ctx, SF_U1 + i, &st);
-        if (rc == SF_OK) rc = sf_field_copy(dst[i], st);
-        if (rc == SF_OK && i < 4) rc = sf_field_enforce_bcs(dst[i]);
-        if (rc != SF_OK) return rc;
-    }
-    return SF_OK;
+    return guarded(ctx, [&]() {
+        with_ctx(ctx, [&](auto& C) {
+            using T = typename std::remove_reference<decltype(C.h[0])>::type;
+            const void* from[5] = {nullptr};
+            const void* into[5] = {nullptr};
+            int ends[5];
+            for (int i = 0; i < 5; ++i) {
+                ends[i] = i == 4 ? COPY_PLAIN : (i == 2 ? COPY_DIRICHLET : COPY_NEUMANN);
+                if (!dst[i]) continue;
+                const sf_field& st = C.state[SF_U1 + i];
+                SF_REQUIRE(same_shape(dst[i], &st) && dst[i]->bc == st.bc, SF_ERR_ARG,
+                           "field shape/BC mismatch (Field.h:285)");
+                from[i] = st.d;
+                into[i] = dst[i]->d;
+            }
+            // a field fetched into the solver's own state, or two into one
+            // field, keep the order of the arguments
+            bool once = C.independent(5, from, into);
+            for (int i = 0; i < 5; ++i)
+                for (int j = 0; j < i; ++j) once = once && (!into[i] || into[i] != into[j]);
+            const cx<T>* s[5];
+            cx<T>* d[5];
+            for (int i = 0; i < 5; ++i) {
+                s[i] = static_cast<const cx<T>*>(from[i]);
+                d[i] = dst[i] ? static_cast<cx<T>*>(dst[i]->d) : nullptr;
+                if (!once) C.copy_fields(1, s + i, d + i, ends + i);
+            }
+            if (once) C.copy_fields(5, s, d, ends);
+        });
+    });
 }
 
 int sf_energy_f64(sf_ctx* ctx, double* ke, double* pe) { return sf_energy(ctx, ke, pe); }

@@ -1,5 +1,5 @@
 // sf_fields.hip -- whole-field kernels behind the StateVector algebra: FP64
-// inner products.
+// inner products and copies between states.
 #include "sf_kernels.h"
 
 namespace sf {
@@ -101,7 +101,63 @@ hipError_t launch_dot(const DotArgs<T>& a, int pairs, hipStream_t s) {
     return hipGetLastError();
 }
 
-#define SF_FIELDS_INST(T) template hipError_t launch_dot<T>(const DotArgs<T>&, int, hipStream_t);
+// ---------------------------------------------------------------------------
+// A state's fields copied in one launch (blockIdx.y = field): CopyToSolver,
+// CopyFromSolver with the end conditions of EnforceBCs (StateVector.h:415-421,
+// 511-543), the populated snapshot, SetBackground.  Moving a 2D field takes
+// less time than launching its copy, so five copies and four end-condition
+// passes cost nine launches' time; here one.  16 bytes per thread and load; the
+// level of an element is only needed where end conditions are.
+// ---------------------------------------------------------------------------
+template <typename T>
+__global__ __launch_bounds__(FB) void k_copy(CopyArgs<T> A) {
+    using V = cx<T>;
+    constexpr int NV = 16 / int(sizeof(V));  // values per thread and round
+    struct alignas(16) Pack {
+        V v[NV];
+    };
+    const int f = blockIdx.y;
+    const V* src = A.src[f];  // may be dst (no restrict)
+    V* dst = A.dst[f];
+    const int ends = A.ends[f];
+    const unsigned packs = A.n / NV, A1 = A.A1, N3 = A.N3;
+    for (unsigned i = blockIdx.x * FB + threadIdx.x; i < packs; i += gridDim.x * FB) {
+        Pack p;
+        if (src) {
+            p = reinterpret_cast<const Pack*>(src)[i];
+            if (ends != COPY_PLAIN) {
+#pragma unroll
+                for (int q = 0; q < NV; ++q) {
+                    const unsigned e = i * NV + q;
+                    const unsigned z = (e / A1) % N3;
+                    if (ends == COPY_NEUMANN) {
+                        if (z == 0) p.v[q] = src[e + A1];
+                        if (z == N3 - 1) p.v[q] = src[e - A1];
+                    } else if (z <= 2 || z >= N3 - 2) {
+                        p.v[q] = czero<V>();
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < NV; ++q) p.v[q] = czero<V>();
+        }
+        reinterpret_cast<Pack*>(dst)[i] = p;
+    }
+}
+
+template <typename T>
+hipError_t launch_copy(const CopyArgs<T>& a, int fields, hipStream_t s) {
+    if (fields < 1 || fields > COPY_MAX || a.n % 2 != 0) return hipErrorInvalidValue;
+    unsigned blocks = (a.n / (16 / unsigned(sizeof(cx<T>))) + FB - 1) / FB;
+    if (blocks > 2048) blocks = 2048;  // eight per CU
+    hipLaunchKernelGGL((k_copy<T>), dim3(blocks, fields), dim3(FB), 0, s, a);
+    return hipGetLastError();
+}
+
+#define SF_FIELDS_INST(T)                                                      \
+    template hipError_t launch_dot<T>(const DotArgs<T>&, int, hipStream_t);    \
+    template hipError_t launch_copy<T>(const CopyArgs<T>&, int, hipStream_t);
 
 SF_FIELDS_INST(float)
 SF_FIELDS_INST(double)

@@ -135,6 +135,18 @@ struct DotArgs {
 };
 template <typename T>
 hipError_t launch_dot(const DotArgs<T>& a, int pairs, hipStream_t s);
+// copies of up to COPY_MAX modal fields in one launch (sf_fields.hip)
+constexpr int COPY_MAX = 5;
+enum CopyEnds { COPY_PLAIN = 0, COPY_NEUMANN, COPY_DIRICHLET };  // end conditions put on the copy (EnforceBCs)
+template <typename T>
+struct CopyArgs {
+    const cx<T>* src[COPY_MAX];  // null: the copy is zero
+    cx<T>* dst[COPY_MAX];
+    int ends[COPY_MAX];
+    unsigned n, A1, N3;  // n = A1*A2*N3 values per field, even (N3 is)
+};
+template <typename T>
+hipError_t launch_copy(const CopyArgs<T>& a, int fields, hipStream_t s);
 template <typename T>
 hipError_t launch_maxabs(const T* f, size_t n, int N3, const T* add, double* partial, double* out, int slot,
                          hipStream_t s);

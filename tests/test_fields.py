@@ -121,3 +121,46 @@ def test_advected_preconditioner(shape, prec, bc):
         tol = 32 * eps * np.linalg.cond(A, np.inf) * np.abs(x).max() + 4 * eps * np.abs(a[j2, j1]).max()
         assert np.abs(o[j2, j1] - (x - 0.5 * a[j2, j1])).max() <= tol, (j2, j1)
     s.close()
+
+
+@pytest.mark.parametrize("prec", [4, 8])
+@pytest.mark.parametrize("shape", [(6, 1, 8, 1), (16, 1, 12, 1), (64, 1, 64, 1), (12, 6, 36, 0), (16, 12, 100, 0),
+                                   (192, 96, 64, 0)])
+def test_states_to_and_from_the_solver(shape, prec):
+    """CopyToSolver and CopyFromSolver in one launch: odd and even rows (two
+    FP32 values share a 16-byte access), each end condition, absent fields,
+    several rounds of blocks; the solver's fields as arguments keep the order
+    of the copies."""
+    s = solver(shape, prec)
+    names = ["u1", "u2", "u3", "b", "p"] if s.N2 > 1 else ["u1", "u3", "b", "p"]
+    bc = {n: sf.DIRICHLET if n == "u3" else sf.NEUMANN for n in names}
+    f, a = {}, {}
+    for i, n in enumerate(names):
+        f[n], a[n] = random_field(s, bc[n], 10 + i)
+    s.CopyToSolver(f["u1"], f.get("u2"), f["u3"], f["b"], f["p"])
+    out = {n: s.field(sf.MODAL, bc[n]) for n in names}
+    s.CopyFromSolver(out["u1"], out.get("u2"), out["u3"], out["b"], out["p"])
+    print(shape, prec, flush=True)
+    for n in names:
+        assert np.array_equal(s.get(n), a[n]), n
+        w = a[n].copy()
+        if n == "u3":
+            w[..., [0, 1, 2, -2, -1]] = 0
+        elif n != "p":
+            w[..., 0], w[..., -1] = w[..., 1], w[..., -2]
+        assert np.array_equal(out[n].download(), w), n
+    # p absent: zero; b bound to the solver's u1, which the first copy has replaced
+    s.CopyToSolver(f["b"], f.get("u2"), f["u3"], s.state("u1"))
+    assert np.array_equal(s.get("b"), a["b"]) and not s.get("p").any()
+    # two results in one field: the last one stays
+    s.CopyToSolver(f["u1"], f.get("u2"), f["u3"], f["b"], f["p"])
+    s.CopyFromSolver(out["u1"], None, out["u3"], out["u1"])
+    w = a["b"].copy()
+    w[..., 0], w[..., -1] = w[..., 1], w[..., -2]
+    assert np.array_equal(out["u1"].download(), w)
+    # the linearisation state
+    s.SetLinearBackground(f["u1"], None, f["u3"], f["b"])
+    assert np.array_equal(s.get("b_tot"), a["b"]) and not s.get("u2_tot").any()
+    s.SetLinearBackground(s.state("b_tot"), f["p"], f["u3"], s.state("u2_tot"))
+    assert np.array_equal(s.get("u1_tot"), a["b"]) and np.array_equal(s.get("b_tot"), a["p"])
+    s.close()
