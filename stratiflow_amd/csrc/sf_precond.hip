@@ -2,6 +2,8 @@
 // form, a real system, is k_diffprec in sf_kernels_impl.h).
 #include "sf_kernels.h"
 
+#include <type_traits>
+
 namespace sf {
 
 namespace {
@@ -106,7 +108,7 @@ __device__ __forceinline__ void ctri_solve(const T (&a)[M], const cx<T> (&b)[M],
 // coef = tnu/delta, adv = tadv kx/delta: strictly diagonally dominant for
 // delta > 0 but for the Neumannified rows.
 //
-// One wavefront per mode, MB modes of consecutive j1 per block.  A sweep down
+// FP64: one wavefront per mode, MB modes of consecutive j1 per block.  A sweep down
 // the column on one lane per mode is a chain of N3 dependent divisions and
 // global loads in each direction (182 us for a 256x1x256 FP64 field whatever
 // its number of modes); here the chain is M - 1 rows and six exchanges long.
@@ -191,6 +193,103 @@ __global__ __launch_bounds__(MB * 64) void k_advprec(DiffPrecArgs<T> P) {
     }
 }
 
+// FP32: a Thomas sweep per mode on one lane, which keeps the rounding of every
+// operation in its place (results of the wavefront form differ by 1e-7).  Its
+// chain is a complex division per row; what it needs from memory does not have
+// to be in that chain: the block stages its SWEEP_T columns and the
+// coefficient rows in LDS first and writes the result back at the end.
+constexpr int SWEEP_T = 8;  // modes per block: N3 = 512 takes 72 KB of LDS
+constexpr int SWEEP_BS = 64;
+template <typename T>
+__global__ __launch_bounds__(SWEEP_BS) void k_advprec_sweep(DiffPrecArgs<T> P) {
+    using V = cx<T>;
+    extern __shared__ unsigned char adv_lds[];
+    const int N = P.N3;
+    V* cp = reinterpret_cast<V*>(adv_lds);  // [z][SWEEP_T]: modified super-diagonal
+    V* dp = cp + N * SWEEP_T;               // [z][SWEEP_T]: input, then modified right-hand side
+    T* zl = reinterpret_cast<T*>(dp + N * SWEEP_T);  // sub-, main and super-diagonal of Dzz, U
+    const bool dir = P.dirichlet != 0;
+    const int lo = dir ? ZC_DZZD_LO : ZC_DZZN_LO;
+    const int ja = blockIdx.y, j10 = blockIdx.x * SWEEP_T;
+    for (int i = threadIdx.x; i < N * SWEEP_T; i += SWEEP_BS) {
+        const int z = i / SWEEP_T, j1 = j10 + i % SWEEP_T;
+        dp[i] = j1 < P.A1 ? P.in[sidx(ja, z, j1, N, P.A1)] : czero<V>();
+    }
+    for (int z = threadIdx.x; z < N; z += SWEEP_BS) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) zl[c * N + z] = P.zc[(lo + c) * P.N3p + z];
+        zl[3 * N + z] = P.zc[ZC_UBAR * P.N3p + z];
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    const int j1 = min(j10 + t, P.A1 - 1);
+    const T kk = P.kx2[j1], kl = P.ky2[ja];
+    if (t < SWEEP_T && !(-(kk + kl) > P.k2max)) {
+        const T coef = P.tnu / P.delta;
+        const T rs = T(-1) / P.delta;
+        const T adv = P.tadv * P.kx[j1] / P.delta;
+        // rows of (I - coef (Dzz - k^2) + i adv U) with the Neumannify/Dirichletify
+        // replacements of the implicit solves
+        auto rowc = [&](int j, T& a, V& b, T& c) {
+            a = -(coef * zl[j]);
+            b.x = T(1) - coef * ((zl[N + j] + kk) + kl);
+            b.y = adv * zl[3 * N + j];
+            c = -(coef * zl[2 * N + j]);
+            if (j == 0) a = 0;
+            if (j == N - 1) c = 0;
+            const bool id = dir ? (j <= 2 || j >= N - 2) : (j == 0 || j == N - 1);
+            if (id) {
+                a = 0;
+                b = mkc<T>(1, 0);
+                c = 0;
+            } else if (!dir && j == 1) {
+                a = 0;
+                b = mkc<T>(1, 0);
+                c = -1;
+            } else if (!dir && j == N - 2) {
+                a = 1;
+                b = mkc<T>(-1, 0);
+                c = 0;
+            }
+        };
+        auto rhs = [&](int j) {
+            const bool end = j <= 1 || j >= N - 2 || (dir && j == 2);
+            return end ? czero<V>() : cscale(rs, dp[j * SWEEP_T + t]);
+        };
+        auto cdiv = [](V a, V b) {
+            const T r = T(1) / (b.x * b.x + b.y * b.y);
+            return cscale(r, cmulc(a, b));
+        };
+        V cprev = czero<V>(), dprev = czero<V>();
+#pragma unroll 4
+        for (int j = 0; j < N; ++j) {
+            T a, c;
+            V b;
+            rowc(j, a, b, c);
+            const V den = csub(b, cscale(a, cprev));
+            const V cj = cdiv(mkc<T>(c, 0), den);
+            const V dj = cdiv(csub(rhs(j), cscale(a, dprev)), den);
+            cp[j * SWEEP_T + t] = cj;
+            dp[j * SWEEP_T + t] = dj;
+            cprev = cj;
+            dprev = dj;
+        }
+        V x = dprev;
+#pragma unroll 4
+        for (int j = N - 2; j >= 0; --j) {
+            x = csub(dp[j * SWEEP_T + t], cmul(cp[j * SWEEP_T + t], x));
+            dp[j * SWEEP_T + t] = x;
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < N * SWEEP_T; i += SWEEP_BS) {
+        const int z = i / SWEEP_T, j1 = j10 + i % SWEEP_T;
+        if (j1 >= P.A1) continue;
+        const size_t e = sidx(ja, z, j1, N, P.A1);
+        P.out[e] = -(P.kx2[j1] + kl) > P.k2max ? cscale(T(-1), P.in[e]) : csub(dp[i], cscale(T(0.5), P.in[e]));
+    }
+}
+
 template <typename T, int M>
 static void launch_advprec_m(const DiffPrecArgs<T>& p, hipStream_t s) {
     // up to four modes per CU the GPU is not filled by one mode per block
@@ -204,15 +303,23 @@ template <typename T>
 hipError_t launch_advprec(const DiffPrecArgs<T>& p, hipStream_t s) {
     if (p.A1 <= 0 || p.A2 <= 0 || p.in == p.out || !(p.delta > T(0)) || p.N3 > advprec_rows<T>())
         return hipErrorInvalidValue;
-    switch ((p.N3 + 63) / 64) {
-#define SF_M(m)                                                        \
-    case m:                                                            \
-        if constexpr (64 * m <= advprec_rows<T>()) launch_advprec_m<T, m>(p, s); \
-        break;
-        SF_M(1) SF_M(2) SF_M(3) SF_M(4) SF_M(5) SF_M(6) SF_M(7) SF_M(8)
-#undef SF_M
-        default:
-            return hipErrorInvalidValue;
+    if constexpr (std::is_same<T, float>::value) {
+        const size_t lds = size_t(p.N3) * (2 * SWEEP_T * sizeof(cx<T>) + 4 * sizeof(T));
+        if (lds > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_advprec_sweep<T>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL((k_advprec_sweep<T>), dim3((p.A1 + SWEEP_T - 1) / SWEEP_T, p.A2), dim3(SWEEP_BS), lds, s, p);
+    } else {
+        static_assert(advprec_rows<double>() == 256, "up to four rows per lane");
+        switch ((p.N3 + 63) / 64) {
+            case 1: launch_advprec_m<T, 1>(p, s); break;
+            case 2: launch_advprec_m<T, 2>(p, s); break;
+            case 3: launch_advprec_m<T, 3>(p, s); break;
+            case 4: launch_advprec_m<T, 4>(p, s); break;
+            default: return hipErrorInvalidValue;
+        }
     }
     return hipGetLastError();
 }
