@@ -94,6 +94,7 @@ struct Ctx {
     T* zc = nullptr;
     T *kx = nullptr, *ky = nullptr, *kx2 = nullptr, *ky2 = nullptr;
     V *tw1 = nullptr, *tw2 = nullptr;
+    V* twx = nullptr;  // of the whole-field x transforms
     V* tw1_r8 = nullptr;  // x twiddles of the plan with first radix 8 (made on first use)
     double* partial = nullptr;
     double* scal = nullptr;
@@ -202,6 +203,7 @@ struct Ctx {
         ky2 = dalloc<T>(A2);
         tw1 = dalloc<V>(2 * N1);
         tw2 = dalloc<V>(2 * N2);
+        twx = dalloc<V>(3 * N1 / 2);
         partial = dalloc<double>(DOT_MAX * DOT_BLOCKS);
         ticket = dalloc<unsigned>(1);
         scal = dalloc<double>(16);
@@ -322,19 +324,20 @@ struct Ctx {
         SF_HIP(hipMemcpyAsync(ky, hky.data(), A2 * sizeof(T), hipMemcpyHostToDevice, stream));
         SF_HIP(hipMemcpyAsync(ky2, hky2.data(), A2 * sizeof(T), hipMemcpyHostToDevice, stream));
         // FFT twiddles, computed in double
-        auto tw = [&](int n, V* dst) {
-            std::vector<double> re(2 * n), im(2 * n);
-            fft_twiddles(n, re.data(), im.data());
-            std::vector<V> w(2 * n);
-            for (int k = 0; k < 2 * n; ++k) {
+        auto tw = [&](void (*table)(int, double*, double*), int n, int entries, V* dst) {
+            std::vector<double> re(entries), im(entries);
+            table(n, re.data(), im.data());
+            std::vector<V> w(entries);
+            for (int k = 0; k < entries; ++k) {
                 w[k].x = T(re[k]);
                 w[k].y = T(im[k]);
             }
-            SF_HIP(hipMemcpyAsync(dst, w.data(), 2 * n * sizeof(V), hipMemcpyHostToDevice, stream));
+            SF_HIP(hipMemcpyAsync(dst, w.data(), entries * sizeof(V), hipMemcpyHostToDevice, stream));
             SF_HIP(hipStreamSynchronize(stream));
         };
-        tw(N1, tw1);
-        tw(N2, tw2);
+        tw(fft_twiddles, N1, 2 * N1, tw1);
+        tw(fft_twiddles, N2, 2 * N2, tw2);
+        tw(xt_twiddles, N1, 3 * N1 / 2, twx);
         SF_HIP(hipStreamSynchronize(stream));
     }
 
@@ -575,43 +578,47 @@ struct Ctx {
         check(launch_modal<T>(m, stream), "remove_divergence");
     }
 
-    // ModalField::ToNodal (Field.h:965-994)
-    void to_nodal(const V* modal, T* nodal) {
+    // ModalField::ToNodal (Field.h:965-994) of up to four fields (null: none)
+    void to_nodal(int count, const V* const* modal, T* const* nodal) {
         XTArgs<T> x{};
         x.N3 = N3;
         x.A1 = A1;
-        x.tw = tw1;
-        x.nodal_out = nodal;
+        x.tw = twx;
         x.scale = T(1);
-        x.nzt = 16;
+        YArgs<T> a{};
+        for (int i = 0; i < count; ++i) {
+            if (!nodal[i]) continue;
+            if (three) {
+                a.in[a.nf] = modal[i];
+                a.out[a.nf] = X[a.nf];
+                x.spec[x.nf] = X[a.nf++];
+            } else {
+                x.spec[x.nf] = const_cast<V*>(modal[i]);  // read
+            }
+            x.nodal[x.nf++] = nodal[i];
+        }
         if (three) {
-            YArgs<T> a{};
             a.N3 = N3;
             a.A1 = A1;
             a.A2 = A2;
-            a.nf = 1;
-            a.in[0] = modal;
-            a.out[0] = X[0];
             a.tw = tw2;
             a.scale = T(1);
             check(launch_yinv<T>(a, N2, stream), "to_nodal:y");
-            x.spec_in = X[0];
-        } else {
-            x.spec_in = modal;
         }
         check(launch_x_c2r<T>(x, N1, N2, stream), "to_nodal:x");
     }
+    void to_nodal(const V* modal, T* nodal) { to_nodal(1, &modal, &nodal); }
 
     // NodalField::ToModal (Field.h:734-769): scale 1/(N1*N2), keep active modes
     void to_modal(const T* nodal, V* modal) {
         XTArgs<T> x{};
         x.N3 = N3;
         x.A1 = A1;
-        x.tw = tw1;
-        x.nodal_in = nodal;
-        x.nzt = 16;
+        x.nf = 1;
+        x.tw = twx;
+        x.nodal[0] = const_cast<T*>(nodal);  // read
         if (three) {
-            x.spec_out = X[0];
+            x.spec[0] = X[0];
             x.scale = T(1);
             check(launch_x_r2c<T>(x, N1, N2, stream), "to_modal:x");
             YArgs<T> a{};
@@ -627,7 +634,7 @@ struct Ctx {
             a.scale = T(1.0 / (double(N1) * double(N2)));
             check(launch_yfwd<T>(a, N2, stream), "to_modal:y");
         } else {
-            x.spec_out = modal;
+            x.spec[0] = modal;
             x.scale = T(1.0 / double(N1));
             check(launch_x_r2c<T>(x, N1, N2, stream), "to_modal:x");
         }
@@ -671,10 +678,7 @@ struct Ctx {
         }
         copy_fields(4, from, to);
         use_snap = true;
-        to_nodal(mf(SF_U1), static_cast<T*>(state[SF_NODAL_U1].d));
-        if (three) to_nodal(mf(SF_U2), static_cast<T*>(state[SF_NODAL_U2].d));
-        to_nodal(mf(SF_U3), static_cast<T*>(state[SF_NODAL_U3].d));
-        to_nodal(mf(SF_B), static_cast<T*>(state[SF_NODAL_B].d));
+        refresh_nodal();
     }
 
     // the nodal fields U1..B as the reference holds them between calls: the
@@ -682,10 +686,13 @@ struct Ctx {
     // pending, else of the state (every stage ends with PopulateNodalVariables,
     // IMEXRK.cpp:8-24).  The step itself never writes them.
     void refresh_nodal() {
+        const V* from[4];
+        T* to[4];
         for (int i = 0; i < 4; ++i) {
-            if (i == 1 && !three) continue;
-            to_nodal(src(i), static_cast<T*>(state[SF_NODAL_U1 + i].d));
+            from[i] = src(i);
+            to[i] = has_field(i) ? static_cast<T*>(state[SF_NODAL_U1 + i].d) : nullptr;
         }
+        to_nodal(4, from, to);
     }
 
     // ---- adjoint step (IMEXRK.h:86-126) ----
@@ -784,9 +791,8 @@ struct Ctx {
                 bind_r();
             }
             // PopulateNodalVariables: the nodal fields follow the new state
-            for (int i = 0; i < 4; ++i)
-                if (has_field(i)) to_nodal(mf(SF_U1 + i), nod[i]);
             use_snap = false;
+            refresh_nodal();
             frac += h[k] / T(dt);
         }
     }
@@ -883,9 +889,10 @@ struct Ctx {
     double cfl() {
         // the reference reads whatever U1..U3 hold (IMEXRK.h:359-365): the
         // populated snapshot if one is pending, else the current state
-        to_nodal(src(0), static_cast<T*>(state[SF_NODAL_U1].d));
-        if (three) to_nodal(src(1), static_cast<T*>(state[SF_NODAL_U2].d));
-        to_nodal(src(2), static_cast<T*>(state[SF_NODAL_U3].d));
+        const V* from[3] = {src(0), src(1), src(2)};
+        T* to[3] = {static_cast<T*>(state[SF_NODAL_U1].d), three ? static_cast<T*>(state[SF_NODAL_U2].d) : nullptr,
+                    static_cast<T*>(state[SF_NODAL_U3].d)};
+        to_nodal(3, from, to);
         const double d1 = cfl_d[0], d2 = cfl_d[1], d3 = cfl_d[2];
         const T* ubar = zc + size_t(ZC_UBAR) * N3p;
         check(launch_maxabs<T>(static_cast<T*>(state[SF_NODAL_U1].d), nnodal, N3, ubar, partial, scal, 0, stream),

@@ -143,6 +143,16 @@ __device__ __forceinline__ void bst(V v, rsrc_t r, int voff, int soff = 0) {
 __device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double recip(double x) { return 1.0 / x; }
 
+// Workgroups go to the XCDs round-robin (block b to XCD b % 8), each XCD with
+// its own L2.  Blocks whose tiles share cache lines (neighbouring j1 tiles)
+// are renumbered so that they land on the same XCD at about the same time:
+// XCD x takes the x-th contiguous eighth of the tile sequence.
+__device__ __forceinline__ int xcd_tile(int b, int nb) {
+    constexpr int NXCD = 8;
+    if (nb % NXCD) return b;
+    return (b % NXCD) * (nb / NXCD) + b / NXCD;
+}
+
 // Per-z coefficient table rows (filled by the context set-up in sf_api.hip).
 enum ZCoef {
     ZC_DZZN_LO = 0,

@@ -20,6 +20,9 @@
 
 #include <cmath>
 
+// transform lengths the kernels are instantiated for
+#define SF_SIZES(X) X(6) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
+
 namespace sf {
 
 // ---- compile-time cos(2*pi*m/R) -------------------------------------------

@@ -69,15 +69,14 @@ __host__ __device__ inline size_t ytile_idx(int n2, int z, int j1, int N2, int A
     return ((size_t(z) * size_t(A1 >> 4) + size_t(j1 >> 4)) * size_t(N2) + size_t(n2)) * 16 + size_t(j1 & 15);
 }
 
-// Single-field x transforms between nodal and x-spectral layouts.
+// x transforms of nf fields between nodal and x-spectral layouts.
+constexpr int XT_MAX = 12;
 template <typename T>
 struct XTArgs {
-    int N3, A1, nzt;
-    const cx<T>* spec_in;
-    cx<T>* spec_out;
-    const T* nodal_in;
-    T* nodal_out;
-    const cx<T>* tw;
+    int N3, A1, nf;
+    cx<T>* spec[XT_MAX];
+    T* nodal[XT_MAX];
+    const cx<T>* tw;  // xt_twiddles
     T scale;
 };
 
@@ -233,6 +232,8 @@ void fft_twiddles_plan(int n, int r1f, double* re, double* im);
 // as contiguous runs (A1 a multiple of 16 and k_yfwd_seq's LDS tile fits)
 bool yfwd_tiles(int N2, int A1, int precision);
 int fft_first_radix(int n, int r1f);
+// the table of the whole-field x transforms: 3n/2 entries
+void xt_twiddles(int n, double* re, double* im);
 int max_rows_per_lane();
 // blocks (and so partial maxima) of the two-pass max-abs reduction
 int max_reduction_blocks();

@@ -455,16 +455,6 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
     store(A.p, pp);
 }
 
-// Workgroups go to the XCDs round-robin (block b to XCD b % 8), each XCD with
-// its own L2.  Blocks whose tiles share cache lines (neighbouring j1 tiles)
-// are renumbered so that they land on the same XCD at about the same time:
-// XCD x takes the x-th contiguous eighth of the tile sequence.
-__device__ __forceinline__ int xcd_tile(int b, int nb) {
-    constexpr int NXCD = 8;
-    if (nb % NXCD) return b;
-    return (b % NXCD) * (nb / NXCD) + b / NXCD;
-}
-
 template <typename T, int M, bool FULL, int MB>
 __global__ __launch_bounds__(MB * 64) void k_modal(ModalArgs<T> A) {
     __shared__ cx<T> tile[64 * M * (MB + 1)];
@@ -640,8 +630,6 @@ int max_rows_per_lane() { return MODAL_MAX_M; }
 // separate halo pass is needed.  The inverse transform uses
 // ifft(x) = conj(fft(conj(x))), so both directions share the forward kernel.
 // ---------------------------------------------------------------------------
-#define SF_SIZES(X) X(6) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
-
 #ifdef SF_KERNELS_HOST_DEFS
 bool tz_supported(int n) {
     switch (n) {
@@ -1531,116 +1519,6 @@ bool yfwd_tiles(int N2, int A1, int precision) {
 }
 #endif
 
-// ---------------------------------------------------------------------------
-// single-field x transforms (ToNodal / ToModal for API fields), one block per
-// (range of nzt z levels, n2)
-// ---------------------------------------------------------------------------
-template <typename T, int N1, int NL>
-__global__ __launch_bounds__(BS) void k_x_c2r(XTArgs<T> A) {
-    using V = cx<T>;
-    constexpr int LDP = fft_ldp<N1>();
-    __shared__ V buf[NL * LDP];
-    const int n2 = blockIdx.y;
-    const int N3 = A.N3, A1 = A.A1;
-    for (int z0 = blockIdx.x * A.nzt; z0 < min(N3, (int(blockIdx.x) + 1) * A.nzt); z0 += NL) {
-        const int nband = N1 - 2 * A1 + 1;
-        for (int idx = threadIdx.x; idx < NL * nband; idx += BS)
-            buf[(idx / nband) * LDP + (A1 + idx % nband)] = czero<V>();
-        for (int idx = threadIdx.x; idx < NL * A1; idx += BS) {
-            const int j1 = idx % A1;
-            const int t = idx / A1;
-            const int z = z0 + t;
-            V X = czero<V>();
-            if (z < N3) X = A.spec_in[sidx(n2, z, j1, N3, A1)];
-            V* L = buf + t * LDP;
-            if (j1 == 0) {
-                L[(0)] = mkc<T>(X.x, T(0));
-            } else {
-                L[(j1)] = X;
-                L[(N1 - j1)] = mkc<T>(X.x, -X.y);
-            }
-        }
-        sync_lds();
-        lds_fft<T, N1, NL, BS, +1>(buf, A.tw);
-        for (int idx = threadIdx.x; idx < NL * N1; idx += BS) {
-            const int t = idx % NL;
-            const int n = idx / NL;
-            const int z = z0 + t;
-            if (z < N3) A.nodal_out[(size_t(n2) * N1 + n) * N3 + z] = buf[t * LDP + (n)].x;
-        }
-        sync_lds();
-    }
-}
-
-template <typename T, int N1, int NL>
-__global__ __launch_bounds__(BS) void k_x_r2c(XTArgs<T> A) {
-    using V = cx<T>;
-    constexpr int LDP = fft_ldp<N1>();
-    __shared__ V buf[NL * LDP];
-    const int n2 = blockIdx.y;
-    const int N3 = A.N3, A1 = A.A1;
-    for (int z0 = blockIdx.x * A.nzt; z0 < min(N3, (int(blockIdx.x) + 1) * A.nzt); z0 += NL) {
-        for (int idx = threadIdx.x; idx < NL * N1; idx += BS) {
-            const int t = idx % NL;
-            const int n = idx / NL;
-            const int z = z0 + t;
-            V v = czero<V>();
-            if (z < N3) v.x = A.nodal_in[(size_t(n2) * N1 + n) * N3 + z];
-            buf[t * LDP + (n)] = v;
-        }
-        sync_lds();
-        lds_fft<T, N1, NL, BS, -1>(buf, A.tw);
-        for (int idx = threadIdx.x; idx < NL * A1; idx += BS) {
-            const int k = idx % A1;
-            const int t = idx / A1;
-            const int z = z0 + t;
-            if (z < N3) A.spec_out[sidx(n2, z, k, N3, A1)] = cscale(A.scale, buf[t * LDP + (k)]);
-        }
-        sync_lds();
-    }
-}
-
-template <typename T, int N1>
-static hipError_t launch_xt_n(const XTArgs<T>& a, int N2, bool c2r, hipStream_t s) {
-    // z levels per LDS batch (a block sweeps a.nzt levels): 16 levels make the
-    // nodal side's z runs 16 values long (4 levels: 115.5 -> 100.5 us for one
-    // 384x192x384 FP32 field)
-    constexpr int NL = 16;
-    XTArgs<T> b = a;
-    if (b.nzt % NL) b.nzt = ((b.nzt + NL - 1) / NL) * NL;
-    dim3 grid((a.N3 + b.nzt - 1) / b.nzt, N2);
-    if (c2r)
-        hipLaunchKernelGGL((k_x_c2r<T, N1, NL>), grid, dim3(BS), 0, s, b);
-    else
-        hipLaunchKernelGGL((k_x_r2c<T, N1, NL>), grid, dim3(BS), 0, s, b);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_x_c2r(const XTArgs<T>& a, int N1, int N2, hipStream_t s) {
-    switch (N1) {
-#define SF_CASE(n) \
-    case n:        \
-        return launch_xt_n<T, n>(a, N2, true, s);
-        SF_SIZES(SF_CASE)
-#undef SF_CASE
-        default:
-            return hipErrorInvalidValue;
-    }
-}
-template <typename T>
-hipError_t launch_x_r2c(const XTArgs<T>& a, int N1, int N2, hipStream_t s) {
-    switch (N1) {
-#define SF_CASE(n) \
-    case n:        \
-        return launch_xt_n<T, n>(a, N2, false, s);
-        SF_SIZES(SF_CASE)
-#undef SF_CASE
-        default:
-            return hipErrorInvalidValue;
-    }
-}
-
 // max |f + add[z]| over a nodal field (NodalField::Max, Field.h:771-786)
 constexpr int MAX_BLOCKS = 1024;
 
@@ -1848,8 +1726,6 @@ hipError_t launch_diffprec(const DiffPrecArgs<T>& p, hipStream_t s) {
     template hipError_t launch_xpass<T>(const XArgs<T>&, int, int, bool, hipStream_t); \
     template hipError_t launch_yinv<T>(const YArgs<T>&, int, hipStream_t); \
     template hipError_t launch_yfwd<T>(const YArgs<T>&, int, hipStream_t); \
-    template hipError_t launch_x_c2r<T>(const XTArgs<T>&, int, int, hipStream_t); \
-    template hipError_t launch_x_r2c<T>(const XTArgs<T>&, int, int, hipStream_t); \
     template hipError_t launch_axpby<T>(cx<T>*, T, const cx<T>*, T, size_t, hipStream_t); \
     template hipError_t launch_maxabs<T>(const T*, size_t, int, const T*, double*, double*, int, hipStream_t); \
     template hipError_t launch_ends<T>(cx<T>*, int, int, int, int, hipStream_t); \

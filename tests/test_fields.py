@@ -164,3 +164,35 @@ def test_states_to_and_from_the_solver(shape, prec):
     s.SetLinearBackground(s.state("b_tot"), f["p"], f["u3"], s.state("u2_tot"))
     assert np.array_equal(s.get("u1_tot"), a["b"]) and np.array_equal(s.get("b_tot"), a["p"])
     s.close()
+
+
+@pytest.mark.parametrize("shape,prec", [((6, 1, 8, 1), 4), ((8, 1, 12, 1), 8), ((12, 1, 36, 1), 4), ((16, 1, 100, 1), 8),
+                                        ((64, 1, 20, 1), 4), ((96, 1, 36, 1), 8), ((192, 1, 24, 1), 8),
+                                        ((256, 1, 28, 1), 8), ((384, 1, 20, 1), 8), ((384, 1, 52, 1), 4),
+                                        ((512, 1, 20, 1), 4), ((24, 12, 36, 0), 4), ((48, 24, 16, 0), 8)])
+def test_whole_field_transforms(shape, prec):
+    """ToNodal and ToModal against numpy for every length class (one register
+    DFT and two passes of N1/2 points), 16 and 8 levels per block, and levels
+    that do not fill a block; a level's result does not depend on its
+    neighbours, bit for bit."""
+    s = solver(shape, prec)
+    N1, N2, N3, dim = shape
+    f, a = random_field(s, sf.NEUMANN, 6)
+    a[0, 0] = a[0, 0].real
+    for j2 in range(1, (N2 + 1) // 2):  # a real field's j1 = 0 column
+        a[N2 - j2, 0] = a[j2, 0].conj()
+    a[..., 1] = a[..., 0]  # equal levels
+    f.upload(a)
+    a = f.download()
+    n, back = s.field(sf.NODAL, sf.NEUMANN), s.field(sf.MODAL, sf.NEUMANN)
+    f.ToNodal(n)
+    want = np.fft.irfft2(a, s=(N2, N1), axes=(0, 1)) * (N1 * N2)
+    got = n.download()
+    tol = 8 * np.finfo(np.float32 if prec == 4 else np.float64).eps * np.log2(N1 * N2)
+    e = np.linalg.norm(got - want) / np.linalg.norm(want)
+    n.ToModal(back)
+    b = np.linalg.norm(back.download() - a) / np.linalg.norm(a)
+    print(shape, prec, "%.2e %.2e" % (e / tol, b / tol), flush=True)
+    assert e < tol and b < 2 * tol
+    assert np.array_equal(got[..., 0], got[..., 1])
+    s.close()
