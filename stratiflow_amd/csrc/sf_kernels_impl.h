@@ -21,6 +21,7 @@
 #pragma once
 #include "sf_fft.h"
 #include "sf_kernels.h"
+#include "sf_rows.h"
 #include "sf_tri.h"
 
 #include <type_traits>
@@ -32,95 +33,6 @@ constexpr int BS = 256;
 // ---------------------------------------------------------------------------
 // k_modal
 // ---------------------------------------------------------------------------
-template <typename T, int M>
-__device__ __forceinline__ void nb_prev(const cx<T> (&x)[M], cx<T> (&xm)[M], int lane) {
-    using V = cx<T>;
-    V s;
-    s.x = __shfl(x[M - 1].x, (lane - 1) & 63, 64);
-    s.y = __shfl(x[M - 1].y, (lane - 1) & 63, 64);
-    if (lane == 0) s = czero<V>();
-    xm[0] = s;
-#pragma unroll
-    for (int t = 1; t < M; ++t) xm[t] = x[t - 1];
-}
-template <typename T, int M>
-__device__ __forceinline__ void nb_next(const cx<T> (&x)[M], cx<T> (&xp)[M], int lane) {
-    using V = cx<T>;
-    V s;
-    s.x = __shfl(x[0].x, (lane + 1) & 63, 64);
-    s.y = __shfl(x[0].y, (lane + 1) & 63, 64);
-    if (lane == 63) s = czero<V>();
-#pragma unroll
-    for (int t = 0; t < M - 1; ++t) xp[t] = x[t + 1];
-    xp[M - 1] = s;
-}
-
-// kind: 0 velocity Neumann, 1 velocity Dirichlet, 2 buoyancy Neumann,
-// 3 pressure Laplacian.  Matrix rows as built in IMEXRK.h:55-78, 502-545
-// with Neumannify/Dirichlify (Differentiation.h:17-59).
-// zcoef(c, t): coefficient row c at the lane's row t (zero beyond N3).
-template <typename T, int M, typename ZC>
-__device__ __forceinline__ void build_rows(int kind, const ModalArgs<T>& A, const int (&row)[M], T kk, T kl,
-                                           bool zero_mode, T coef, ZC zcoef, T (&a)[M], T (&b)[M], T (&c)[M]) {
-    const int N = A.N3;
-    const bool dir = (kind == 1);
-#pragma unroll
-    for (int t = 0; t < M; ++t) {
-        const int j = row[t];
-        if (j >= N) {
-            a[t] = 0;
-            b[t] = 1;
-            c[t] = 0;
-            continue;
-        }
-        const T lo = zcoef(dir ? ZC_DZZD_LO : ZC_DZZN_LO, t);
-        const T di = zcoef(dir ? ZC_DZZD_DI : ZC_DZZN_DI, t);
-        const T up = zcoef(dir ? ZC_DZZD_UP : ZC_DZZN_UP, t);
-        const T ldi = (di + kk) + kl;
-        T aa, bb, cc;
-        if (kind == 3) {
-            aa = lo;
-            bb = ldi;
-            cc = up;
-        } else {
-            aa = -(coef * lo);
-            bb = T(1) - coef * ldi;
-            cc = -(coef * up);
-        }
-        if (j == 0) aa = 0;
-        if (j == N - 1) cc = 0;
-        if (!dir) {
-            if (j == 0) {
-                bb = 1;
-                cc = 0;
-            } else if (j == 1) {
-                aa = 0;
-                bb = 1;
-                cc = -1;
-            } else if (j == N - 2) {
-                aa = 1;
-                bb = -1;
-                cc = 0;
-            } else if (j == N - 1) {
-                aa = 0;
-                bb = 1;
-            }
-        } else if (j <= 2 || j >= N - 2) {
-            aa = 0;
-            bb = 1;
-            cc = 0;
-        }
-        if (kind == 3 && zero_mode && j <= 1) {
-            aa = 0;
-            bb = 1;
-            cc = 0;
-        }
-        a[t] = aa;
-        b[t] = bb;
-        c[t] = cc;
-    }
-}
-
 // largest rows per lane of the modal kernel (N3 <= 64 * MODAL_MAX_M)
 constexpr int MODAL_MAX_M = 8;
 
@@ -173,6 +85,8 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
         if constexpr (FULL) return bld<T>(zr, zoff[0], (c * A.N3p + t) * int(sizeof(T)));
         else return bld<T>(zr, zoff[t], c * A.N3p * int(sizeof(T)));
     };
+    auto dzzn = [&](int i, int t) -> T { return coefz(ZC_DZZN_LO + i, t); };
+    auto dzzd = [&](int i, int t) -> T { return coefz(ZC_DZZD_LO + i, t); };
     // tile element owned by this thread in the cooperative (coalesced) phase:
     // rows z = tid/MB + t*64 for t < M (N3 <= 64*M), mode w = tid % MB.  Every
     // modal field has the same layout, so one table of byte offsets serves all
@@ -277,8 +191,8 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
             if (!zero_mode) {
 #pragma unroll
                 for (int t = 0; t < M; ++t) {
-                    const V ifb = cadd(cscale(coefz(ZC_IFULL_LO, t), bm[t]), cscale(coefz(ZC_IFULL_DI, t), bb[t]));
-                    rn3[t] = cadd(cscale(A.Ri, ifb), rn3[t]);
+                    const V ifb = mad2(coefz(ZC_IFULL_LO, t), bm[t], coefz(ZC_IFULL_DI, t), bb[t]);
+                    rn3[t] = tmadc(A.Ri, ifb, rn3[t]);
                 }
             }
             V u3p[M];
@@ -286,7 +200,7 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
 #pragma unroll
             for (int t = 0; t < M; ++t) {
                 const V idr = cadd(cscale(T(0.5), u3[t]), cscale(T(0.5), u3p[t]));
-                rnB[t] = csub(rnB[t], cscale(coefz(ZC_S, t), idr));
+                rnB[t] = tmadc(-coefz(ZC_S, t), idr, rnB[t]);
             }
         }
         store(A.rn1, rn1);
@@ -306,12 +220,9 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
             const int zlo = dir ? ZC_DZZD_LO : ZC_DZZN_LO;
 #pragma unroll
             for (int t = 0; t < M; ++t) {
-                V r = cadd(cadd(u[t], cscale(A.hz, ro_[t])), cscale(A.mh, gp[t]));
-                r = cadd(r, cscale(A.hb, rn[t]));
-                const V dzz = cadd(cadd(cscale(coefz(zlo, t), um[t]), cscale(coefz(zlo + 1, t), u[t])),
-                                   cscale(coefz(zlo + 2, t), up[t]));
-                const V lap = cadd(cadd(cscale(kk, u[t]), cscale(kl, u[t])), dzz);
-                R[t] = cadd(r, cscale(c, lap));
+                const V dzz = dzz_row(coefz(zlo, t), um[t], coefz(zlo + 1, t), u[t], coefz(zlo + 2, t), up[t]);
+                const V lap = cadd(mad2(kk, u[t], kl, u[t]), dzz);
+                R[t] = rhs_row(u[t], A.hz, ro_[t], A.mh, gp[t], A.hb, rn[t], c, lap);
             }
             zero_ends(R, dir);
         };
@@ -320,7 +231,7 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
         TriFactor<T, M> F;
         T ta[M], tb[M], tc[M];
         // u1 and u2 share the velocity Neumann matrix
-        build_rows<T, M>(0, A, row, kk, kl, zero_mode, A.cv, coefz, ta, tb, tc);
+        build_rows<T, M>(0, A, row, kk, kl, zero_mode, A.cv, dzzn, ta, tb, tc);
         tri_factor<T, M>(F, ta, tb, tc, lane);
 #pragma unroll
         for (int t = 0; t < M; ++t) gp[t] = cik(kx, pp[t]);
@@ -344,9 +255,8 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
 #pragma unroll
             for (int t = 0; t < M; ++t) {
                 const int j = row[t];
-                const V dzz = cadd(cadd(cscale(coefz(ZC_DZZN_LO, t), um[t]), cscale(coefz(ZC_DZZN_DI, t), ub[t])),
-                                   cscale(coefz(ZC_DZZN_UP, t), up[t]));
-                R[t] = (j <= 1 || j >= N - 2) ? czero<V>() : cadd(ub[t], cscale(A.cv, dzz));
+                const V dzz = dzz_row(coefz(ZC_DZZN_LO, t), um[t], coefz(ZC_DZZN_DI, t), ub[t], coefz(ZC_DZZN_UP, t), up[t]);
+                R[t] = (j <= 1 || j >= N - 2) ? czero<V>() : tmadc(A.cv, dzz, ub[t]);
             }
             tri_apply<T, M>(F, R, lane);
 #pragma unroll
@@ -366,9 +276,9 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
             V pm[M];
             nb_prev<T, M>(pp, pm, lane);
 #pragma unroll
-            for (int t = 0; t < M; ++t) gp[t] = cscale(coefz(ZC_DZND, t), csub(pp[t], pm[t]));
+            for (int t = 0; t < M; ++t) gp[t] = tscale(coefz(ZC_DZND, t), csub(pp[t], pm[t]));
         }
-        build_rows<T, M>(1, A, row, kk, kl, zero_mode, A.cv, coefz, ta, tb, tc);
+        build_rows<T, M>(1, A, row, kk, kl, zero_mode, A.cv, dzzd, ta, tb, tc);
         tri_factor<T, M>(F, ta, tb, tc, lane);
         assemble(R, u3, A.ro3, g2, rn3, gp, true, A.cv);
         issue(A.roB, g3);
@@ -378,7 +288,7 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
         // b: buoyancy Neumann matrix, no pressure term
 #pragma unroll
         for (int t = 0; t < M; ++t) gp[t] = czero<V>();
-        build_rows<T, M>(2, A, row, kk, kl, zero_mode, A.cb, coefz, ta, tb, tc);
+        build_rows<T, M>(2, A, row, kk, kl, zero_mode, A.cb, dzzn, ta, tb, tc);
         tri_factor<T, M>(F, ta, tb, tc, lane);
         assemble(R, bb, A.roB, g3, rnB, gp, false, A.cb);
         tri_apply<T, M>(F, R, lane);
@@ -392,12 +302,7 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
         V u3p[M], dv[M];
         nb_next<T, M>(u3, u3p, lane);
 #pragma unroll
-        for (int t = 0; t < M; ++t) {
-            const V dz = cscale(coefz(ZC_DZDN, t), csub(u3p[t], u3[t]));
-            V h = cik(kx, u1[t]);
-            if (three) h = cadd(h, cik(ky, u2[t]));
-            dv[t] = cadd(h, dz);
-        }
+        for (int t = 0; t < M; ++t) dv[t] = div_row(kx, u1[t], three, ky, u2[t], coefz(ZC_DZDN, t), u3[t], u3p[t]);
         zero_ends(dv, false);
         if (std::is_same<T, float>::value && zero_mode) {
             // The pinned Neumann Poisson problem of the (0,0) mode
@@ -407,7 +312,7 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
             TriFactor<double, M> F;
             double ta[M], tb[M], tc[M];
             T fa[M], fb[M], fc[M];
-            build_rows<T, M>(3, A, row, kk, kl, zero_mode, T(0), coefz, fa, fb, fc);
+            build_rows<T, M>(3, A, row, kk, kl, zero_mode, T(0), dzzn, fa, fb, fc);
 #pragma unroll
             for (int t = 0; t < M; ++t) {
                 ta[t] = fa[t];
@@ -435,17 +340,17 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
         } else {
             TriFactor<T, M> F;
             T ta[M], tb[M], tc[M];
-            build_rows<T, M>(3, A, row, kk, kl, zero_mode, T(0), coefz, ta, tb, tc);
+            build_rows<T, M>(3, A, row, kk, kl, zero_mode, T(0), dzzn, ta, tb, tc);
             tri_factor<T, M>(F, ta, tb, tc, lane);
             tri_apply<T, M>(F, dv, lane);  // dv now holds q
             V qm[M];
             nb_prev<T, M>(dv, qm, lane);
 #pragma unroll
             for (int t = 0; t < M; ++t) {
-                u1[t] = csub(u1[t], cik(kx, dv[t]));
-                if (three) u2[t] = csub(u2[t], cik(ky, dv[t]));
-                u3[t] = csub(u3[t], cscale(coefz(ZC_DZND, t), csub(dv[t], qm[t])));
-                pp[t] = cadd(pp[t], cscale(A.pmult, dv[t]));
+                u1[t] = minus_ik(kx, dv[t], u1[t]);
+                if (three) u2[t] = minus_ik(ky, dv[t], u2[t]);
+                u3[t] = tmadc(-coefz(ZC_DZND, t), csub(dv[t], qm[t]), u3[t]);
+                pp[t] = tmadc(A.pmult, dv[t], pp[t]);
             }
         }
     }
@@ -581,30 +486,14 @@ static void launch_modal_mb(const ModalArgs<T>& a, hipStream_t s) {
     else hipLaunchKernelGGL((k_modal<T, M, false, MB>), grid, dim3(MB * 64), 0, s, a);
 }
 
-// Grids with at most this many modes (one per CU) take one mode per block:
-// the GPU is far from full and latency sets the time, so each mode's wave
-// runs alone on its CU (2D 256 x 1 x 256 FP32: 82 against 112 us per step
-// with 8 modes per block); larger grids keep the wide tiles that make the
-// loads coalesce.
-inline int modal_small_grid() {
-    static const int n = []() {
-        int dev = 0, ncu = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        return ncu;
-    }();
-    return n;
-}
-
 template <typename T>
 hipError_t launch_modal(const ModalArgs<T>& a, hipStream_t s) {
+    if (modal_cols_fit(a.A1, a.A2, a.N3, int(sizeof(cx<T>)))) return launch_modal_cols<T>(a, s);
     const int M = (a.N3 + 63) / 64;
     switch (M) {
-#define SF_M(m)                                                                                              \
-    case m:                                                                                                  \
-        if (a.A1 * a.A2 <= modal_small_grid())                                                               \
-            launch_modal_mb<T, m, 1>(a, s);                                                                  \
-        else                                                                                                 \
-            launch_modal_mb<T, m, modal_mb<T, m>()>(a, s);                                                   \
+#define SF_M(m)                                        \
+    case m:                                            \
+        launch_modal_mb<T, m, modal_mb<T, m>()>(a, s); \
         break;
         SF_M(1) SF_M(2) SF_M(3) SF_M(4) SF_M(5) SF_M(6) SF_M(7) SF_M(8)
 #undef SF_M
@@ -1686,7 +1575,8 @@ __global__ __launch_bounds__(64) void k_diffprec(DiffPrecArgs<T> P) {
         A.N3p = P.N3p;
         A.zc = P.zc;
         T a[M], b[M], c[M];
-        auto zcoef = [&](int cr, int t) -> T { return row[t] < N ? P.zc[cr * P.N3p + row[t]] : T(0); };
+        const T* dzz = P.zc + (dir ? ZC_DZZD_LO : ZC_DZZN_LO) * P.N3p;
+        auto zcoef = [&](int i, int t) -> T { return row[t] < N ? dzz[i * P.N3p + row[t]] : T(0); };
         build_rows<T, M>(dir ? 1 : 0, A, row, kk, kl, false, P.tnu / P.delta, zcoef, a, b, c);
         TriFactor<T, M> F;
         tri_factor<T, M>(F, a, b, c, lane);

@@ -22,6 +22,27 @@
 
 namespace sf {
 
+// Products and fused multiply-adds of the solver, rounded as written: left to
+// the compiler, which products of a chain are fused depends on the code around
+// the inlined solver, and kernels that share it would differ in the last bit.
+template <typename T>
+__device__ __forceinline__ T tmul(T a, T b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+template <typename T>
+__device__ __forceinline__ T tmad(T a, T b, T c) {  // a*b + c
+    return __builtin_elementwise_fma(a, b, c);
+}
+template <typename T>
+__device__ __forceinline__ cx<T> tscale(T a, cx<T> v) {
+    return mkc<T>(tmul(a, v.x), tmul(a, v.y));
+}
+template <typename T>
+__device__ __forceinline__ cx<T> tmadc(T a, cx<T> v, cx<T> c) {  // a*v + c
+    return mkc<T>(tmad(a, v.x, c.x), tmad(a, v.y, c.y));
+}
+
 template <typename T>
 __device__ __forceinline__ T shfl_idx(T v, int src) {
     return __shfl(v, src, 64);
@@ -60,25 +81,25 @@ __device__ __forceinline__ void tri_factor(TriFactor<T, M>& F, const T (&a)[M], 
         F.rden[0] = recip(den);
 #pragma unroll
         for (int t = 0; t < M - 2; ++t) {
-            F.cc[t] = c[t] * F.rden[t];
-            den = b[t + 1] - a[t + 1] * F.cc[t];
+            F.cc[t] = tmul(c[t], F.rden[t]);
+            den = tmad(-a[t + 1], F.cc[t], b[t + 1]);
             F.rden[t + 1] = recip(den);
         }
         // spike v: A_int^{-1} (a_0 e_0)
         {
             T D[M];
-            D[0] = a[0] * F.rden[0];
+            D[0] = tmul(a[0], F.rden[0]);
 #pragma unroll
-            for (int t = 1; t <= M - 2; ++t) D[t] = (-a[t] * D[t - 1]) * F.rden[t];
+            for (int t = 1; t <= M - 2; ++t) D[t] = tmul(tmul(-a[t], D[t - 1]), F.rden[t]);
             F.v[M - 2] = D[M - 2];
 #pragma unroll
-            for (int t = M - 3; t >= 0; --t) F.v[t] = D[t] - F.cc[t] * F.v[t + 1];
+            for (int t = M - 3; t >= 0; --t) F.v[t] = tmad(-F.cc[t], F.v[t + 1], D[t]);
         }
         // spike w: A_int^{-1} (c_{M-2} e_{M-2})
         {
-            F.w[M - 2] = c[M - 2] * F.rden[M - 2];
+            F.w[M - 2] = tmul(c[M - 2], F.rden[M - 2]);
 #pragma unroll
-            for (int t = M - 3; t >= 0; --t) F.w[t] = -F.cc[t] * F.w[t + 1];
+            for (int t = M - 3; t >= 0; --t) F.w[t] = tmul(-F.cc[t], F.w[t + 1]);
         }
         const T aI = a[M - 1], cI = c[M - 1];
         F.aI = aI;
@@ -90,9 +111,9 @@ __device__ __forceinline__ void tri_factor(TriFactor<T, M>& F, const T (&a)[M], 
             wn0 = 0;
         }
         F.vn0 = vn0;
-        As = -aI * F.v[M - 2];
-        Bs = b[M - 1] - aI * F.w[M - 2] - cI * vn0;
-        Cs = -cI * wn0;
+        As = tmul(-aI, F.v[M - 2]);
+        Bs = tmad(-cI, vn0, tmad(-aI, F.w[M - 2], b[M - 1]));
+        Cs = tmul(-cI, wn0);
     }
     // parallel cyclic reduction on the 64-unknown Schur system
 #pragma unroll
@@ -110,13 +131,13 @@ __device__ __forceinline__ void tri_factor(TriFactor<T, M>& F, const T (&a)[M], 
             Bp = 1;
             Cp = 0;
         }
-        const T al = -As * recip(Bm);
-        const T ga = -Cs * recip(Bp);
+        const T al = tmul(-As, recip(Bm));
+        const T ga = tmul(-Cs, recip(Bp));
         F.alpha[lev] = al;
         F.gamma[lev] = ga;
-        const T nA = al * Am;
-        const T nC = ga * Cp;
-        Bs = Bs + al * Cm + ga * Ap;
+        const T nA = tmul(al, Am);
+        const T nC = tmul(ga, Cp);
+        Bs = tmad(ga, Ap, tmad(al, Cm, Bs));
         As = nA;
         Cs = nC;
     }
@@ -134,16 +155,16 @@ __device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, cx<T> (&d)[M
         Ds = d[0];
     } else {
         // interior forward/back sweep for g
-        g[0] = cscale(F.rden[0], d[0]);
+        g[0] = tscale(F.rden[0], d[0]);
 #pragma unroll
-        for (int t = 1; t <= M - 2; ++t) g[t] = cscale(F.rden[t], csub(d[t], cscale(F.a[t], g[t - 1])));
+        for (int t = 1; t <= M - 2; ++t) g[t] = tscale(F.rden[t], tmadc(-F.a[t], g[t - 1], d[t]));
 #pragma unroll
-        for (int t = M - 3; t >= 0; --t) g[t] = csub(g[t], cscale(F.cc[t], g[t + 1]));
+        for (int t = M - 3; t >= 0; --t) g[t] = tmadc(-F.cc[t], g[t + 1], g[t]);
         V gn0;
         gn0.x = shfl_idx(g[0].x, (lane + 1) & 63);
         gn0.y = shfl_idx(g[0].y, (lane + 1) & 63);
         if (lane == 63) gn0 = czero<V>();
-        Ds = csub(csub(d[M - 1], cscale(F.aI, g[M - 2])), cscale(F.cI, gn0));
+        Ds = tmadc(-F.cI, gn0, tmadc(-F.aI, g[M - 2], d[M - 1]));
     }
 #pragma unroll
     for (int lev = 0; lev < 6; ++lev) {
@@ -155,9 +176,9 @@ __device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, cx<T> (&d)[M
         Dp.y = shfl_idx(Ds.y, (lane + s) & 63);
         if (lane - s < 0) Dm = czero<V>();
         if (lane + s > 63) Dp = czero<V>();
-        Ds = cadd(cadd(Ds, cscale(F.alpha[lev], Dm)), cscale(F.gamma[lev], Dp));
+        Ds = tmadc(F.gamma[lev], Dp, tmadc(F.alpha[lev], Dm, Ds));
     }
-    const V sl = cscale(F.rB, Ds);
+    const V sl = tscale(F.rB, Ds);
     if constexpr (M == 1) {
         d[0] = sl;
     } else {
@@ -166,7 +187,7 @@ __device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, cx<T> (&d)[M
         sm.y = shfl_idx(sl.y, (lane - 1) & 63);
         if (lane == 0) sm = czero<V>();
 #pragma unroll
-        for (int t = 0; t <= M - 2; ++t) d[t] = csub(csub(g[t], cscale(F.v[t], sm)), cscale(F.w[t], sl));
+        for (int t = 0; t <= M - 2; ++t) d[t] = tmadc(-F.w[t], sl, tmadc(-F.v[t], sm, g[t]));
         d[M - 1] = sl;
     }
 }
