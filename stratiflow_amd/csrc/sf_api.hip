@@ -79,7 +79,7 @@ struct Ctx {
     sf_ctx* owner = nullptr;
     int N1 = 0, N2 = 0, N3 = 0, M1 = 0, A1 = 0, A2 = 0, dim = 0, N3p = 0;
     bool three = false;
-    int zch = 4;   // z levels per x-pass block
+    int zch = 4, zch_lin = 4;  // z levels per x-pass block, nonlinear and linearised products
     int device = 0;  // the device current at creation
     double L1 = 0, L2 = 0, L3 = 0, Re = 0, Ri = 0, Pr = 0;
     bool evolve_bg = false;  // FlowParams::EvolveBackground
@@ -109,7 +109,7 @@ struct Ctx {
     int rcur = 0;
     V* nl[4] = {nullptr};
     V* Y[4] = {nullptr};
-    V* Yb[4] = {nullptr};
+    XBase<T>* xbase = nullptr;  // nodal base state of the linearised steps (first use)
     V* X[8] = {nullptr};
     // X[] (the 3D x-pass outputs) in tiles of 16 modes where the paired
     // forward y transform reads them as contiguous runs (yfwd_tiles)
@@ -186,7 +186,8 @@ struct Ctx {
         A1 = N1 / 3;
         A2 = three ? 2 * (N2 / 3) - 1 : 1;
         N3p = N3;
-        zch = xpass_levels(N1, N2, N3, three, int(sizeof(T)));
+        zch = xpass_levels(N1, N2, N3, three, false, int(sizeof(T)));
+        zch_lin = xpass_levels(N1, N2, N3, three, true, int(sizeof(T)));
         nmodal = size_t(A1) * A2 * N3;
         nnodal = size_t(N1) * N2 * N3;
         SF_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
@@ -396,7 +397,38 @@ struct Ctx {
     const V* src(int i) { return use_snap ? snap[i] : mf(SF_U1 + i); }
 
 
-    // nonlinear (or linearised) explicit terms of the current state into nl[]
+    // the base state of the linearised steps (SF_U1_TOT..SF_B_TOT) at the x
+    // points, for all stages of one call: nothing in a step changes it (the
+    // stages add the U_ of their time), callers may between calls
+    void linear_base() {
+        if (!xbase) xbase = dalloc<XBase<T>>(nnodal);
+        XBaseArgs<T> a{};
+        a.N3 = N3;
+        a.A1 = A1;
+        a.tw = tw1;
+        a.out = xbase;
+        for (int i = 0; i < 4; ++i) a.in[i] = mf(SF_U1_TOT + i);
+        if (three) {
+            YArgs<T> y{};
+            y.N3 = N3;
+            y.A1 = A1;
+            y.A2 = A2;
+            y.nf = 4;
+            y.tw = tw2;
+            y.scale = T(1);
+            for (int i = 0; i < 4; ++i) {
+                y.in[i] = a.in[i];
+                y.out[i] = X[i];
+                a.in[i] = X[i];
+            }
+            check(launch_yinv<T>(y, N2, stream), "yinv(base)");
+            mark(SF_K_YINV);
+        }
+        check(launch_xbase<T>(a, N1, N2, three, stream), "xbase");
+    }
+
+    // nonlinear (or, after linear_base, linearised) explicit terms of the current
+    // state into nl[]
     void transform_path(bool linear) {
         if (three) {
             YArgs<T> a{};
@@ -410,23 +442,12 @@ struct Ctx {
             a.scale = T(1);
             check(launch_yinv<T>(a, N2, stream), "yinv");
             mark(SF_K_YINV);
-            if (linear) {
-                if (!Yb[0])
-                    for (int i = 0; i < 4; ++i) Yb[i] = dalloc<V>(size_t(N2) * A1 * N3);
-                a.in[0] = mf(SF_U1_TOT);
-                a.in[1] = mf(SF_U2_TOT);
-                a.in[2] = mf(SF_U3_TOT);
-                a.in[3] = mf(SF_B_TOT);
-                for (int i = 0; i < 4; ++i) a.out[i] = Yb[i];
-                check(launch_yinv<T>(a, N2, stream), "yinv(base)");
-                mark(SF_K_YINV);
-            }
             XArgs<T> x{};
             x.N1 = N1;
             x.N3 = N3;
             x.N3p = N3p;
             x.A1 = A1;
-            x.zch = zch;
+            x.zch = linear ? zch_lin : zch;
             for (int i = 0; i < 4; ++i) x.in[i] = Y[i];
             for (int i = 0; i < 8; ++i) x.out[i] = X[i];
             x.zc = zc;
@@ -436,7 +457,7 @@ struct Ctx {
             x.linear = linear ? 1 : 0;
             x.N2 = N2;
             x.tiled = ytiles ? 1 : 0;
-            for (int i = 0; i < 4; ++i) x.base[i] = linear ? Yb[i] : nullptr;
+            x.base = linear ? xbase : nullptr;
             check(launch_xpass<T>(x, N1, N2, true, stream), "xpass");
             mark(SF_K_XPASS);
             YArgs<T> f{};
@@ -473,7 +494,7 @@ struct Ctx {
         x.N3 = N3;
         x.N3p = N3p;
         x.A1 = A1;
-        x.zch = zch;
+        x.zch = linear ? zch_lin : zch;
         x.in[0] = src(0);
         x.in[1] = nullptr;
         x.in[2] = src(2);
@@ -488,10 +509,7 @@ struct Ctx {
         x.tw = tw1;
         x.scale = T(1.0 / double(N1));
         x.linear = linear ? 1 : 0;
-        x.base[0] = mf(SF_U1_TOT);
-        x.base[1] = nullptr;
-        x.base[2] = mf(SF_U3_TOT);
-        x.base[3] = mf(SF_B_TOT);
+        x.base = linear ? xbase : nullptr;
         return x;
     }
 
@@ -567,6 +585,7 @@ struct Ctx {
     }
 
     void step(int n, bool linear) {
+        if (linear && n > 0) linear_base();
         for (int s = 0; s < n; ++s)
             for (int k = 0; k < 3; ++k) stage(k, linear, k < 2);
     }
@@ -2032,7 +2051,10 @@ int sf_stage(sf_ctx* ctx, int k, int linear) {
     SF_NULLCHK(ctx);
     return guarded(ctx, [&]() {
         SF_REQUIRE(k >= 0 && k < 3, SF_ERR_ARG, "stage must be 0, 1 or 2");
-        with_ctx(ctx, [&](auto& C) { C.stage(k, linear != 0, true); });
+        with_ctx(ctx, [&](auto& C) {
+            if (linear) C.linear_base();
+            C.stage(k, linear != 0, true);
+        });
     });
 }
 

@@ -31,6 +31,19 @@ __host__ __device__ inline size_t sidx(int row, int z, int j1, int N3, int A1) {
     return (size_t(row) * size_t(N3) + size_t(z)) * size_t(A1) + size_t(j1);
 }
 
+// Base state of the linearised products at one x point (U_ not included).
+template <typename T>
+struct alignas(16) XBase {
+    T u1, u2, u3, b;
+};
+template <typename T>
+struct XBaseArgs {
+    int N3, A1;
+    const cx<T>* in[4];  // x spectra of u1, u2, u3, b
+    XBase<T>* out;       // [n2][z][x point]
+    const cx<T>* tw;
+};
+
 // Fused inverse-x / products / forward-x kernel.
 template <typename T>
 struct XArgs {
@@ -44,7 +57,7 @@ struct XArgs {
     const cx<T>* tw;
     T scale;
     int linear;                          // 1: linearised products (BuildRHSLinear)
-    const cx<T>* base[4];                // linear: u1t, u2t, u3t, bt spectra (same layout as in)
+    const XBase<T>* base;                // linear: the base state (launch_xbase)
 };
 
 // y-direction transforms (3D): per (z, tile of consecutive j1).
@@ -88,6 +101,8 @@ hipError_t launch_modal_cols(const ModalArgs<T>& a, hipStream_t s);
 bool modal_cols_fit(int A1, int A2, int N3, int value_bytes);  // whether it is the faster one
 template <typename T>
 hipError_t launch_xpass(const XArgs<T>& a, int N1, int N2, bool threeD, hipStream_t s);
+template <typename T>
+hipError_t launch_xbase(const XBaseArgs<T>& a, int N1, int N2, bool threeD, hipStream_t s);
 // many independent 2D runs per launch: args/start live in device memory,
 // start[r] = first work item of run r (x-pass: z-blocks; modal: tiles of
 // modes), total = start[nruns]; grid-stride loop over `grid` blocks.  The
@@ -225,7 +240,7 @@ hipError_t launch_add_mean(cx<T>* f, int N3, int A1, T value, hipStream_t s);
 bool tz_supported(int n);
 // z levels per x-pass block for this grid (the block height that minimises
 // rounds of resident blocks x (levels + 2))
-int xpass_levels(int N1, int N2, int N3, bool threeD, int precision);
+int xpass_levels(int N1, int N2, int N3, bool threeD, bool linear, int precision);
 // twiddle table of an n-point LDS FFT: 2n entries (the layout its second pass
 // reads, then the same values in the order of the second pass on lane pairs)
 void fft_twiddles(int n, double* re, double* im);

@@ -554,11 +554,23 @@ constexpr int xpass_bs() {
     return BS;
 }
 
-// LDS values of one x-pass block: NP product lines and a ring of 3 x NI
-// input lines at the line pitch x_ldp
-template <int N1, bool THREED, bool LIN, int R1F = 0>
+// LDS values of one x-pass block: NP product lines and a ring of 3 x 2 input
+// lines at the line pitch x_ldp
+template <int N1, bool THREED, int R1F = 0>
 constexpr int xpass_lds() {
-    return ((THREED ? 6 : 3) + 3 * (LIN ? 4 : 2)) * x_ldp<N1, R1F>();
+    return ((THREED ? 6 : 3) + 3 * 2) * x_ldp<N1, R1F>();
+}
+
+// conj of the Hermitian-extended pair line Z = F(a) + i F(b) from the modes x of
+// a and y of b (j1 < A1); the caller clears j = A1 .. N1-A1
+template <typename T>
+__device__ __forceinline__ void pair_line(cx<T>* L, int N1, int j1, cx<T> x, cx<T> y) {
+    if (j1 == 0) {  // c2r ignores the imaginary part of the DC term
+        L[0] = mkc<T>(x.x, -y.x);
+    } else {
+        L[j1] = mkc<T>(x.x - y.y, -(x.y + y.x));
+        L[N1 - j1] = mkc<T>(x.x + y.y, x.y - y.x);
+    }
 }
 
 // R1F: the FFT plan's first radix (0: the default; A.tw must be the table of
@@ -567,12 +579,13 @@ template <typename T, int N1, bool THREED, bool LIN, int R1F = 0>
 __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, const int n2, cx<T>* const lds) {
     using V = cx<T>;
     constexpr int LDP = x_ldp<N1, R1F>();
-    constexpr int NI = LIN ? 4 : 2;        // input pair lines per level
+    constexpr int NI = 2;                  // input pair lines per level
     constexpr int NP = THREED ? 6 : 3;     // product pair lines per level
     constexpr int NB = NP + NI;            // lines per batched FFT
     constexpr int AMAX = N1 / 3;           // A1 <= N1/3
     constexpr int XB = xpass_bs<T, THREED, LIN>();
     constexpr int FI = (NI * AMAX + XB - 1) / XB;
+    constexpr int WI = LIN ? (N1 + XB - 1) / XB : 1;  // x points per thread
     // lds: [NP product lines][ring slot 0: NI lines][slot 1][slot 2]
     V* const prd = lds;
     V* const ring = lds + NP * LDP;
@@ -598,16 +611,15 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
             if (item < NI * A1 && z >= 0 && z < N3) {
                 const int pair = item / A1;
                 const int j1 = item - pair * A1;
-                const V* const* in = (pair >= 2) ? A.base : A.in;
                 const size_t off = sidx(n2, z, j1, N3, A1);
-                if ((pair & 1) == 0) {
-                    X[i] = in[0][off];
-                    Y[i] = in[2][off];
+                if (pair == 0) {
+                    X[i] = A.in[0][off];
+                    Y[i] = A.in[2][off];
                 } else if (THREED) {
-                    X[i] = in[1][off];
-                    Y[i] = in[3][off];
+                    X[i] = A.in[1][off];
+                    Y[i] = A.in[3][off];
                 } else {
-                    X[i] = in[3][off];
+                    X[i] = A.in[3][off];
                 }
             }
         }
@@ -626,19 +638,30 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
             if (item < NI * A1) {
                 const int pair = item / A1;
                 const int j1 = item - pair * A1;
-                V* L = R + pair * LDP;
-                const V x = X[i], y = Y[i];
-                if (j1 == 0) {  // c2r ignores the imaginary part of the DC term
-                    L[0] = mkc<T>(x.x, -y.x);
+                pair_line<T>(R + pair * LDP, N1, j1, X[i], Y[i]);
+            }
+        }
+    };
+    // linearised products: the nodal base state (k_xbase) of this thread's x
+    // points at levels z-1, z, z+1, each level loaded once per block
+    XBase<T> W[WI][3];
+    auto load_base = [&](int z, int d) {
+        if constexpr (LIN) {
+#pragma unroll
+            for (int i = 0; i < WI; ++i) {
+                const int n = tid + i * XB;
+                if (n < N1 && z >= 0 && z < N3) {
+                    W[i][d] = A.base[(size_t(n2) * N3 + z) * N1 + n];
                 } else {
-                    L[j1] = mkc<T>(x.x - y.y, -(x.y + y.x));
-                    L[N1 - j1] = mkc<T>(x.x + y.y, x.y - y.x);
+                    W[i][d] = XBase<T>{T(0), T(0), T(0), T(0)};
                 }
             }
         }
     };
 
     // prologue: levels zbeg-1, zbeg, zbeg+1 into slots 0, 1, 2
+#pragma unroll
+    for (int l = 0; l < 3; ++l) load_base(zbeg - 1 + l, l);
     for (int l = 0; l < 3; ++l) {
         load(zbeg - 1 + l);
         store(l);
@@ -668,7 +691,7 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
             const V* Ls[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) Ls[d] = ring + slot(z - 1 + d) * NI * LDP;
-            for (int n = tid; n < N1; n += XB) {
+            auto products = [&](const int n, const XBase<T>(&Wn)[3]) {
                 T u1[3], u2[3], u3[3], bb[3], w1[3], w2[3], w3[3], wb[3];
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
@@ -679,12 +702,11 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
                     u2[d] = THREED ? c.x : T(0);
                     bb[d] = THREED ? -c.y : c.x;
                     if (LIN) {
-                        const V e = Ls[d][2 * LDP + n];
-                        const V f = Ls[d][3 * LDP + n];
-                        w1[d] = e.x + ub[d];
-                        w3[d] = -e.y;
-                        w2[d] = THREED ? f.x : T(0);
-                        wb[d] = THREED ? -f.y : f.x;
+                        const XBase<T> w = Wn[d];
+                        w1[d] = w.u1 + ub[d];
+                        w2[d] = w.u2;
+                        w3[d] = w.u3;
+                        wb[d] = w.b;
                     } else {
                         w1[d] = w2[d] = w3[d] = wb[d] = T(0);
                     }
@@ -743,7 +765,22 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
                 }
 #pragma unroll
                 for (int q = 0; q < NP; ++q) prd[q * LDP + n] = mkc<T>(P[2 * q], P[2 * q + 1]);
+            };
+            if constexpr (LIN) {
+#pragma unroll
+                for (int i = 0; i < WI; ++i)
+                    if (tid + i * XB < N1) products(tid + i * XB, W[i]);
+            } else {
+                for (int n = tid; n < N1; n += XB) products(n, W[0]);
             }
+        }
+        if (LIN && more) {
+#pragma unroll
+            for (int i = 0; i < WI; ++i) {
+                W[i][0] = W[i][1];
+                W[i][1] = W[i][2];
+            }
+            load_base(z + 2, 2);
         }
         sync_lds();
         if (more) {
@@ -795,8 +832,74 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
 template <typename T, int N1, bool THREED, bool LIN>
 __global__ __launch_bounds__((xpass_bs<T, THREED, LIN>())) __attribute__((amdgpu_waves_per_eu(xpass_waves<T, THREED, LIN>()))) void k_xpass(
     XArgs<T> A) {
-    __shared__ cx<T> lds[xpass_lds<N1, THREED, LIN>()];
+    __shared__ cx<T> lds[xpass_lds<N1, THREED>()];
     xpass_body<T, N1, THREED, LIN>(A, blockIdx.x, blockIdx.y, lds);
+}
+
+// The linearised products' base state at the x points, four values per point,
+// from its x spectra: once per call of any number of steps, since the base does
+// not change within one.  Transforming it inside every stage's x-pass took 12 of
+// the 18 LDS lines of a block and as many FFTs again (104 us per stage at
+// 192x96x192 FP32, with one y transform more).  Bound by HBM; four levels (eight
+// lines) per block fill every round of both FFT passes at 384 points.
+constexpr int XBASE_LEVELS = 4;
+template <typename T, int N1, bool THREED>
+__global__ __launch_bounds__(BS) void k_xbase(XBaseArgs<T> A) {
+    using V = cx<T>;
+    constexpr int LDP = x_ldp<N1>(), NL = 2 * XBASE_LEVELS;
+    __shared__ V buf[NL * LDP];
+    const int N3 = A.N3, A1 = A.A1, n2 = blockIdx.y, z0 = blockIdx.x * XBASE_LEVELS;
+    const int nband = N1 - 2 * A1 + 1;  // j = A1 .. N1-A1 is zero
+    for (int idx = threadIdx.x; idx < NL * nband; idx += BS)
+        buf[(idx / nband) * LDP + A1 + idx % nband] = czero<V>();
+    for (int idx = threadIdx.x; idx < NL * A1; idx += BS) {
+        const int line = idx / A1, j1 = idx - line * A1;
+        const int z = z0 + line / 2;
+        V x = czero<V>(), y = czero<V>();
+        if (z < N3) {
+            const size_t off = sidx(n2, z, j1, N3, A1);
+            if (line % 2 == 0) {
+                x = A.in[0][off];
+                y = A.in[2][off];
+            } else if (THREED) {
+                x = A.in[1][off];
+                y = A.in[3][off];
+            } else {
+                x = A.in[3][off];
+            }
+        }
+        pair_line<T>(buf + line * LDP, N1, j1, x, y);
+    }
+    sync_lds();
+    lds_fft_lines<T, N1, NL, BS, -1, 1, false, 0, true>(NL, [&](int line) { return buf + line * LDP; }, A.tw);
+    for (int idx = threadIdx.x; idx < XBASE_LEVELS * N1; idx += BS) {
+        const int t = idx / N1, n = idx - t * N1;
+        if (z0 + t >= N3) break;
+        const V e = buf[2 * t * LDP + n];        // conj(U1 + i U3)
+        const V f = buf[(2 * t + 1) * LDP + n];  // conj(U2 + i B) or conj(B)
+        A.out[(size_t(n2) * N3 + z0 + t) * N1 + n] =
+            THREED ? XBase<T>{e.x, f.x, -e.y, -f.y} : XBase<T>{e.x, T(0), -e.y, f.x};
+    }
+}
+
+template <typename T>
+hipError_t launch_xbase(const XBaseArgs<T>& a, int N1, int N2, bool threeD, hipStream_t s) {
+    const dim3 grid((a.N3 + XBASE_LEVELS - 1) / XBASE_LEVELS, threeD ? N2 : 1);
+    switch (N1) {
+#define SF_CASE(n)                                                                                   \
+    case n:                                                                                          \
+        if constexpr (2 * XBASE_LEVELS * x_ldp<n>() * int(sizeof(cx<T>)) <= 160 * 1024) {            \
+            if (threeD) hipLaunchKernelGGL((k_xbase<T, n, true>), grid, dim3(BS), 0, s, a);          \
+            else hipLaunchKernelGGL((k_xbase<T, n, false>), grid, dim3(BS), 0, s, a);                \
+            return hipGetLastError();                                                                \
+        } else {                                                                                     \
+            return hipErrorInvalidValue;                                                             \
+        }
+        SF_SIZES(SF_CASE)
+#undef SF_CASE
+        default:
+            return hipErrorInvalidValue;
+    }
 }
 
 // 2D runs with the same N1 in one launch (grid-stride over the z-blocks of
@@ -805,7 +908,7 @@ template <typename T, int N1>
 __global__ __launch_bounds__(BS) void k_xpass_batch(const XArgs<T>* __restrict__ args, const int* __restrict__ start,
                                                     int nruns, int total) {
     static_assert(xpass_bs<T, false, false>() == BS, "the batched 2D x-pass runs blocks of BS threads");
-    __shared__ cx<T> lds[xpass_lds<N1, false, false>()];
+    __shared__ cx<T> lds[xpass_lds<N1, false>()];
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         const int r = find_run(start, nruns, item);
         xpass_body<T, N1, false, false>(args[r], item - start[r], 0, lds);
@@ -820,7 +923,7 @@ template <int NMAX, int R1F>
 constexpr int xpass_mixed_lds() {
     int m = 0;
 #define SF_CASE(n) \
-    if (n <= NMAX && xpass_lds<n, false, false, R1F>() > m) m = xpass_lds<n, false, false, R1F>();
+    if (n <= NMAX && xpass_lds<n, false, R1F>() > m) m = xpass_lds<n, false, R1F>();
     SF_SIZES(SF_CASE)
 #undef SF_CASE
     return m;
@@ -885,7 +988,7 @@ hipError_t launch_xpass_batch(const XArgs<T>* args, const int* start, int nruns,
 
 template <typename T, int N1, bool THREED, bool LIN>
 static hipError_t launch_xpass_v(const XArgs<T>& a, int N2, hipStream_t s) {
-    constexpr int lds = xpass_lds<N1, THREED, LIN>() * int(sizeof(cx<T>));
+    constexpr int lds = xpass_lds<N1, THREED>() * int(sizeof(cx<T>));
     if constexpr (lds > 160 * 1024) {
         return hipErrorInvalidValue;  // not instantiated: does not fit the LDS of one CU
     } else {
@@ -920,7 +1023,7 @@ hipError_t launch_xpass(const XArgs<T>& a, int N1, int N2, bool threeD, hipStrea
 // level per block: more blocks in flight for the same single round).
 template <typename T, int N1, bool THREED, bool LIN>
 static int xpass_resident(int ncu) {
-    constexpr int lds = xpass_lds<N1, THREED, LIN>() * int(sizeof(cx<T>));
+    constexpr int lds = xpass_lds<N1, THREED>() * int(sizeof(cx<T>));
     if constexpr (lds > 160 * 1024) {
         return 0;
     } else {
@@ -934,10 +1037,11 @@ static int xpass_resident(int ncu) {
 // resident x-pass blocks on ncu CUs (each precision's translation unit
 // instantiates its own)
 template <typename T>
-int xpass_slots(int N1, bool threeD, int ncu) {
+int xpass_slots(int N1, bool threeD, bool linear, int ncu) {
     switch (N1) {
-#define SF_CASE(n) \
-    case n:        \
+#define SF_CASE(n)                                                                                              \
+    case n:                                                                                                     \
+        if (linear) return threeD ? xpass_resident<T, n, true, true>(ncu) : xpass_resident<T, n, false, true>(ncu); \
         return threeD ? xpass_resident<T, n, true, false>(ncu) : xpass_resident<T, n, false, false>(ncu);
         SF_SIZES(SF_CASE)
 #undef SF_CASE
@@ -947,12 +1051,12 @@ int xpass_slots(int N1, bool threeD, int ncu) {
 }
 
 #ifdef SF_KERNELS_HOST_DEFS
-extern template int xpass_slots<double>(int, bool, int);  // in the FP64 translation unit
+extern template int xpass_slots<double>(int, bool, bool, int);  // in the FP64 translation unit
 
-int xpass_levels(int N1, int N2, int N3, bool threeD, int precision) {
+int xpass_levels(int N1, int N2, int N3, bool threeD, bool linear, int precision) {
     int dev = 0, ncu = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    int slots = precision == 4 ? xpass_slots<float>(N1, threeD, ncu) : xpass_slots<double>(N1, threeD, ncu);
+    int slots = precision == 4 ? xpass_slots<float>(N1, threeD, linear, ncu) : xpass_slots<double>(N1, threeD, linear, ncu);
     if (slots < 1) slots = ncu;
     const int rows = threeD ? N2 : 1;
     long best = -1;
@@ -1614,6 +1718,7 @@ hipError_t launch_diffprec(const DiffPrecArgs<T>& p, hipStream_t s) {
 #define SF_INST_CORE(T) \
     template hipError_t launch_modal<T>(const ModalArgs<T>&, hipStream_t); \
     template hipError_t launch_xpass<T>(const XArgs<T>&, int, int, bool, hipStream_t); \
+    template hipError_t launch_xbase<T>(const XBaseArgs<T>&, int, int, bool, hipStream_t); \
     template hipError_t launch_yinv<T>(const YArgs<T>&, int, hipStream_t); \
     template hipError_t launch_yfwd<T>(const YArgs<T>&, int, hipStream_t); \
     template hipError_t launch_axpby<T>(cx<T>*, T, const cx<T>*, T, size_t, hipStream_t); \
@@ -1621,7 +1726,7 @@ hipError_t launch_diffprec(const DiffPrecArgs<T>& p, hipStream_t s) {
     template hipError_t launch_ends<T>(cx<T>*, int, int, int, int, hipStream_t); \
     template hipError_t launch_dmul<T>(cx<T>*, const cx<T>*, int, int, int, const T*, const T*, int, const T*, int, hipStream_t); \
     template hipError_t launch_diffprec<T>(const DiffPrecArgs<T>&, hipStream_t); \
-    template int xpass_slots<T>(int, bool, int);
+    template int xpass_slots<T>(int, bool, bool, int);
 
 #define SF_INST_BATCH(T) \
     template hipError_t launch_modal_batch<T>(const ModalArgs<T>*, const int*, int, int, int, int, hipStream_t); \

@@ -55,3 +55,31 @@ def test_linear_steps_fp32(shape):
         e = rel_l2(s.get(f), o.get_modal(f))
         print("linear fp32", f, e)
         assert e < 1e-4, f
+
+
+@pytest.mark.parametrize("shape,prec", [((6, 1, 8, 1), 8), ((256, 1, 36, 1), 8), ((384, 1, 24, 1), 8),
+                                        ((384, 1, 20, 1), 4), ((512, 1, 20, 1), 4), ((96, 12, 36, 0), 8),
+                                        ((384, 6, 12, 0), 8), ((384, 6, 20, 0), 4)])
+def test_linear_base_of_every_point_split(shape, prec):
+    """The base state held per x point: one and two points per thread, levels
+    that do not fill a block of the base transform, and a base that changes
+    between calls (steps, then single stages) is the one the next call uses."""
+    s, o, keep = _with_base(shape, prec)
+    s.TimeStepLinear(1)
+    o.step_linear(1)
+    for f in ("u1", "b"):  # another base, through the solver's own field
+        keep[f] *= 0.5
+        s.state(f + "_tot").assign(keep[f])
+        o.set_modal(f + "t", keep[f].download())
+    o.set_linear_background()
+    s.TimeStepLinear(1)
+    o.step_linear(1)
+    s.Stage(0, linear=True)
+    o.stage(0, linear=True)
+    for f in fields(shape[3]):
+        if prec == 4 and f == "p":
+            continue
+        e = rel_l2(s.get(f), o.get_modal(f))
+        print(shape, prec, f, "%.2e" % e, flush=True)
+        assert e < (1e-9 if prec == 8 else 1e-4), f
+    s.close()
