@@ -244,11 +244,24 @@ __global__ __launch_bounds__(NB) void k_wcast(const float* __restrict__ w, int C
     Wt[(size_t(KT - 1 - t) * Cin + ci) * Cout + co] = x;
 }
 
-// sum of |f|^2 over the active modes of up to 4 complex fields (FP64 partials)
+// RMS of up to 4 complex fields over the active modes: FP64 partial sums of
+// |f|^2, added in block order by the block that draws the last ticket (agent
+// scope: the blocks' XCDs have separate L2s), which leaves s = RMS and 1/s (0
+// for a zero field) in scale[0..1].  The host does not wait for it.
 template <typename T>
-__global__ __launch_bounds__(NB) void k_sumsq(const cx<T>* f0, const cx<T>* f1, const cx<T>* f2, const cx<T>* f3, size_t n,
-                                              double* __restrict__ part) {
+__global__ __launch_bounds__(NB) void k_rms(const cx<T>* f0, const cx<T>* f1, const cx<T>* f2, const cx<T>* f3, size_t n,
+                                            double count, double* __restrict__ part, unsigned* __restrict__ ticket,
+                                            double* __restrict__ scale) {
     __shared__ double red[NB];
+    __shared__ bool last;
+    auto block_sum = [&](double s) {
+        red[threadIdx.x] = s;
+        __syncthreads();
+        for (int k = NB / 2; k > 0; k >>= 1) {
+            if (int(threadIdx.x) < k) red[threadIdx.x] += red[threadIdx.x + k];
+            __syncthreads();
+        }
+    };
     double s = 0;
     const cx<T>* fs[4] = {f0, f1, f2, f3};
     for (int k = 0; k < 4; ++k) {
@@ -258,13 +271,23 @@ __global__ __launch_bounds__(NB) void k_sumsq(const cx<T>* f0, const cx<T>* f1, 
             s += double(v.x) * double(v.x) + double(v.y) * double(v.y);
         }
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int k = NB / 2; k > 0; k >>= 1) {
-        if (int(threadIdx.x) < k) red[threadIdx.x] += red[threadIdx.x + k];
-        __syncthreads();
+    block_sum(s);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(part + blockIdx.x, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+    __syncthreads();
+    if (!last) return;  // block-uniform
+    s = 0;
+    for (unsigned b = threadIdx.x; b < gridDim.x; b += NB)
+        s += __hip_atomic_load(part + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    block_sum(s);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+        const double rms = sqrt(red[0] / count);
+        scale[0] = rms;
+        scale[1] = rms > 0 ? 1.0 / rms : 0.0;
+    }
 }
 
 struct PackArgs {
@@ -273,8 +296,36 @@ struct PackArgs {
     int A1, A2, N3, Cin;
     const void* kx;
     const void* ky;
-    double kxmax, kymax, sinv;
+    int three;
+    const double* scale;  // RMS and its inverse (k_rms)
 };
+
+// a field component scaled to FP32 and then rounded to BF16: two roundings, which
+// the compiler may not merge into one of the FP64 product
+__device__ __forceinline__ bf16 input_value(double x, double sinv) {
+    return bf16(__builtin_canonicalizef(float(x * sinv)));
+}
+
+// input channel c of a mode at height z: Re and Im of the fields over their
+// RMS, then kx and ky over their largest active values (kx rises with j1; the
+// largest ky is that of the last positive row)
+template <typename T>
+__device__ __forceinline__ bf16 input_channel(const PackArgs& A, int c, int ja, int j1, int z) {
+    float v = 0.f;
+    if (c < 2 * A.nf) {
+        const cx<T> x = static_cast<const cx<T>*>(A.f[c >> 1])[sidx(ja, z, j1, A.N3, A.A1)];
+        return input_value(double((c & 1) ? x.y : x.x), A.scale[1]);
+    } else if (c == 2 * A.nf) {
+        const T* kx = static_cast<const T*>(A.kx);
+        const double m = fabs(double(kx[A.A1 - 1]));
+        v = __builtin_canonicalizef(float(double(kx[j1]) / (m > 0 ? m : 1.0)));
+    } else if (c == 2 * A.nf + 1 && A.three) {
+        const T* ky = static_cast<const T*>(A.ky);
+        const double m = fabs(double(ky[(A.A2 - 1) / 2]));
+        v = __builtin_canonicalizef(float(double(ky[ja]) / (m > 0 ? m : 1.0)));
+    }
+    return bf16(v);
+}
 
 // network input: in[p = (ja*A1 + j1)*N3 + z][c]
 template <typename T>
@@ -287,22 +338,12 @@ __global__ __launch_bounds__(NB) void k_pack(PackArgs A, bf16* __restrict__ in) 
         const int z = int(p % size_t(A.N3));
         const size_t mode = p / size_t(A.N3);
         const int j1 = int(mode % size_t(A.A1)), ja = int(mode / size_t(A.A1));
-        float v = 0.f;
-        if (c < 2 * A.nf) {
-            const cx<T> x = static_cast<const cx<T>*>(A.f[c >> 1])[sidx(ja, z, j1, A.N3, A.A1)];
-            v = float(double((c & 1) ? x.y : x.x) * A.sinv);
-        } else if (c == 2 * A.nf) {
-            v = float(double(static_cast<const T*>(A.kx)[j1]) / A.kxmax);
-        } else if (c == 2 * A.nf + 1 && A.kymax > 0) {
-            v = float(double(static_cast<const T*>(A.ky)[ja]) / A.kymax);
-        }
-        in[e] = bf16(v);
+        in[e] = input_channel<T>(A, c, ja, j1, z);
     }
 }
 
 // training target: q / RMS(q) - w / RMS(w) on the real output channels (the
-// direction of A^-1 w at the scale of w, minus w; W.sinv and Q.sinv hold the
-// two inverse RMS values)
+// direction of A^-1 w at the scale of w, minus w)
 template <typename T>
 __global__ __launch_bounds__(NB) void k_pack_target(PackArgs W, PackArgs Q, int Cout, float* __restrict__ tgt) {
     const size_t P = size_t(W.A1) * W.A2 * W.N3;
@@ -318,31 +359,150 @@ __global__ __launch_bounds__(NB) void k_pack_target(PackArgs W, PackArgs Q, int 
             const size_t o = sidx(ja, z, j1, W.N3, W.A1);
             const cx<T> w = static_cast<const cx<T>*>(W.f[c >> 1])[o];
             const cx<T> q = static_cast<const cx<T>*>(Q.f[c >> 1])[o];
-            v = float((c & 1) ? double(q.y) * Q.sinv - double(w.y) * W.sinv : double(q.x) * Q.sinv - double(w.x) * W.sinv);
+            const double qi = Q.scale[1], wi = W.scale[1];
+            v = float((c & 1) ? double(q.y) * qi - double(w.y) * wi : double(q.x) * qi - double(w.x) * wi);
         }
         tgt[e] = v;
     }
 }
 
-// out_f = in_f + s * (y[p][2f] + i y[p][2f+1])
-template <typename T>
-__global__ __launch_bounds__(NB) void k_unpack(PackArgs A, const float* __restrict__ y, int Cout, double s, cx<T>* o0,
-                                               cx<T>* o1, cx<T>* o2, cx<T>* o3) {
-    const size_t P = size_t(A.A1) * A.A2 * A.N3;
-    cx<T>* outs[4] = {o0, o1, o2, o3};
-    for (size_t p = size_t(blockIdx.x) * NB + threadIdx.x; p < P; p += size_t(gridDim.x) * NB) {
-        const int z = int(p % size_t(A.N3));
-        const size_t mode = p / size_t(A.N3);
-        const int j1 = int(mode % size_t(A.A1)), ja = int(mode / size_t(A.A1));
-        const size_t o = sidx(ja, z, j1, A.N3, A.A1);
-        for (int k = 0; k < A.nf; ++k) {
-            const cx<T> x = static_cast<const cx<T>*>(A.f[k])[o];
-            cx<T> r;
-            r.x = T(double(x.x) + s * double(y[p * Cout + 2 * k]));
-            r.y = T(double(x.y) + s * double(y[p * Cout + 2 * k + 1]));
-            outs[k][o] = r;
+// ---------------------------------------------------------------------------
+// The whole preconditioner of one mode in one block: out = in + s net(in / s).
+//
+// A profile is short (N3 <= 512 positions x 64 channels, 74 KB in BF16), so its
+// activations stay in LDS from the packed input to the last layer, which reads
+// and writes one buffer in place: every wave holds the results of its positions
+// in accumulators until all waves have read the layer's input.  A wave takes 64
+// positions and half of the channels (four by two MFMA tiles): per K step it
+// reads four fragments from LDS and two of the weights through L1, so that
+// both paths and the matrix cores are equally busy (with 16 positions and all
+// channels per wave the weights are read four times as often: 59 against 23 us).
+// Rows of 8 extra channels keep the fragments' 16-byte reads off each other's
+// banks; PADROWS rows of zeros on both sides are the convolution's padding.
+// Layer by layer through HBM took a pack, four convolutions of 11-17 us, an
+// unpack and a wait for the RMS (89 us at 256x1x256 FP64, 85 profiles); the order
+// of the accumulation is k_conv's, so the results are the same bits.
+// ---------------------------------------------------------------------------
+constexpr int PADROWS = 2 * NET_DMAX;
+constexpr int FUSED_POS = 4;  // tiles of 16 positions per wave
+constexpr int LAYERS_MAX = 8;
+
+struct FusedArgs {
+    PackArgs P;
+    void* out[4];
+    int L, Z, pitch;  // pitch: channels per row of LDS
+    int C[LAYERS_MAX + 1], dil[LAYERS_MAX];
+    const bf16* W[LAYERS_MAX];
+    const float* bias[LAYERS_MAX];
+};
+
+// accumulates a layer for 64 positions from p0 and NT tiles of 16 channels from
+// j0 on
+template <int CIN, int NT>
+__device__ __forceinline__ void fused_layer(const bf16* act, int pitch, const bf16* __restrict__ W, int Cout, int dil,
+                                            int p0, int j0, int Z, f32x4 (&acc)[FUSED_POS][2]) {
+    const int lane = threadIdx.x & 63;
+    const int m = lane & 15, kg = lane >> 4;
+    const bf16* wl = W + size_t(j0 * 16 + m) * CIN + kg * 8;
+    const bf16* al[FUSED_POS];
+#pragma unroll
+    for (int q = 0; q < FUSED_POS; ++q)  // past the column: rows whose results are dropped
+        al[q] = act + (PADROWS + min(p0 + q * 16 + m, Z - 1) - 2 * dil) * pitch + kg * 8;
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int c0 = 0; c0 < CIN; c0 += 32) {
+            bf16x8 w[NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) w[j] = ld8(wl + (size_t(t) * Cout + j * 16) * CIN + c0);
+#pragma unroll
+            for (int q = 0; q < FUSED_POS; ++q) {
+                const bf16x8 a = ld8(al[q] + t * dil * pitch + c0);
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[q][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[j], acc[q][j], 0, 0, 0);
+            }
         }
+}
+
+// two waves per 64 positions, one per half of the channels
+template <typename T>
+__global__ __launch_bounds__(1024) void k_net_fused(FusedArgs A) {
+    extern __shared__ __align__(16) unsigned char net_lds[];
+    bf16* act = reinterpret_cast<bf16*>(net_lds);  // [PADROWS + Z + PADROWS][pitch]
+    const int Z = A.Z, pitch = A.pitch, nf = A.P.nf;
+    const int ja = blockIdx.x / A.P.A1, j1 = blockIdx.x - ja * A.P.A1;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const int p0 = (wave >> 1) * 16 * FUSED_POS, half = wave & 1;
+    for (int i = threadIdx.x; i < nf * Z; i += blockDim.x) {
+        const int k = i / Z, z = i - k * Z;
+        bf16* a = act + (PADROWS + z) * pitch + 2 * k;
+        const cx<T> x = static_cast<const cx<T>*>(A.P.f[k])[sidx(ja, z, j1, Z, A.P.A1)];
+        a[0] = input_value(double(x.x), A.P.scale[1]);
+        a[1] = input_value(double(x.y), A.P.scale[1]);
     }
+    const bf16 kxc = input_channel<T>(A.P, 2 * nf, ja, j1, 0), kyc = input_channel<T>(A.P, 2 * nf + 1, ja, j1, 0);
+    for (int z = threadIdx.x; z < Z; z += blockDim.x) {
+        bf16* a = act + (PADROWS + z) * pitch;
+        a[2 * nf] = kxc;
+        a[2 * nf + 1] = kyc;
+        for (int c = 2 * nf + 2; c < A.C[0]; ++c) a[c] = bf16(0.f);
+    }
+    for (int i = threadIdx.x; i < PADROWS * pitch; i += blockDim.x) {
+        act[i] = bf16(0.f);
+        act[(PADROWS + Z) * pitch + i] = bf16(0.f);
+    }
+    __syncthreads();
+    const int n = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;  // accumulator: rows g*4.. of column n
+    f32x4 acc[FUSED_POS][2];
+    for (int l = 0; l < A.L; ++l) {
+        const bool last = l == A.L - 1;
+#pragma unroll
+        for (int q = 0; q < FUSED_POS; ++q)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[q][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int Cout = A.C[l + 1];
+        // channel tiles of this wave; the real channels of the last layer are the
+        // first eight at most
+        const int NT = last ? 1 - half : Cout / 32, j0 = half * NT;
+        if (NT == 2) {
+            if (A.C[l] == 64) fused_layer<64, 2>(act, pitch, A.W[l], Cout, A.dil[l], p0, j0, Z, acc);
+            else fused_layer<32, 2>(act, pitch, A.W[l], Cout, A.dil[l], p0, j0, Z, acc);
+        } else if (NT == 1) {
+            if (A.C[l] == 64) fused_layer<64, 1>(act, pitch, A.W[l], Cout, A.dil[l], p0, j0, Z, acc);
+            else fused_layer<32, 1>(act, pitch, A.W[l], Cout, A.dil[l], p0, j0, Z, acc);
+        }
+        if (last) break;
+        __syncthreads();  // every wave has read the layer's input
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (j >= NT) break;
+            const int co = (j0 + j) * 16 + n;
+            const float bias = A.bias[l][co];
+#pragma unroll
+            for (int q = 0; q < FUSED_POS; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int z = p0 + q * 16 + g * 4 + i;
+                    if (z < Z) act[(PADROWS + z) * pitch + co] = bf16(fmaxf(acc[q][j][i] + bias, 0.f));
+                }
+        }
+        __syncthreads();
+    }
+    if (half || n >= 2 * nf) return;
+    const double s = A.P.scale[0];
+    const float bias = A.bias[A.L - 1][n];
+    const T* in = static_cast<const T*>(A.P.f[n >> 1]);
+    T* out = static_cast<T*>(A.out[n >> 1]);
+#pragma unroll
+    for (int q = 0; q < FUSED_POS; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int z = p0 + q * 16 + g * 4 + i;
+            if (z >= Z) continue;
+            const size_t o = 2 * sidx(ja, z, j1, Z, A.P.A1) + (n & 1);
+            out[o] = T(double(in[o]) + s * double(acc[q][0][i] + bias));
+        }
 }
 
 // gather training profiles idx[] into a contiguous batch
@@ -405,6 +565,8 @@ struct Net {
     float* part = nullptr;
     size_t part_n = 0;
     double* dpart = nullptr;
+    unsigned* ticket = nullptr;  // of k_rms's blocks
+    double* scale = nullptr;     // its results, for two inputs
     int* didx = nullptr;
     int didx_n = 0;
     static constexpr int DW_BLOCKS = 240;
@@ -424,6 +586,8 @@ struct Net {
         F(set_t);
         free_work();
         F(dpart);
+        F(ticket);
+        F(scale);
         F(didx);
     }
     void free_work() {
@@ -498,6 +662,8 @@ struct Net {
             Wt.push_back(dalloc<bf16>(size_t(KT) * C[l + 1] * C[l]));
         }
         dpart = dalloc<double>(4096);
+        ticket = dalloc<unsigned>(1);
+        scale = dalloc<double>(4);
         cast_weights();
         SF_HIP(hipStreamSynchronize(st()));
     }
@@ -601,7 +767,7 @@ struct Net {
     }
 
     template <typename T>
-    PackArgs pack_args(sf_field* const* f, double sinv) const {
+    PackArgs pack_args(sf_field* const* f, const double* sc) const {
         PackArgs A{};
         int k = 0;
         for (int i = 0; i < 4; ++i) {
@@ -616,23 +782,14 @@ struct Net {
         A.Cin = C[0];
         A.kx = info.kx;
         A.ky = info.ky;
-        A.kxmax = kmax<T>(info.kx, info.A1);
-        A.kymax = info.three ? kmax<T>(info.ky, info.A2) : 0.0;
-        A.sinv = sinv;
+        A.three = info.three ? 1 : 0;
+        A.scale = sc;
         return A;
     }
 
+    // RMS of the fields and its inverse into sc[0..1] on the device
     template <typename T>
-    double kmax(const void* k, int n) const {
-        std::vector<T> h(n);
-        SF_HIP(hipMemcpy(h.data(), k, n * sizeof(T), hipMemcpyDeviceToHost));
-        double m = 0;
-        for (T x : h) m = std::max(m, std::fabs(double(x)));
-        return m > 0 ? m : 1.0;
-    }
-
-    template <typename T>
-    double rms(sf_field* const* f) {
+    void rms(sf_field* const* f, double* sc) {
         const size_t n = size_t(info.A1) * info.A2 * info.N3;
         const cx<T>* p[4] = {nullptr, nullptr, nullptr, nullptr};
         int nf_ = 0;
@@ -641,35 +798,38 @@ struct Net {
                 p[i] = static_cast<const cx<T>*>(f[i]->d);
                 ++nf_;
             }
-        const unsigned g = grid_for(n, 1024);
-        hipLaunchKernelGGL((k_sumsq<T>), dim3(g), dim3(NB), 0, st(), p[0], p[1], p[2], p[3], n, dpart);
+        hipLaunchKernelGGL((k_rms<T>), dim3(grid_for(n, 1024)), dim3(NB), 0, st(), p[0], p[1], p[2], p[3], n,
+                           double(n * size_t(nf_)), dpart, ticket, sc);
         SF_HIP(hipGetLastError());
-        std::vector<double> h(g);
-        SF_HIP(hipMemcpyAsync(h.data(), dpart, g * sizeof(double), hipMemcpyDeviceToHost, st()));
-        SF_HIP(hipStreamSynchronize(st()));
-        double s = 0;
-        for (double x : h) s += x;
-        return std::sqrt(s / double(n * size_t(nf_)));
     }
 
     template <typename T>
     void apply(sf_field* const* in, sf_field* const* out) {
-        const int P = int(profiles()) * Z;
-        ensure_work(size_t(P));
-        const double s = rms<T>(in);
-        PackArgs A = pack_args<T>(in, s > 0 ? 1.0 / s : 0.0);
-        hipLaunchKernelGGL((k_pack<T>), dim3(grid_for(size_t(P) * C[0])), dim3(NB), 0, st(), A, act[0]);
-        SF_HIP(hipGetLastError());
-        forward(P);
-        cx<T>* o[4] = {nullptr, nullptr, nullptr, nullptr};
+        FusedArgs A{};
+        A.P = pack_args<T>(in, scale);
         int k = 0;
         for (int i = 0; i < 4; ++i) {
             if (!info.three && i == 1) continue;
             SF_REQUIRE(out[i] != nullptr, SF_ERR_ARG, "missing output field");
-            o[k++] = static_cast<cx<T>*>(out[i]->d);
+            A.out[k++] = out[i]->d;
         }
-        hipLaunchKernelGGL((k_unpack<T>), dim3(grid_for(size_t(P))), dim3(NB), 0, st(), A, pre[L - 1], C[L], s, o[0],
-                           o[1], o[2], o[3]);
+        A.L = L;
+        A.Z = Z;
+        A.pitch = std::max(C[0], H) + 8;
+        for (int l = 0; l <= L; ++l) A.C[l] = C[l];
+        for (int l = 0; l < L; ++l) {
+            A.dil[l] = dil[l];
+            A.W[l] = Wb[l];
+            A.bias[l] = w + boff[l];
+        }
+        rms<T>(in, scale);
+        const dim3 grid(static_cast<unsigned>(profiles()));
+        const unsigned threads = 128u * unsigned((Z + 16 * FUSED_POS - 1) / (16 * FUSED_POS));  // N3 <= 512: at most 1024
+        const size_t lds = size_t(Z + 2 * PADROWS) * A.pitch * sizeof(bf16);                    // at most 77 KB
+        if (lds > 64 * 1024)
+            SF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_net_fused<T>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        hipLaunchKernelGGL((k_net_fused<T>), grid, dim3(threads), lds, st(), A);
         SF_HIP(hipGetLastError());
     }
 
@@ -695,10 +855,14 @@ struct Net {
     void add_pair(sf_field* const* wf, sf_field* const* qf) {
         const int np = int(profiles());
         grow_set(np);
-        const double s = rms<T>(wf), sq = rms<T>(qf);
-        if (!(s > 0) || !(sq > 0)) return;
-        PackArgs W = pack_args<T>(wf, 1.0 / s);
-        PackArgs Q = pack_args<T>(qf, 1.0 / sq);
+        PackArgs W = pack_args<T>(wf, scale);
+        PackArgs Q = pack_args<T>(qf, scale + 2);
+        rms<T>(wf, scale);
+        rms<T>(qf, scale + 2);
+        double sc[4];
+        SF_HIP(hipMemcpyAsync(sc, scale, sizeof(sc), hipMemcpyDeviceToHost, st()));
+        SF_HIP(hipStreamSynchronize(st()));
+        if (!(sc[0] > 0) || !(sc[2] > 0)) return;
         bf16* di = set_in + size_t(set_n) * Z * C[0];
         float* dt = set_t + size_t(set_n) * Z * C[L];
         const size_t P = size_t(np) * Z;

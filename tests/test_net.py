@@ -134,3 +134,54 @@ def test_training_lowers_loss_and_identity_until_trained():
     l0, l1 = net.train(epochs=60, batch=32, lr=2e-3)
     print("loss first epoch %.4e last %.4e" % (l0, l1))
     assert l1 < 0.1 * l0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,prec,hidden,layers", [((6, 1, 8, 1), 8, 64, 2), ((12, 1, 20, 1), 4, 32, 3),
+                                                      ((48, 1, 64, 1), 8, 64, 4), ((24, 1, 100, 1), 4, 64, 8),
+                                                      ((24, 1, 256, 1), 8, 64, 4), ((24, 1, 260, 1), 8, 32, 5),
+                                                      ((12, 1, 512, 1), 4, 64, 4), ((24, 12, 36, 0), 8, 64, 4)])
+def test_fused_application_matches_layers(shape, prec, hidden, layers):
+    """apply() keeps a profile in LDS through all layers; the layer-by-layer
+    forward pass of the packed input gives the same correction: fewer positions
+    than a wave's tile, ragged tiles, one and two tiles per wave, both widths,
+    the fewest and most layers, the largest dilation, 2D and 3D."""
+    import stratiflow_amd as sf
+    N1, N2, N3, dim = shape
+    s = sf.IMEXRK(N1, N2, N3, dim, 2 * np.pi / 0.44, np.pi / 0.44, 10.0, 1000.0, 0.1, 1.0, precision=prec)
+    net = sf.Net(s, hidden=hidden, layers=layers, seed=3)
+    net.set_dilations([1, 2, 4, 8, 1, 3, 8, 1][:layers])
+    rng = np.random.default_rng(2)
+    names = ("u1", "u2", "u3", "b") if dim == 0 else ("u1", "u3", "b")
+    nf = len(names)
+    net.set_params(_rand_params(rng, net.channels, 2 * nf + 2, 2 * nf).astype(np.float32))
+    fin, fout, a = {}, {}, {}
+    for n in names:
+        bc = sf.DIRICHLET if n == "u3" else sf.NEUMANN
+        fin[n], fout[n] = s.field(sf.MODAL, bc), s.field(sf.MODAL, bc)
+        fin[n].upload(rng.standard_normal(fin[n].shape) + 1j * rng.standard_normal(fin[n].shape))
+        a[n] = fin[n].download()
+    order = ("u1", "u2", "u3", "b")
+    net.apply([fin.get(n) for n in order], [fout.get(n) for n in order])
+    A1, h = N1 // 3, N2 // 3
+    rows = list(range(h)) + list(range(N2 - h + 1, N2)) if dim == 0 else [0]
+    act = {n: a[n][rows][:, :A1].reshape(len(rows) * A1, N3) for n in names}
+    rms = np.sqrt(sum((np.abs(v) ** 2).sum() for v in act.values()) / (nf * act["b"].size))
+    x = np.zeros((len(rows) * A1, N3, 32), np.float32)
+    for i, n in enumerate(names):
+        x[..., 2 * i], x[..., 2 * i + 1] = act[n].real * (1 / rms), act[n].imag * (1 / rms)
+    x[..., 2 * nf] = np.tile(np.arange(A1) / (A1 - 1), len(rows))[:, None]
+    if dim == 0:
+        ky = np.array([j if j <= N2 // 2 else j - N2 for j in rows]) / (h - 1)
+        x[..., 2 * nf + 1] = np.repeat(ky, A1)[:, None]
+    y = net.forward_raw(x).astype(np.float64)
+    eps = np.finfo(np.float32 if prec == 4 else np.float64).eps
+    print(shape, prec, hidden, layers, flush=True)
+    for i, n in enumerate(names):
+        want = act[n] + rms * (y[..., 2 * i] + 1j * y[..., 2 * i + 1])
+        got = fout[n].download()[rows][:, :A1].reshape(want.shape)
+        # the sums differ by roundings of the RMS and of the result; an input within
+        # those of a BF16 rounding boundary may fall to its other side
+        off = np.abs(got - want) > 16 * eps * (np.abs(act[n]) + np.abs(want)).max()
+        assert off.mean() < 1e-3 and np.abs(got - want).max() <= 2.0 ** -7 * np.abs(want).max(), n
+    s.close()
