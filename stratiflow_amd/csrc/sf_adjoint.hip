@@ -3,13 +3,13 @@
 // IMEXRK.cpp:260-379).
 //
 // The context drives the step from the host (sf_api.hip): it interpolates the
-// direct state (k_lerp), adds the background velocity through a nodal round
-// trip (k_add_profile), transforms the direct state and its horizontal
-// derivatives to nodal space, forms every explicit adjoint term as a nodal
-// field in one pass (k_adj_products), transforms those to modal space and
-// combines them with their horizontal derivatives into the explicit terms
-// (k_adj_combine), which the stage kernel then consumes with its linear
-// buoyancy terms switched off.  All of these kernels are HBM-bound streams.
+// direct state with the background velocity (k_adj_lerp), transforms it and its
+// horizontal derivatives to nodal space, forms every explicit adjoint term as a
+// nodal field in one pass (k_adj_products) and transforms their sums and x
+// derivatives to the explicit terms, which the stage kernel then consumes with
+// its linear buoyancy terms switched off.  Each transform is one launch over
+// all its fields: at 96x48x128 the 76 launches of a stage that took the fields
+// one by one set its time.
 // The file also holds the small kernels of the diagnostics (JoverK, horizontal
 // averages) and of the field helpers (PhaseShift, RemoveAverage).
 #include "sf_kernels.h"
@@ -28,22 +28,43 @@ __host__ __device__ inline unsigned grid_of(size_t n) {
 }
 }  // namespace
 
-// out = (1 - f) * above + f * below (IMEXRK.h:98-101); a null input is zero
+// The direct state at a stage (IMEXRK.h:96-107): (1 - f) above + f below (a null
+// input is zero), with U_ added to the mean of u1.  The reference adds U_ in
+// nodal space and transforms back, which also leaves u1 the spectrum of a real
+// field: f(0, -j2) = conj f(0, j2).
 template <typename T>
-__global__ __launch_bounds__(ABS) void k_lerp(cx<T>* out, const cx<T>* above, const cx<T>* below, T f, size_t n) {
-    const T g = T(1) - f;
-    for (size_t i = size_t(blockIdx.x) * ABS + threadIdx.x; i < n; i += size_t(gridDim.x) * ABS) {
-        const cx<T> a = above ? above[i] : czero<cx<T>>();
-        const cx<T> b = below ? below[i] : czero<cx<T>>();
-        cx<T> r;
-        r.x = g * a.x + f * b.x;
-        r.y = g * a.y + f * b.y;
-        out[i] = r;
+__global__ __launch_bounds__(ABS) void k_adj_lerp(AdjLerp<T> A) {
+    using V = cx<T>;
+    const int i = blockIdx.y;
+    const V* above = A.above[i];
+    const V* below = A.below[i];
+    V* out = A.out[i];
+    if (out == nullptr) return;
+    const T f = A.f, g = T(1) - f;
+    auto lerp = [&](unsigned e) {
+        const V a = above ? above[e] : czero<V>();
+        const V b = below ? below[e] : czero<V>();
+        return mkc<T>(g * a.x + f * b.x, g * a.y + f * b.y);
+    };
+    const unsigned A1 = A.A1, N3 = A.N3;
+    for (unsigned e = blockIdx.x * ABS + threadIdx.x; e < A.n; e += gridDim.x * ABS) {
+        V r = lerp(e);
+        if (i == 0) {
+            const unsigned row = e / A1;
+            if (row * A1 == e) {  // j1 = 0
+                const unsigned ja = row / N3, z = row - ja * N3;
+                const unsigned other = ja == 0 ? 0 : A.A2 - ja;
+                const V c = lerp((other * N3 + z) * A1);
+                r = mkc<T>(T(0.5) * (r.x + c.x), T(0.5) * (r.y - c.y));
+                if (ja == 0) r.x += A.ubar[z];
+            }
+        }
+        out[e] = r;
     }
 }
 template <typename T>
-hipError_t launch_lerp(cx<T>* out, const cx<T>* above, const cx<T>* below, T f, size_t n, hipStream_t s) {
-    hipLaunchKernelGGL((k_lerp<T>), dim3(grid_of<T>(n)), dim3(ABS), 0, s, out, above, below, f, n);
+hipError_t launch_adj_lerp(const AdjLerp<T>& a, hipStream_t s) {
+    hipLaunchKernelGGL((k_adj_lerp<T>), dim3(grid_of<T>(a.n), 4), dim3(ABS), 0, s, a);
     return hipGetLastError();
 }
 
@@ -87,8 +108,9 @@ __global__ __launch_bounds__(ABS) void k_adj_products(const AdjArgs<T> A) {
     const int N = A.N3;
     const T* zc = A.zc;
     const int P = A.N3p;
-    for (size_t e = size_t(blockIdx.x) * ABS + threadIdx.x; e < A.n; e += size_t(gridDim.x) * ABS) {
-        const size_t o = e - e % size_t(N);
+    const unsigned n = unsigned(A.n);
+    for (unsigned e = blockIdx.x * ABS + threadIdx.x; e < n; e += gridDim.x * ABS) {
+        const unsigned o = e - e % unsigned(N);
         const int j = int(e - o);
         auto at = [&](const T* f, int jj) -> T { return f[o + jj]; };
         auto ibar = [&](const T* f, int jj) -> T {
@@ -179,43 +201,6 @@ hipError_t launch_adj_products(const AdjArgs<T>& a, bool three, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Explicit adjoint terms from the transformed products (modal layout
-// [ja][z][j1]):
-//   r1 = ikx M0 + M1 + iky M6,   r2 = iky M7 + ikx M8 + M9,
-//   r3 = ikx M2 + M3 + iky M10,  rB = ikx M4 + M5 + iky M11.
-template <typename T>
-__global__ __launch_bounds__(ABS) void k_adj_combine(AdjCombine<T> C) {
-    const size_t n = size_t(C.A1) * C.A2 * C.N3;
-    for (size_t e = size_t(blockIdx.x) * ABS + threadIdx.x; e < n; e += size_t(gridDim.x) * ABS) {
-        const size_t rowz = e / size_t(C.A1);
-        const int j1 = int(e - rowz * size_t(C.A1));
-        const int ja = int(rowz / size_t(C.N3));
-        const T kx = C.kx[j1], ky = C.ky[ja];
-        auto term = [&](int i, int kind) -> cx<T> {  // kind 0: ikx, 1: iky, 2: plain
-            const cx<T> v = C.M[i][e];
-            return kind == 0 ? cik(kx, v) : (kind == 1 ? cik(ky, v) : v);
-        };
-        cx<T> r1 = cadd(term(0, 0), term(1, 2));
-        cx<T> r3 = cadd(term(2, 0), term(3, 2));
-        cx<T> rB = cadd(term(4, 0), term(5, 2));
-        if (C.three) {
-            r1 = cadd(r1, term(6, 1));
-            r3 = cadd(r3, term(10, 1));
-            rB = cadd(rB, term(11, 1));
-            C.out[1][e] = cadd(cadd(term(7, 1), term(8, 0)), term(9, 2));
-        }
-        C.out[0][e] = r1;
-        C.out[2][e] = r3;
-        C.out[3][e] = rB;
-    }
-}
-template <typename T>
-hipError_t launch_adj_combine(const AdjCombine<T>& c, hipStream_t s) {
-    const size_t n = size_t(c.A1) * c.A2 * c.N3;
-    hipLaunchKernelGGL((k_adj_combine<T>), dim3(grid_of<T>(n)), dim3(ABS), 0, s, c);
-    return hipGetLastError();
-}
-
 // J integrand of UpdateAdjointVariables (IMEXRK.h:478-483): -(B - <b>) W with
 // <b> the real part of the (0,0) mode of the modal buoyancy
 template <typename T>
@@ -284,10 +269,9 @@ hipError_t launch_add_mean(cx<T>* f, int N3, int A1, T value, hipStream_t s) {
 }
 
 #define SF_ADJ_INST(T)                                                                                     \
-    template hipError_t launch_lerp<T>(cx<T>*, const cx<T>*, const cx<T>*, T, size_t, hipStream_t);       \
+    template hipError_t launch_adj_lerp<T>(const AdjLerp<T>&, hipStream_t);                                \
     template hipError_t launch_add_profile<T>(T*, const T*, size_t, int, hipStream_t);                    \
     template hipError_t launch_adj_products<T>(const AdjArgs<T>&, bool, hipStream_t);                     \
-    template hipError_t launch_adj_combine<T>(const AdjCombine<T>&, hipStream_t);                         \
     template hipError_t launch_mix_product<T>(T*, const T*, const T*, const cx<T>*, size_t, int, int, hipStream_t); \
     template hipError_t launch_mean_profile<T>(const cx<T>*, double*, int, int, hipStream_t);             \
     template hipError_t launch_phase_shift<T>(cx<T>*, size_t, int, double, hipStream_t);                    \

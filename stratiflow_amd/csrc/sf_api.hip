@@ -715,32 +715,107 @@ struct Ctx {
     }
 
     // ---- adjoint step (IMEXRK.h:86-126) ----
-    // nodal: direct totals, their horizontal derivatives, explicit terms;
-    // modal: transformed explicit terms and one derivative scratch field.
-    // Allocated on the first adjoint step.
+    // nodal direct totals, their horizontal derivatives and the explicit terms;
+    // allocated on the first adjoint step
     T* adjT[4] = {nullptr};
     T* adjDX[4] = {nullptr};
     T* adjDY[4] = {nullptr};
     T* adjQ[12] = {nullptr};
-    V* adjM[12] = {nullptr};
-    V* adjD = nullptr;
 
     int adj_terms() const { return three ? 12 : 6; }
     bool has_field(int i) const { return three || i != 1; }
 
     void adjoint_alloc() {
-        if (adjD) return;
+        if (adjQ[0]) return;
         for (int i = 0; i < 4; ++i) {
             if (!has_field(i)) continue;
             adjT[i] = dalloc<T>(nnodal);
             adjDX[i] = dalloc<T>(nnodal);
             if (three) adjDY[i] = dalloc<T>(nnodal);
         }
-        for (int q = 0; q < adj_terms(); ++q) {
-            adjQ[q] = dalloc<T>(nnodal);
-            adjM[q] = dalloc<V>(nmodal);
+        for (int q = 0; q < adj_terms(); ++q) adjQ[q] = dalloc<T>(nnodal);
+    }
+
+    // nodal totals and their horizontal derivatives (UpdateAdjointVariables,
+    // IMEXRK.h:461-500, and IMEXRK.cpp:312-360): in 3D one y transform of each
+    // total and of its y derivative, then one x transform of all, in which a
+    // total and its x derivative share their spectrum
+    void adjoint_totals(V* const tot[4]) {
+        XTArgs<T> x{};
+        x.N3 = N3;
+        x.A1 = A1;
+        x.tw = twx;
+        x.kx = kx;
+        x.scale = T(1);
+        YArgs<T> y{};
+        y.N3 = N3;
+        y.A1 = A1;
+        y.A2 = A2;
+        y.tw = tw2;
+        y.ky = ky;
+        y.scale = T(1);
+        auto add = [&](const V* spec, T* nodal, bool dx) {
+            x.spec[x.nf] = const_cast<V*>(spec);  // read
+            x.nodal[x.nf] = nodal;
+            if (dx) x.ikx |= 1u << x.nf;
+            ++x.nf;
+        };
+        for (int i = 0; i < 4; ++i) {
+            if (!has_field(i)) continue;
+            const V* spec = tot[i];
+            if (three) {
+                y.in[y.nf] = tot[i];
+                y.out[y.nf] = X[i];
+                ++y.nf;
+                y.in[y.nf] = tot[i];
+                y.out[y.nf] = X[4 + i];
+                y.iky |= 1u << y.nf;
+                ++y.nf;
+                spec = X[i];
+                add(X[4 + i], adjDY[i], false);
+            }
+            add(spec, adjT[i], false);
+            add(spec, adjDX[i], true);
         }
-        adjD = dalloc<V>(nmodal);
+        if (three) check(launch_yinv<T>(y, N2, stream), "adjoint:yinv");
+        check(launch_x_c2r<T>(x, N1, N2, stream), "adjoint:c2r");
+    }
+
+    // the explicit terms from their nodal products (k_adj_products):
+    //   r1 = ikx Q0 + Q1 + iky Q6,   r2 = ikx Q8 + Q9 + iky Q7,
+    //   r3 = ikx Q2 + Q3 + iky Q10,  rB = ikx Q4 + Q5 + iky Q11
+    void adjoint_rhs() {
+        static const int q[4][3] = {{1, 0, 6}, {9, 8, 7}, {3, 2, 10}, {5, 4, 11}};  // plain, ikx, iky
+        XSumArgs<T> x{};
+        x.N3 = N3;
+        x.A1 = A1;
+        x.tw = twx;
+        x.kx = kx;
+        x.scale = three ? T(1) : T(1.0 / double(N1));
+        for (int i = 0; i < 4; ++i) {
+            if (!has_field(i)) continue;
+            x.a[x.nf] = adjQ[q[i][0]];
+            x.b[x.nf] = adjQ[q[i][1]];
+            x.spec[x.nf++] = three ? X[2 * i] : nl[i];
+            if (three) {
+                x.a[x.nf] = adjQ[q[i][2]];
+                x.spec[x.nf++] = X[2 * i + 1];
+            }
+        }
+        check(launch_x_sum<T>(x, N1, N2, stream), "adjoint:r2c");
+        if (!three) return;
+        YArgs<T> y{};
+        y.N3 = N3;
+        y.A1 = A1;
+        y.A2 = A2;
+        y.nf = 4;
+        y.paired = 1;
+        for (int i = 0; i < 8; ++i) y.in[i] = X[i];
+        for (int i = 0; i < 4; ++i) y.out[i] = nl[i];
+        y.ky = ky;
+        y.tw = tw2;
+        y.scale = T(1.0 / (double(N1) * double(N2)));
+        check(launch_yfwd<T>(y, N2, stream), "adjoint:yfwd");
     }
 
     // below/above: the direct state (u1, u2, u3, b; device modal fields of this
@@ -748,37 +823,31 @@ struct Ctx {
     void step_adjoint(const V* const below[4], const V* const above[4]) {
         adjoint_alloc();
         V* tot[4] = {mf(SF_U1_TOT), mf(SF_U2_TOT), mf(SF_U3_TOT), mf(SF_B_TOT)};
-        T* nod[4] = {static_cast<T*>(state[SF_NODAL_U1].d), static_cast<T*>(state[SF_NODAL_U2].d),
-                     static_cast<T*>(state[SF_NODAL_U3].d), static_cast<T*>(state[SF_NODAL_B].d)};
         const T* ubar = zc + size_t(ZC_UBAR) * N3p;
         T frac = T(0);
         for (int k = 0; k < 3; ++k) {
             // the direct state at this stage, with the background velocity
-            // added through a nodal round trip (IMEXRK.h:96-107)
-            for (int i = 0; i < 4; ++i)
-                if (has_field(i)) check(launch_lerp<T>(tot[i], above[i], below[i], frac, nmodal, stream), "lerp");
-            to_nodal(tot[0], adjT[0]);
-            check(launch_add_profile<T>(adjT[0], ubar, nnodal, N3, stream), "add_profile");
-            to_modal(adjT[0], tot[0]);
-            // UpdateAdjointVariables (IMEXRK.h:461-500) and the nodal
-            // derivatives of BuildRHSAdjoint (IMEXRK.cpp:312-360)
+            AdjLerp<T> l{};
+            l.N3 = N3;
+            l.A1 = A1;
+            l.A2 = A2;
+            l.n = unsigned(nmodal);
+            l.f = frac;
+            l.ubar = ubar;
             for (int i = 0; i < 4; ++i) {
-                if (!has_field(i)) continue;
-                to_nodal(tot[i], adjT[i]);
-                check(launch_dmul<T>(adjD, tot[i], A1, A2, N3, kx, ky, 0, zc, N3p, stream), "ddx");
-                to_nodal(adjD, adjDX[i]);
-                if (three) {
-                    check(launch_dmul<T>(adjD, tot[i], A1, A2, N3, kx, ky, 1, zc, N3p, stream), "ddy");
-                    to_nodal(adjD, adjDY[i]);
-                }
+                l.above[i] = above[i];
+                l.below[i] = below[i];
+                l.out[i] = has_field(i) ? tot[i] : nullptr;
             }
+            check(launch_adj_lerp<T>(l, stream), "lerp");
+            adjoint_totals(tot);
             AdjArgs<T> a{};
             a.N3 = N3;
             a.N3p = N3p;
             a.A1 = A1;
             a.n = nnodal;
             for (int i = 0; i < 4; ++i) {
-                a.U[i] = has_field(i) ? nod[i] : nullptr;
+                a.U[i] = has_field(i) ? static_cast<T*>(state[SF_NODAL_U1 + i].d) : nullptr;
                 a.Tt[i] = adjT[i];
                 a.DX[i] = adjDX[i];
                 a.DY[i] = adjDY[i];
@@ -789,17 +858,7 @@ struct Ctx {
             a.Ri = T(Ri);
             for (int q = 0; q < adj_terms(); ++q) a.Q[q] = adjQ[q];
             check(launch_adj_products<T>(a, three, stream), "adj_products");
-            for (int q = 0; q < adj_terms(); ++q) to_modal(adjQ[q], adjM[q]);
-            AdjCombine<T> c{};
-            c.N3 = N3;
-            c.A1 = A1;
-            c.A2 = A2;
-            c.three = three ? 1 : 0;
-            c.kx = kx;
-            c.ky = ky;
-            for (int q = 0; q < adj_terms(); ++q) c.M[q] = adjM[q];
-            for (int i = 0; i < 4; ++i) c.out[i] = has_field(i) ? nl[i] : nullptr;
-            check(launch_adj_combine<T>(c, stream), "adj_combine");
+            adjoint_rhs();
             // ExplicitRK, FinishRHS, CrankNicolson, RemoveDivergence(1/h), FilterAll
             const bool store_r = k < 2;
             ModalArgs<T> m = stage_modal_args(k, store_r, rcur);

@@ -71,6 +71,7 @@ struct YArgs {
     T scale;
     int paired;       // forward: out[r] = scale*(F(in[2r]) + i ky F(in[2r+1]))
     int tiled;        // paired forward: inputs in tiles of 16 modes (ytile_idx)
+    unsigned iky;     // inverse: bit f set: field f is the y derivative of in[f]
 };
 
 // Offset of (n2, z, j1) in an x-spectral field stored in tiles of 16 modes,
@@ -90,6 +91,20 @@ struct XTArgs {
     cx<T>* spec[XT_MAX];
     T* nodal[XT_MAX];
     const cx<T>* tw;  // xt_twiddles
+    T scale;
+    unsigned ikx;  // c2r: bit f set: field f is the x derivative of its spectrum
+    const T* kx;
+};
+// forward x transforms of sums: spec[f] = scale*(F(a[f]) + ikx F(b[f])) (b null: F(a) alone)
+constexpr int XS_MAX = 8;
+template <typename T>
+struct XSumArgs {
+    int N3, A1, nf;
+    const T* a[XS_MAX];
+    const T* b[XS_MAX];
+    cx<T>* spec[XS_MAX];
+    const cx<T>* tw;
+    const T* kx;
     T scale;
 };
 
@@ -132,6 +147,8 @@ template <typename T>
 hipError_t launch_x_c2r(const XTArgs<T>& a, int N1, int N2, hipStream_t s);
 template <typename T>
 hipError_t launch_x_r2c(const XTArgs<T>& a, int N1, int N2, hipStream_t s);
+template <typename T>
+hipError_t launch_x_sum(const XSumArgs<T>& a, int N1, int N2, hipStream_t s);
 // FP64 inner products (sf_fields.hip): one launch for up to DOT_MAX pairs,
 // results and then the sequence number of the call in pinned host memory
 constexpr int DOT_MAX = 4;
@@ -212,21 +229,23 @@ struct AdjArgs {
     T Ri;
     T* Q[12];            // nodal explicit terms
 };
+// direct state at a stage: out[i] = (1-f) above[i] + f below[i], plus U_ on u1
 template <typename T>
-struct AdjCombine {
-    int N3, A1, A2, three;
-    const T *kx, *ky;
-    const cx<T>* M[12];  // modal transforms of the nodal explicit terms
-    cx<T>* out[4];       // explicit terms r1, r2, r3, rB
+struct AdjLerp {
+    int N3, A1, A2;
+    unsigned n;  // A1*A2*N3
+    T f;
+    const T* ubar;
+    const cx<T>* above[4];
+    const cx<T>* below[4];
+    cx<T>* out[4];  // null: absent
 };
 template <typename T>
-hipError_t launch_lerp(cx<T>* out, const cx<T>* above, const cx<T>* below, T f, size_t n, hipStream_t s);
+hipError_t launch_adj_lerp(const AdjLerp<T>& a, hipStream_t s);
 template <typename T>
 hipError_t launch_add_profile(T* f, const T* prof, size_t n, int N3, hipStream_t s);
 template <typename T>
 hipError_t launch_adj_products(const AdjArgs<T>& a, bool three, hipStream_t s);
-template <typename T>
-hipError_t launch_adj_combine(const AdjCombine<T>& c, hipStream_t s);
 template <typename T>
 hipError_t launch_mix_product(T* out, const T* Bt, const T* Wt, const cx<T>* bt, size_t n, int N3, int A1,
                               hipStream_t s);

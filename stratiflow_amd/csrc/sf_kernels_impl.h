@@ -1184,7 +1184,7 @@ __global__ __launch_bounds__(BS) void k_yinv(YArgs<T> A) {
                 const int ja = rest % A2;
                 const int fl = rest / A2;
                 const int j2 = (ja < h) ? ja : ja + N2 - 2 * h + 1;
-                buf[(fl * YJ + jj) * LDP + j2] = g[i];
+                buf[(fl * YJ + jj) * LDP + j2] = ((A.iky >> (f0 + fl)) & 1) ? cik(A.ky[ja], g[i]) : g[i];
             }
         }
         sync_lds();
@@ -1400,6 +1400,14 @@ __global__ __launch_bounds__(BS) void k_yinv_dma(YArgs<T> A) {
         }
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
+        if ((A.iky >> f) & 1) {  // block-uniform
+            for (int idx = threadIdx.x; idx < A2 * YJ; idx += BS) {
+                const int ja = idx / YJ;
+                V& v = buf[(ja < h ? ja : ja + nband) * YJ + idx % YJ];
+                v = cik(A.ky[ja], v);
+            }
+            sync_lds();
+        }
         lds_fft_lines<T, N2, YJ, BS, +1, YJ, true>(YJ, [&](int line) { return buf + line; }, A.tw);
         const rsrc_t o = make_rsrc(A.out[f], ybytes);
         for (int idx = threadIdx.x; idx < N2 * YJ; idx += BS) {

@@ -45,6 +45,7 @@ __global__ __launch_bounds__(BS) void k_x_c2r(XTArgs<T> A) {
     const V* __restrict__ in = A.spec[blockIdx.z];
     T* __restrict__ out = A.nodal[blockIdx.z];
     const V* __restrict__ wt = A.tw + 2 * M;
+    const bool dx = (A.ikx >> blockIdx.z) & 1;
     // modes k and M - k of a level give points k and M - k of its line:
     //   Z_k = (X_k + conj X_{M-k}) + i conj(w^k) (X_k - conj X_{M-k})
     constexpr int H = M / 2 + 1;
@@ -57,6 +58,10 @@ __global__ __launch_bounds__(BS) void k_x_c2r(XTArgs<T> A) {
             const V* X = in + sidx(n2, z, 0, N3, A1);
             if (k < A1) a = X[k];
             if (M - k < A1) b = X[M - k];
+        }
+        if (dx) {  // ikx X
+            a = cik(A.kx[min(k, A1 - 1)], a);
+            b = cik(A.kx[min(M - k, A1 - 1)], b);
         }
         if (k == 0) a.y = 0;  // c2r ignores the imaginary part of the DC term
         V* L = buf + t * LDP;
@@ -123,6 +128,80 @@ __global__ __launch_bounds__(BS) void k_x_r2c(XTArgs<T> A) {
     }
 }
 
+// spec = scale*(F(a) + ikx F(b)): a transform of b whose modes wait in registers
+// for the transform of a, so that a sum of two nodal fields leaves as one
+// spectrum
+template <typename T, int N1>
+__global__ __launch_bounds__(BS) void k_x_sum(XSumArgs<T> A) {
+    using V = cx<T>;
+    constexpr int M = N1 / 2, LDP = xt_ldp<M>(), NL = xt_levels<T, N1>();
+    constexpr int PER = (NL * (N1 / 3) + BS - 1) / BS;  // modes per thread
+    __shared__ V buf[NL * LDP];
+    const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    const int n2 = tile / gridDim.x, z0 = (tile % gridDim.x) * NL;
+    const int N3 = A.N3, A1 = A.A1;
+    const V* __restrict__ wt = A.tw + 2 * M;
+    V sum[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) sum[i] = czero<V>();
+    const T h = T(0.5) * A.scale;
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+        const T* in = pass == 0 ? A.b[blockIdx.z] : A.a[blockIdx.z];
+        if (in == nullptr) continue;  // block-uniform
+        constexpr int P = NL / 2;
+#pragma unroll 4
+        for (int idx = threadIdx.x; idx < P * M; idx += BS) {
+            const int u = idx % P;
+            const int m = idx / P;
+            const int z = z0 + 2 * u;
+            V a = czero<V>(), b = czero<V>();
+            if (z < N3) {
+                const T* i = in + (size_t(n2) * N1 + 2 * m) * N3 + z;
+                a = *reinterpret_cast<const V*>(i);
+                b = *reinterpret_cast<const V*>(i + N3);
+            }
+            buf[2 * u * LDP + m] = mkc<T>(a.x, b.x);
+            buf[(2 * u + 1) * LDP + m] = mkc<T>(a.y, b.y);
+        }
+        sync_lds();
+        lds_fft_lines<T, M, NL, BS, -1>(NL, [&](int line) { return buf + line * LDP; }, A.tw);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int idx = int(threadIdx.x) + i * BS;
+            const int t = idx / A1;
+            const int k = idx - t * A1;
+            if (t >= NL) continue;
+            const V Z = buf[t * LDP + k], W = buf[t * LDP + (k ? M - k : 0)];
+            const V s = mkc<T>(Z.x + W.x, Z.y - W.y), d = mkc<T>(Z.x - W.x, Z.y + W.y);
+            const V o = cmul(d, wt[k]);
+            const V x = mkc<T>(h * (s.x + o.y), h * (s.y - o.x));
+            if (pass == 0) {
+                sum[i] = cik(A.kx[k], x);
+            } else if (z0 + t < N3) {
+                A.spec[blockIdx.z][sidx(n2, z0 + t, k, N3, A1)] = cadd(sum[i], x);
+            }
+        }
+        sync_lds();
+    }
+}
+
+template <typename T>
+hipError_t launch_x_sum(const XSumArgs<T>& a, int N1, int N2, hipStream_t s) {
+    if (a.nf < 1 || a.nf > XS_MAX || a.N3 % 2 != 0 || a.A1 > N1 / 3) return hipErrorInvalidValue;
+    switch (N1) {
+#define SF_CASE(n)                                                                                                 \
+    case n:                                                                                                        \
+        hipLaunchKernelGGL((k_x_sum<T, n>), dim3((a.N3 + xt_levels<T, n>() - 1) / xt_levels<T, n>(), N2, a.nf),    \
+                           dim3(BS), 0, s, a);                                                                     \
+        return hipGetLastError();
+        SF_SIZES(SF_CASE)
+#undef SF_CASE
+        default:
+            return hipErrorInvalidValue;
+    }
+}
+
 template <typename T, int N1>
 static hipError_t launch_xt_n(const XTArgs<T>& a, int N2, bool c2r, hipStream_t s) {
     constexpr int NL = xt_levels<T, N1>();
@@ -179,7 +258,8 @@ void xt_twiddles(int n, double* re, double* im) {
 
 #define SF_TRANSFORM_INST(T)                                                     \
     template hipError_t launch_x_c2r<T>(const XTArgs<T>&, int, int, hipStream_t); \
-    template hipError_t launch_x_r2c<T>(const XTArgs<T>&, int, int, hipStream_t);
+    template hipError_t launch_x_r2c<T>(const XTArgs<T>&, int, int, hipStream_t); \
+    template hipError_t launch_x_sum<T>(const XSumArgs<T>&, int, int, hipStream_t);
 
 SF_TRANSFORM_INST(float)
 SF_TRANSFORM_INST(double)

@@ -297,3 +297,19 @@ def test_gpu_adjoint_step_matches_oracle(dim, N1, N2, N3, prec, tol):
         err = np.abs(got[n] - want[n]).max() / scale
         print("  %s max rel err %.3e (scale %.3e)" % (n, err, scale))
         assert err < tol, (n, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,N1,N2,N3", [(O.TWO_D, 6, 1, 12), (O.TWO_D, 256, 1, 36), (O.TWO_D, 384, 1, 24),
+                                          (O.THREE_D, 96, 48, 20), (O.THREE_D, 192, 12, 36), (O.THREE_D, 16, 24, 12)])
+def test_gpu_adjoint_step_on_every_transform_path(dim, N1, N2, N3):
+    """The batched transforms of the adjoint step: x lines of one and two passes,
+    16 and 8 levels per block with remainders, y tiles through LDS loads and
+    through registers (odd numbers of modes)."""
+    print("adjoint paths", dim, N1, N2, N3, flush=True)
+    got, want = _gpu_adjoint(N1, N2, N3, dim, 8, 1, dt=0.002)
+    for n in want:
+        err = np.abs(got[n] - want[n]).max() / np.abs(want[n]).max()
+        print("  %s %.3e" % (n, err), flush=True)
+        # one step of FP64 rounding (p: rescaled by 1/h)
+        assert err < (1e-10 if n == "p" else 1e-12), n
