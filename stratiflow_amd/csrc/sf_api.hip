@@ -92,6 +92,7 @@ struct Ctx {
     std::vector<void*> allocs;
 
     T* zc = nullptr;
+    T* zl = nullptr;  // zc in the order of the modal kernels' lanes (ModalArgs)
     T *kx = nullptr, *ky = nullptr, *kx2 = nullptr, *ky2 = nullptr;
     V *tw1 = nullptr, *tw2 = nullptr;
     V* twx = nullptr;  // of the whole-field x transforms
@@ -198,6 +199,7 @@ struct Ctx {
         std::memset(dot_host, 0, sizeof(DotResult));
 
         zc = dalloc<T>(size_t(ZC_COUNT) * N3p);
+        zl = dalloc<T>(size_t(ZC_COUNT) * 64 * rows_per_lane());
         kx = dalloc<T>(A1);
         kx2 = dalloc<T>(A1);
         ky = dalloc<T>(A2);
@@ -251,10 +253,17 @@ struct Ctx {
         for (int i = 0; i < 4; ++i) state[SF_R1 + i].d = rbuf[rcur][i];
     }
 
+    int rows_per_lane() const { return (N3 + 63) / 64; }
+
     void upload_coefficients() {
         std::vector<T> h(zc_host.size());
         for (size_t i = 0; i < h.size(); ++i) h[i] = T(zc_host[i]);
         SF_HIP(hipMemcpyAsync(zc, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, stream));
+        const int M = rows_per_lane();
+        std::vector<T> l(size_t(ZC_COUNT) * 64 * M, T(0));
+        for (int c = 0; c < ZC_COUNT; ++c)
+            for (int j = 0; j < N3; ++j) l[(size_t(c) * M + j % M) * 64 + j / M] = h[size_t(c) * N3p + j];
+        SF_HIP(hipMemcpyAsync(zl, l.data(), l.size() * sizeof(T), hipMemcpyHostToDevice, stream));
         SF_HIP(hipStreamSynchronize(stream));
     }
 
@@ -556,7 +565,7 @@ struct Ctx {
         m.A2 = A2;
         m.nmodes = A1 * A2;
         m.threeD = three ? 1 : 0;
-        m.zc = zc;
+        m.zl = zl;
         m.kx = kx;
         m.ky = ky;
         m.kx2 = kx2;

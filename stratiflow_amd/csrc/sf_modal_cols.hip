@@ -44,15 +44,14 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
     }
     const bool step = A.mode == 0;
 
-    int row[M], zoff[M], foff[M];
+    int row[M], foff[M];
 #pragma unroll
     for (int t = 0; t < M; ++t) {
         row[t] = lane * M + t;
-        zoff[t] = row[t] < N ? row[t] * int(sizeof(T)) : BUF_OOB;
         foff[t] = row[t] < N ? int(sidx(ja, row[t], j1, N, A1) * sizeof(V)) : BUF_OOB;
     }
-    const rsrc_t zr = make_rsrc(A.zc, size_t(ZC_COUNT) * A.N3p * sizeof(T));
-    auto coefz = [&](int c, int t) -> T { return bld<T>(zr, zoff[t], c * A.N3p * int(sizeof(T))); };
+    const rsrc_t zr = make_rsrc(A.zl, size_t(ZC_COUNT) * M * 64 * sizeof(T));
+    auto coefz = [&](int c, int t) -> T { return bld<T>(zr, lane * int(sizeof(T)), (c * M + t) * 64 * int(sizeof(T))); };
     const size_t fbytes = size_t(A1) * size_t(A.A2) * size_t(N) * sizeof(V);
     auto load = [&](const V* f, V (&g)[M]) {
         if (f == nullptr) {  // wave-uniform
@@ -134,7 +133,7 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
                 if (wave == CW_U3) {
                     V bb[M], bm[M];
                     get(CW_B, bb);
-                    nb_prev<T, M>(bb, bm, lane);
+                    nb_prev(bb, bm, lane);
                     if (!zero_mode) {
 #pragma unroll
                         for (int t = 0; t < M; ++t) {
@@ -145,7 +144,7 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
                 } else if (wave == CW_B) {
                     V u3[M], u3p[M];
                     get(CW_U3, u3);
-                    nb_next<T, M>(u3, u3p, lane);
+                    nb_next(u3, u3p, lane);
 #pragma unroll
                     for (int t = 0; t < M; ++t) {
                         const V idr = cadd(cscale(T(0.5), u3[t]), cscale(T(0.5), u3p[t]));
@@ -158,7 +157,7 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
             get(CW_P, pp);
             if (wave == CW_U3) {
                 V pm[M];
-                nb_prev<T, M>(pp, pm, lane);
+                nb_prev(pp, pm, lane);
 #pragma unroll
                 for (int t = 0; t < M; ++t) gp[t] = tscale(z2[t], csub(pp[t], pm[t]));
             } else {
@@ -169,8 +168,8 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
             // ExplicitRK, FinishRHS and the explicit Crank-Nicolson half
             // (IMEXRK.cpp:75-134)
             V R[M], um[M], up[M];
-            nb_prev<T, M>(x, um, lane);
-            nb_next<T, M>(x, up, lane);
+            nb_prev(x, um, lane);
+            nb_next(x, up, lane);
 #pragma unroll
             for (int t = 0; t < M; ++t) {
                 const V d2 = dzz_row(dzz[0][t], um[t], dzz[1][t], x[t], dzz[2][t], up[t]);
@@ -184,9 +183,9 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
             if (wave == CW_U1 && A.ubar != nullptr && zero_mode) {  // EvolveBackground, as in k_modal
                 V ub[M];
 #pragma unroll
-                for (int t = 0; t < M; ++t) ub[t] = mkc<T>(coefz(ZC_UBAR, t), T(0));
-                nb_prev<T, M>(ub, um, lane);
-                nb_next<T, M>(ub, up, lane);
+                for (int t = 0; t < M; ++t) ub[t] = mkc<T>(row[t] < N ? A.ubar[row[t]] : T(0), T(0));
+                nb_prev(ub, um, lane);
+                nb_next(ub, up, lane);
 #pragma unroll
                 for (int t = 0; t < M; ++t) {
                     const int j = row[t];
@@ -211,7 +210,7 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
         get(CW_U1, u1);
         get(CW_U3, u3);
         if (three) get(CW_U2, u2);
-        nb_next<T, M>(u3, u3p, lane);
+        nb_next(u3, u3p, lane);
 #pragma unroll
         for (int t = 0; t < M; ++t) dv[t] = div_row(kx, u1[t], three, ky, u2[t], z0[t], u3[t], u3p[t]);
         zero_ends(dv, false);
@@ -233,7 +232,7 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
 #pragma unroll
             for (int t = 0; t < M; ++t) dd[t] = mkc<double>(double(dv[t].x), double(dv[t].y));
             tri_apply<double, M>(D, dd, lane);
-            nb_prev<double, M>(dd, qm, lane);
+            nb_prev(dd, qm, lane);
 #pragma unroll
             for (int t = 0; t < M; ++t) {
                 const double dzq = double(z2[t]) * (dd[t].x - qm[t].x);
@@ -261,7 +260,7 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
             get(CW_P, q);
             if (wave == CW_U3) {
                 V qm[M];
-                nb_prev<T, M>(q, qm, lane);
+                nb_prev(q, qm, lane);
 #pragma unroll
                 for (int t = 0; t < M; ++t) x[t] = tmadc(-z2[t], csub(q[t], qm[t]), x[t]);
             } else {

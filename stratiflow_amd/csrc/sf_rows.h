@@ -6,24 +6,19 @@
 
 namespace sf {
 
-template <typename T, int M>
-__device__ __forceinline__ void nb_prev(const cx<T> (&x)[M], cx<T> (&xm)[M], int lane) {
-    using V = cx<T>;
-    V s;
-    s.x = __shfl(x[M - 1].x, (lane - 1) & 63, 64);
-    s.y = __shfl(x[M - 1].y, (lane - 1) & 63, 64);
-    if (lane == 0) s = czero<V>();
+// the rows before and after each row of the lane (V complex or one part)
+template <int M, typename V>
+__device__ __forceinline__ void nb_prev(const V (&x)[M], V (&xm)[M], int lane) {
+    V s = shfl_idx(x[M - 1], (lane - 1) & 63);
+    if (lane == 0) set_zero(s);
     xm[0] = s;
 #pragma unroll
     for (int t = 1; t < M; ++t) xm[t] = x[t - 1];
 }
-template <typename T, int M>
-__device__ __forceinline__ void nb_next(const cx<T> (&x)[M], cx<T> (&xp)[M], int lane) {
-    using V = cx<T>;
-    V s;
-    s.x = __shfl(x[0].x, (lane + 1) & 63, 64);
-    s.y = __shfl(x[0].y, (lane + 1) & 63, 64);
-    if (lane == 63) s = czero<V>();
+template <int M, typename V>
+__device__ __forceinline__ void nb_next(const V (&x)[M], V (&xp)[M], int lane) {
+    V s = shfl_idx(x[0], (lane + 1) & 63);
+    if (lane == 63) set_zero(s);
 #pragma unroll
     for (int t = 0; t < M - 1; ++t) xp[t] = x[t + 1];
     xp[M - 1] = s;

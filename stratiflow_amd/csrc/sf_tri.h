@@ -44,8 +44,28 @@ __device__ __forceinline__ cx<T> tmadc(T a, cx<T> v, cx<T> c) {  // a*v + c
 }
 
 template <typename T>
-__device__ __forceinline__ T shfl_idx(T v, int src) {
-    return __shfl(v, src, 64);
+__device__ __forceinline__ T tscale(T a, T v) {
+    return tmul(a, v);
+}
+template <typename T>
+__device__ __forceinline__ T tmadc(T a, T v, T c) {
+    return tmad(a, v, c);
+}
+
+__device__ __forceinline__ float shfl_idx(float v, int src) { return __shfl(v, src, 64); }
+__device__ __forceinline__ double shfl_idx(double v, int src) { return __shfl(v, src, 64); }
+template <typename V>
+__device__ __forceinline__ V shfl_idx(V v, int src) {
+    V r;
+    r.x = __shfl(v.x, src, 64);
+    r.y = __shfl(v.y, src, 64);
+    return r;
+}
+__device__ __forceinline__ void set_zero(float& v) { v = 0; }
+__device__ __forceinline__ void set_zero(double& v) { v = 0; }
+template <typename V>
+__device__ __forceinline__ void set_zero(V& v) {
+    v = czero<V>();
 }
 
 template <typename T, int M>
@@ -145,12 +165,11 @@ __device__ __forceinline__ void tri_factor(TriFactor<T, M>& F, const T (&a)[M], 
 }
 
 // Solve in place: d holds the lane's M right-hand-side rows on entry and the
-// solution on exit.
-template <typename T, int M>
-__device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, cx<T> (&d)[M], int lane) {
-    using V = cx<T>;
-    V Ds;
-    V g[M];
+// solution on exit.  D is complex, or T for one part of it.
+template <typename T, int M, typename D>
+__device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, D (&d)[M], int lane) {
+    D Ds;
+    D g[M];
     if constexpr (M == 1) {
         Ds = d[0];
     } else {
@@ -160,32 +179,24 @@ __device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, cx<T> (&d)[M
         for (int t = 1; t <= M - 2; ++t) g[t] = tscale(F.rden[t], tmadc(-F.a[t], g[t - 1], d[t]));
 #pragma unroll
         for (int t = M - 3; t >= 0; --t) g[t] = tmadc(-F.cc[t], g[t + 1], g[t]);
-        V gn0;
-        gn0.x = shfl_idx(g[0].x, (lane + 1) & 63);
-        gn0.y = shfl_idx(g[0].y, (lane + 1) & 63);
-        if (lane == 63) gn0 = czero<V>();
+        D gn0 = shfl_idx(g[0], (lane + 1) & 63);
+        if (lane == 63) set_zero(gn0);
         Ds = tmadc(-F.cI, gn0, tmadc(-F.aI, g[M - 2], d[M - 1]));
     }
 #pragma unroll
     for (int lev = 0; lev < 6; ++lev) {
         const int s = 1 << lev;
-        V Dm, Dp;
-        Dm.x = shfl_idx(Ds.x, (lane - s) & 63);
-        Dm.y = shfl_idx(Ds.y, (lane - s) & 63);
-        Dp.x = shfl_idx(Ds.x, (lane + s) & 63);
-        Dp.y = shfl_idx(Ds.y, (lane + s) & 63);
-        if (lane - s < 0) Dm = czero<V>();
-        if (lane + s > 63) Dp = czero<V>();
+        D Dm = shfl_idx(Ds, (lane - s) & 63), Dp = shfl_idx(Ds, (lane + s) & 63);
+        if (lane - s < 0) set_zero(Dm);
+        if (lane + s > 63) set_zero(Dp);
         Ds = tmadc(F.gamma[lev], Dp, tmadc(F.alpha[lev], Dm, Ds));
     }
-    const V sl = tscale(F.rB, Ds);
+    const D sl = tscale(F.rB, Ds);
     if constexpr (M == 1) {
         d[0] = sl;
     } else {
-        V sm;
-        sm.x = shfl_idx(sl.x, (lane - 1) & 63);
-        sm.y = shfl_idx(sl.y, (lane - 1) & 63);
-        if (lane == 0) sm = czero<V>();
+        D sm = shfl_idx(sl, (lane - 1) & 63);
+        if (lane == 0) set_zero(sm);
 #pragma unroll
         for (int t = 0; t <= M - 2; ++t) d[t] = tmadc(-F.w[t], sl, tmadc(-F.v[t], sm, g[t]));
         d[M - 1] = sl;
