@@ -102,7 +102,7 @@ struct Ctx {
     double* scal_host = nullptr;
     unsigned* ticket = nullptr;       // of the inner products' blocks
     DotResult* dot_host = nullptr;    // pinned: what the inner products leave for the host
-    unsigned long long dot_seq = 0;   // number of the last inner-product launch
+    unsigned dot_call = 0;            // number of the last inner-product launch
     std::vector<double> zc_host;  // double copy of the coefficient table
 
     sf_field state[17];
@@ -956,15 +956,36 @@ struct Ctx {
         d.partial = partial;
         d.ticket = ticket;
         d.host = dot_host;
-        d.seq = ++dot_seq;
+        d.call = ++dot_call;
+        const int sums = dot_sums(nmodal);
         check(launch_dot<T>(d, pairs, stream), "dot");
-        auto arrived = [&]() { return __atomic_load_n(&dot_host->seq, __ATOMIC_ACQUIRE) == d.seq; };
-        for (int i = 0; i < 4000 && !arrived(); ++i) __builtin_ia32_pause();
-        if (!arrived()) {
+        auto word = [&](int i, int k, int h) {
+            return __atomic_load_n(&dot_host->sum[i][k].half[h], __ATOMIC_ACQUIRE);
+        };
+        auto arrived = [&]() {
+            for (int i = 0; i < pairs; ++i)
+                for (int k = 0; k < sums; ++k)
+                    if (unsigned(word(i, k, 0)) != d.call || unsigned(word(i, k, 1)) != d.call) return false;
+            return true;
+        };
+        bool done = arrived();
+        for (int i = 0; i < 4000 && !done; ++i) {
+            __builtin_ia32_pause();
+            done = arrived();
+        }
+        if (!done) {
             SF_HIP(hipStreamSynchronize(stream));
             SF_REQUIRE(arrived(), SF_ERR_STATE, "inner product: no result after its launch");
         }
-        for (int i = 0; i < pairs; ++i) out[i] = dot_host->val[i];
+        for (int i = 0; i < pairs; ++i) {
+            out[i] = 0;
+            for (int k = 0; k < sums; ++k) {
+                const unsigned long long b = (word(i, k, 0) >> 32) | (word(i, k, 1) >> 32 << 32);
+                double v;
+                std::memcpy(&v, &b, sizeof(v));
+                out[i] += v;
+            }
+        }
     }
     void read_scalars(int n, double* out) {
         SF_HIP(hipMemcpyAsync(scal_host, scal, n * sizeof(double), hipMemcpyDeviceToHost, stream));

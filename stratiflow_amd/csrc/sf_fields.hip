@@ -21,13 +21,19 @@ __device__ __forceinline__ double wave_sum(double v) {
 //
 // A 2D field is 0.2-0.7 MB, so latency and launches bound this, not HBM: the
 // separate finishing kernel, the copy of the result to the host and the wait
-// on the stream cost more than the sums.  Every block stores its partial sum
-// and draws a ticket; the block with the last ticket adds the partials in
-// block order (the same bits on every call) and writes the results and then
-// the call's sequence number to pinned host memory, which the host reads.
-// Partials and ticket go through agent-scope accesses, since the blocks run
-// on XCDs with separate L2s.
+// on the stream cost more than the sums.  Results go straight to pinned host
+// memory, which the host watches.  Up to DOT_HOST blocks each write their own sum
+// and the host adds them; beyond that every block draws a ticket and the one with
+// the last adds the partials (through agent-scope accesses: the blocks' XCDs have
+// separate L2s), which costs 2 us more.  Either way the sums are added in block
+// order: the same bits on every call.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void dot_send(DotWord* to, double v, unsigned call) {
+    const unsigned long long b = __double_as_longlong(v);
+    __hip_atomic_store(&to->half[0], (b << 32) | call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&to->half[1], (b >> 32 << 32) | call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <typename T>
 __global__ __launch_bounds__(FB) void k_dot(DotArgs<T> A) {
     __shared__ double red[FB / 64];
@@ -46,18 +52,23 @@ __global__ __launch_bounds__(FB) void k_dot(DotArgs<T> A) {
         const double re = double(x.x) * double(v.x) + double(x.y) * double(v.y);
         return (m00 ? 1.0 : 2.0) * double(w[z]) * re;
     };
-    unsigned e = blockIdx.x * FB + threadIdx.x;
-    for (; e < n && n - e > 3 * stride; e += 4 * stride) {  // four elements in flight
+    // four elements in flight; past the end the first one with a zero factor, so
+    // that the last round is no chain of single loads
+    for (unsigned e = blockIdx.x * FB + threadIdx.x; e < n; e += 4 * stride) {
         cx<T> x[4], v[4];
+        unsigned at[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            x[i] = a[e + i * stride];
-            v[i] = b[e + i * stride];
+            at[i] = n - e > i * stride ? e + i * stride : e;
+            x[i] = a[at[i]];
+            v[i] = b[at[i]];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc += term(e + i * stride, x[i], v[i]);
+        for (int i = 0; i < 4; ++i) {
+            const double t = term(at[i], x[i], v[i]);
+            acc += i == 0 || at[i] != e ? t : 0.0;
+        }
     }
-    for (; e < n; e += stride) acc += term(e, a[e], b[e]);
     acc = wave_sum(acc);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) red[wave] = acc;
@@ -66,9 +77,14 @@ __global__ __launch_bounds__(FB) void k_dot(DotArgs<T> A) {
         double s = 0;
 #pragma unroll
         for (int i = 0; i < FB / 64; ++i) s += red[i];
-        __hip_atomic_store(A.partial + y * gridDim.x + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned t = __hip_atomic_fetch_add(A.ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        last = t + 1 == gridDim.x * gridDim.y;
+        if (gridDim.x <= DOT_HOST) {
+            dot_send(&A.host->sum[y][blockIdx.x], s, A.call);
+            last = false;
+        } else {
+            __hip_atomic_store(A.partial + y * gridDim.x + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned t = __hip_atomic_fetch_add(A.ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            last = t + 1 == gridDim.x * gridDim.y;
+        }
     }
     __syncthreads();
     if (!last) return;  // block-uniform
@@ -78,26 +94,30 @@ __global__ __launch_bounds__(FB) void k_dot(DotArgs<T> A) {
         for (unsigned i = lane; i < gridDim.x; i += 64)
             s += __hip_atomic_load(A.partial + wave * gridDim.x + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s = wave_sum(s);
-        if (lane == 0) __hip_atomic_store(&A.host->val[wave], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (lane == 0) dot_send(&A.host->sum[wave][0], s, A.call);
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0)
         __hip_atomic_store(A.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-        __hip_atomic_store(&A.host->seq, A.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
 }
 
-// Blocks per pair: four elements a thread, so that the 2D fields (some
-// thousand modes and levels) take a few dozen blocks and the last one has few
-// partials to add, up to DOT_BLOCKS where HBM bandwidth sets the time.
+// Blocks per pair: four elements a thread, up to DOT_BLOCKS where HBM bandwidth
+// sets the time; fields of up to 16 elements a thread of DOT_HOST blocks take those.
+static unsigned dot_blocks(size_t n) {
+    const size_t four = (n + 4 * FB - 1) / (4 * FB);
+    if (four <= DOT_HOST) return four < 1 ? 1 : unsigned(four);
+    if (n <= size_t(DOT_HOST) * FB * 16) return DOT_HOST;
+    return unsigned(four < size_t(DOT_BLOCKS) ? four : size_t(DOT_BLOCKS));
+}
+int dot_sums(size_t n) {
+    const unsigned b = dot_blocks(n);
+    return b <= DOT_HOST ? int(b) : 1;
+}
+
 template <typename T>
 hipError_t launch_dot(const DotArgs<T>& a, int pairs, hipStream_t s) {
     static_assert(DOT_MAX <= FB / 64, "the last block adds one pair per wave");
     if (pairs < 1 || pairs > DOT_MAX) return hipErrorInvalidValue;
-    unsigned blocks = unsigned((a.n + 4 * FB - 1) / (4 * FB));
-    if (blocks > unsigned(DOT_BLOCKS)) blocks = DOT_BLOCKS;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL((k_dot<T>), dim3(blocks, pairs), dim3(FB), 0, s, a);
+    hipLaunchKernelGGL((k_dot<T>), dim3(dot_blocks(a.n), pairs), dim3(FB), 0, s, a);
     return hipGetLastError();
 }
 

@@ -151,14 +151,21 @@ template <typename T>
 hipError_t launch_x_r2c(const XTArgs<T>& a, int N1, int N2, hipStream_t s);
 template <typename T>
 hipError_t launch_x_sum(const XSumArgs<T>& a, int N1, int N2, hipStream_t s);
-// FP64 inner products (sf_fields.hip): one launch for up to DOT_MAX pairs,
-// results and then the sequence number of the call in pinned host memory
+// FP64 inner products (sf_fields.hip): one launch for up to DOT_MAX pairs, the
+// results in pinned host memory
 constexpr int DOT_MAX = 4;
 constexpr int DOT_BLOCKS = 1024;  // blocks (partial sums) per pair
-struct DotResult {
-    double val[DOT_MAX];
-    unsigned long long seq;
+constexpr int DOT_HOST = 32;      // up to here the host adds the blocks' sums
+// A double as two words that each carry the number of the call it belongs to,
+// so that the host can tell when both halves have arrived.
+struct DotWord {
+    unsigned long long half[2];  // bits 32..63: a half of the double, 0..31: the call
 };
+struct DotResult {
+    DotWord sum[DOT_MAX][DOT_HOST];
+};
+// sums the host finds for each pair: the blocks' own, or their total
+int dot_sums(size_t n);
 template <typename T>
 struct DotArgs {
     const cx<T>* a[DOT_MAX];
@@ -168,7 +175,7 @@ struct DotArgs {
     double* partial;      // DOT_MAX * DOT_BLOCKS values
     unsigned* ticket;     // zero between launches
     DotResult* host;
-    unsigned long long seq;
+    unsigned call;        // number of the call
 };
 template <typename T>
 hipError_t launch_dot(const DotArgs<T>& a, int pairs, hipStream_t s);
