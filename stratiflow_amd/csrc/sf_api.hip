@@ -1,4 +1,5 @@
 // sf_api.hip -- context, fields and the extern "C" boundary (include/sfhip.h).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -939,7 +940,7 @@ struct Ctx {
         const V *a, *b;
         int bc;
     };
-    // The result arrives in pinned memory with its sequence number, which the
+    // The sums arrive in pinned memory with the number of the call, which the
     // host watches for about the time of a short queue (a dozen 2D launches)
     // before it waits for the stream: waiting takes a barrier packet and a
     // signal (13 us more per inner product of a 256x1x256 field).
@@ -1138,14 +1139,14 @@ template <typename T>
 struct Batch {
     using V = cx<T>;
     struct Group {
-        int key = 0;  // N1 (x-pass), rows per lane M (grouped modal), modes per block (mixed modal)
+        int key = 0;  // N1 (x-pass), rows per lane M (grouped modal), modes per block
         std::vector<int> members;
         int total = 0;
         int grid = 1;
         int zch = 2;
         int span = 1;  // mixed launches: the largest N1 (x-pass) or rows per lane (modal) of the members
         void* args = nullptr;
-        int* start = nullptr;
+        int2* items = nullptr;
     };
     std::vector<Ctx<T>*> runs;
     hipStream_t stream = nullptr;
@@ -1179,9 +1180,9 @@ struct Batch {
     }
     static void free_group(Group& g) {
         if (g.args) (void)hipFree(g.args);
-        if (g.start) (void)hipFree(g.start);
+        if (g.items) (void)hipFree(g.items);
         g.args = nullptr;
-        g.start = nullptr;
+        g.items = nullptr;
     }
     void release_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
@@ -1227,7 +1228,10 @@ struct Batch {
                 g.members = kv.second;
                 mg[k].push_back(g);
             }
+            // the longest columns first: their blocks are the last to finish
             mmix[k].members = all;
+            std::stable_sort(mmix[k].members.begin(), mmix[k].members.end(),
+                             [&](int a, int b) { return runs[a]->N3 > runs[b]->N3; });
             mmix[k].key = 4;
             mmix[k].span = mmax;
         }
@@ -1240,33 +1244,46 @@ struct Batch {
         for (auto* c : runs) SF_HIP(hipStreamSynchronize(c->stream));
     }
 
+    // Arguments of the members and the table of their work items, count[m] of each.
+    // Blocks go to the eight XCDs in turn: of every 64 items each XCD takes eight
+    // consecutive ones, which are of one run as a rule and share its coefficients
+    // and the cache lines that two neighbouring tiles of modes have in common.  Per
+    // stage of 16 runs of 64..256 x 100..384 FP32 the modal launch (4 modes) takes
+    // 32 us with 1 item in turn, 27 with 4, 24 with 8, 25 with 12, and that of 64
+    // runs (8 modes) 59, 54, 55, 54; whole runs on an XCD are as good for 16
+    // runs and 10 us worse for 64, by their unequal lengths.  The x-pass is within 3%.
     template <typename A>
-    void upload_group(Group& g, const std::vector<A>& a, const std::vector<int>& st) {
+    void upload_group(Group& g, const std::vector<A>& a, const std::vector<int>& count, int grid) {
+        g.total = 0;
+        for (int n : count) g.total += n;
+        std::vector<int2> items(g.total);
+        int n = 0;
+        for (int m = 0; m < int(count.size()); ++m)
+            for (int i = 0; i < count[m]; ++i, ++n) {
+                const bool window = n / 64 < g.total / 64;  // else the last items, in order
+                items[window ? n / 64 * 64 + n % 8 * 8 + n / 8 % 8 : n] = make_int2(m, i);
+            }
+        g.grid = std::max(1, std::min(g.total, grid));
         free_group(g);
         SF_HIP(hipMalloc(&g.args, a.size() * sizeof(A)));
-        SF_HIP(hipMalloc(reinterpret_cast<void**>(&g.start), st.size() * sizeof(int)));
+        SF_HIP(hipMalloc(reinterpret_cast<void**>(&g.items), items.size() * sizeof(int2)));
         SF_HIP(hipMemcpy(g.args, a.data(), a.size() * sizeof(A), hipMemcpyHostToDevice));
-        SF_HIP(hipMemcpy(g.start, st.data(), st.size() * sizeof(int), hipMemcpyHostToDevice));
+        SF_HIP(hipMemcpy(g.items, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
     }
 
     // r1f: first radix of the FFT plans (mixed launches; 0 = default)
     void build_xgroup(Group& g, int zch, int grid, int r1f = 0) {
         std::vector<XArgs<T>> a;
-        std::vector<int> st;
-        int total = 0;
+        std::vector<int> count;
         for (int r : g.members) {
             XArgs<T> x = runs[r]->xargs_2d(false, true);
             x.zch = zch;
             x.tw = runs[r]->x_twiddles(r1f);
             a.push_back(x);
-            st.push_back(total);
-            total += (runs[r]->N3 + zch - 1) / zch;
+            count.push_back((runs[r]->N3 + zch - 1) / zch);
         }
-        st.push_back(total);
         g.zch = zch;
-        g.total = total;
-        g.grid = std::max(1, std::min(total, grid));
-        upload_group(g, a, st);
+        upload_group(g, a, count, grid);
     }
 
     // modal group: arguments of run r from args(r), mb modes per block for
@@ -1274,19 +1291,14 @@ struct Batch {
     template <typename Fn>
     void build_mgroup(Group& g, bool mixed, Fn args) {
         std::vector<ModalArgs<T>> a;
-        std::vector<int> st;
-        int total = 0;
+        std::vector<int> count;
         for (int r : g.members) {
             Ctx<T>* c = runs[r];
             a.push_back(args(r));
-            st.push_back(total);
             const int mb = mixed ? g.key : modal_modes_per_block(g.key, int(sizeof(T)));
-            total += ((c->A1 + mb - 1) / mb) * c->A2;
+            count.push_back(((c->A1 + mb - 1) / mb) * c->A2);
         }
-        st.push_back(total);
-        g.total = total;
-        g.grid = std::max(1, std::min(total, 8 * ncu));
-        upload_group(g, a, st);
+        upload_group(g, a, count, 8 * ncu);
     }
 
     // the explicit terms ping-pong as in Ctx::stage: stage 0 writes
@@ -1323,30 +1335,29 @@ struct Batch {
 
     void launch_x(bool mixed) {
         if (mixed) {
-            const hipError_t e = launch_xpass_mixed<T>(static_cast<const XArgs<T>*>(xmix.args), xmix.start,
-                                                       int(xmix.members.size()), xmix.total, xmix.span, xr1f(),
-                                                       xmix.grid, stream);
+            const hipError_t e = launch_xpass_mixed<T>(static_cast<const XArgs<T>*>(xmix.args), xmix.items, xmix.total,
+                                                       xmix.span, xr1f(), xmix.grid, stream);
             if (e != hipSuccess) throw Error(SF_ERR_HIP, std::string("batched xpass: ") + hipGetErrorString(e));
             return;
         }
         for (auto& g : xg) {
-            const hipError_t e = launch_xpass_batch<T>(static_cast<const XArgs<T>*>(g.args), g.start,
-                                                       int(g.members.size()), g.total, g.key, g.grid, stream);
+            const hipError_t e = launch_xpass_batch<T>(static_cast<const XArgs<T>*>(g.args), g.items, g.total, g.key,
+                                                       g.grid, stream);
             if (e != hipSuccess) throw Error(SF_ERR_HIP, std::string("batched xpass: ") + hipGetErrorString(e));
         }
     }
 
     void launch_m(int plan, std::vector<Group>& groups, Group& mix) {
         if (plan != SF_BATCH_GROUPED) {
+            const ModalArgs<T>* args = static_cast<const ModalArgs<T>*>(mix.args);
             const hipError_t e =
-                launch_modal_mixed<T>(static_cast<const ModalArgs<T>*>(mix.args), mix.start, int(mix.members.size()),
-                                      mix.total, mix.key, mix.span, mix.grid, stream);
+                launch_modal_mixed<T>(args, mix.items, mix.total, mix.key, mix.span, mix.grid, stream);
             if (e != hipSuccess) throw Error(SF_ERR_HIP, std::string("batched modal: ") + hipGetErrorString(e));
             return;
         }
         for (auto& g : groups) {
-            const hipError_t e = launch_modal_batch<T>(static_cast<const ModalArgs<T>*>(g.args), g.start,
-                                                       int(g.members.size()), g.total, g.key, g.grid, stream);
+            const hipError_t e = launch_modal_batch<T>(static_cast<const ModalArgs<T>*>(g.args), g.items, g.total, g.key,
+                                                       g.grid, stream);
             if (e != hipSuccess) throw Error(SF_ERR_HIP, std::string("batched modal: ") + hipGetErrorString(e));
         }
     }
@@ -1383,11 +1394,11 @@ struct Batch {
                     const double ms = time_ms([&]() {
                         hipError_t e;
                         if (mixed)
-                            e = launch_xpass_mixed<T>(static_cast<const XArgs<T>*>(g.args), g.start,
-                                                      int(g.members.size()), g.total, g.span, r1f, g.grid, stream);
+                            e = launch_xpass_mixed<T>(static_cast<const XArgs<T>*>(g.args), g.items, g.total, g.span,
+                                                      r1f, g.grid, stream);
                         else
-                            e = launch_xpass_batch<T>(static_cast<const XArgs<T>*>(g.args), g.start,
-                                                      int(g.members.size()), g.total, g.key, g.grid, stream);
+                            e = launch_xpass_batch<T>(static_cast<const XArgs<T>*>(g.args), g.items, g.total, g.key,
+                                                      g.grid, stream);
                         if (e != hipSuccess) throw Error(SF_ERR_HIP, "batched xpass (tuning)");
                     });
                     if (ms < best) {
@@ -1445,14 +1456,14 @@ struct Batch {
             std::vector<Group> tg = mg[0];
             for (auto& g : tg) {
                 g.args = nullptr;
-                g.start = nullptr;
+                g.items = nullptr;
                 build_mgroup(g, false, sargs);
             }
             tuned_ms[3] = time_ms([&]() { launch_m(SF_BATCH_GROUPED, tg, mmix[0]); });
             for (auto& g : tg) free_group(g);
             Group tm = mmix[0];
             tm.args = nullptr;
-            tm.start = nullptr;
+            tm.items = nullptr;
             for (int q = 0; q < 2; ++q) {
                 tm.key = q ? 8 : 4;
                 build_mgroup(tm, true, sargs);

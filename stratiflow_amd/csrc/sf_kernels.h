@@ -120,26 +120,27 @@ template <typename T>
 hipError_t launch_xpass(const XArgs<T>& a, int N1, int N2, bool threeD, hipStream_t s);
 template <typename T>
 hipError_t launch_xbase(const XBaseArgs<T>& a, int N1, int N2, bool threeD, hipStream_t s);
-// many independent 2D runs per launch: args/start live in device memory,
-// start[r] = first work item of run r (x-pass: z-blocks; modal: tiles of
-// modes), total = start[nruns]; grid-stride loop over `grid` blocks.  The
+// many independent 2D runs per launch: args and items live in device memory,
+// items[i] = (run, work item of the run: x-pass z-block, modal tile of modes);
+// grid-stride loop over `grid` blocks.  (A table of the items, since a search in
+// the runs' first items is a chain of dependent loads before a block can start.)  The
 // _batch launches take runs of one N1 (x-pass) or one rows-per-lane M
 // (modal); the _mixed launches take runs of any N1 / N3, the modal one with
 // mb (4 or 8) modes per block for every run.
 template <typename T>
-hipError_t launch_modal_batch(const ModalArgs<T>* args, const int* start, int nruns, int total, int M, int grid,
+hipError_t launch_modal_batch(const ModalArgs<T>* args, const int2* items, int total, int M, int grid,
                               hipStream_t s);
 template <typename T>
-hipError_t launch_xpass_batch(const XArgs<T>* args, const int* start, int nruns, int total, int N1, int grid,
+hipError_t launch_xpass_batch(const XArgs<T>* args, const int2* items, int total, int N1, int grid,
                               hipStream_t s);
 // (mmax: the largest rows per lane of the runs; nmax: the largest N1)
 template <typename T>
-hipError_t launch_modal_mixed(const ModalArgs<T>* args, const int* start, int nruns, int total, int mb, int mmax,
+hipError_t launch_modal_mixed(const ModalArgs<T>* args, const int2* items, int total, int mb, int mmax,
                               int grid, hipStream_t s);
 // (r1f: first radix of the FFT plans, 0 for the defaults or 8; each run's tw
 // must be the table of its N1 under that plan, fft_twiddles_plan)
 template <typename T>
-hipError_t launch_xpass_mixed(const XArgs<T>* args, const int* start, int nruns, int total, int nmax, int r1f,
+hipError_t launch_xpass_mixed(const XArgs<T>* args, const int2* items, int total, int nmax, int r1f,
                               int grid, hipStream_t s);
 template <typename T>
 hipError_t launch_yinv(const YArgs<T>& a, int N2, hipStream_t s);

@@ -361,32 +361,19 @@ __global__ __launch_bounds__(MB * 64) void k_modal(ModalArgs<T> A) {
     modal_body<T, M, MB, FULL>(A, t / nt, (t % nt) * MB, tile);
 }
 
-// index r of the run owning work item `item`: start[r] <= item < start[r+1]
-__device__ __forceinline__ int find_run(const int* __restrict__ start, int nruns, int item) {
-    int lo = 0, hi = nruns - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (start[mid] <= item) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // Many independent runs in one launch: a grid-stride (persistent) loop over
 // the work items of all runs, one item = one block's tile of modes.  Every
 // run has the same rows-per-lane M; each reads its own arguments.
 template <typename T, int M>
 __global__ __launch_bounds__((modal_mb<T, M>() * 64)) void k_modal_batch(const ModalArgs<T>* __restrict__ args,
-                                                                      const int* __restrict__ start, int nruns,
-                                                                      int total) {
+                                                                      const int2* __restrict__ items, int total) {
     constexpr int MB = modal_mb<T, M>();
     __shared__ cx<T> tile[64 * M * (MB + 1)];
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
-        const int r = find_run(start, nruns, item);
-        const ModalArgs<T>& a = args[r];
+        const int2 it = items[item];  // run, item of the run
+        const ModalArgs<T>& a = args[it.x];
         const int nt = (a.A1 + MB - 1) / MB;
-        const int local = item - start[r];
-        modal_body<T, M, MB>(a, local / nt, (local % nt) * MB, tile);
+        modal_body<T, M, MB>(a, it.y / nt, (it.y % nt) * MB, tile);
     }
 }
 
@@ -396,14 +383,13 @@ __global__ __launch_bounds__((modal_mb<T, M>() * 64)) void k_modal_batch(const M
 // demanding case compiled in.
 template <typename T, int MB, int MMAX>
 __global__ __launch_bounds__(MB * 64) void k_modal_mixed(const ModalArgs<T>* __restrict__ args,
-                                                        const int* __restrict__ start, int nruns, int total) {
+                                                        const int2* __restrict__ items, int total) {
     __shared__ cx<T> tile[64 * MMAX * (MB + 1)];
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
-        const int r = find_run(start, nruns, item);
-        const ModalArgs<T>& a = args[r];
+        const int2 it = items[item];  // run, item of the run
+        const ModalArgs<T>& a = args[it.x];
         const int nt = (a.A1 + MB - 1) / MB;
-        const int local = item - start[r];
-        const int ja = local / nt, j10 = (local % nt) * MB;
+        const int ja = it.y / nt, j10 = (it.y % nt) * MB;
         switch ((a.N3 + 63) / 64) {
 #define SF_M(m)                                                       \
     case m:                                                           \
@@ -419,23 +405,23 @@ __global__ __launch_bounds__(MB * 64) void k_modal_mixed(const ModalArgs<T>* __r
 
 // the variant compiled for rows per lane up to 3, 6 or 8 that covers mmax
 template <typename T, int MB>
-static void launch_modal_mixed_mb(const ModalArgs<T>* args, const int* start, int nruns, int total, int mmax, int grid,
+static void launch_modal_mixed_mb(const ModalArgs<T>* args, const int2* items, int total, int mmax, int grid,
                                   hipStream_t s) {
     if (mmax <= 3)
-        hipLaunchKernelGGL((k_modal_mixed<T, MB, 3>), dim3(grid), dim3(MB * 64), 0, s, args, start, nruns, total);
+        hipLaunchKernelGGL((k_modal_mixed<T, MB, 3>), dim3(grid), dim3(MB * 64), 0, s, args, items, total);
     else if (mmax <= 6)
-        hipLaunchKernelGGL((k_modal_mixed<T, MB, 6>), dim3(grid), dim3(MB * 64), 0, s, args, start, nruns, total);
+        hipLaunchKernelGGL((k_modal_mixed<T, MB, 6>), dim3(grid), dim3(MB * 64), 0, s, args, items, total);
     else
-        hipLaunchKernelGGL((k_modal_mixed<T, MB, 8>), dim3(grid), dim3(MB * 64), 0, s, args, start, nruns, total);
+        hipLaunchKernelGGL((k_modal_mixed<T, MB, 8>), dim3(grid), dim3(MB * 64), 0, s, args, items, total);
 }
 
 template <typename T>
-hipError_t launch_modal_mixed(const ModalArgs<T>* args, const int* start, int nruns, int total, int mb, int mmax,
+hipError_t launch_modal_mixed(const ModalArgs<T>* args, const int2* items, int total, int mb, int mmax,
                               int grid, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     if (mmax < 1 || mmax > MODAL_MAX_M) return hipErrorInvalidValue;
-    if (mb == 4) launch_modal_mixed_mb<T, 4>(args, start, nruns, total, mmax, grid, s);
-    else if (mb == 8) launch_modal_mixed_mb<T, 8>(args, start, nruns, total, mmax, grid, s);
+    if (mb == 4) launch_modal_mixed_mb<T, 4>(args, items, total, mmax, grid, s);
+    else if (mb == 8) launch_modal_mixed_mb<T, 8>(args, items, total, mmax, grid, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -455,14 +441,14 @@ int modal_modes_per_block(int M, int precision) {
 #endif
 
 template <typename T>
-hipError_t launch_modal_batch(const ModalArgs<T>* args, const int* start, int nruns, int total, int M, int grid,
+hipError_t launch_modal_batch(const ModalArgs<T>* args, const int2* items, int total, int M, int grid,
                               hipStream_t s) {
     if (total <= 0) return hipSuccess;
     switch (M) {
 #define SF_M(m)                                                                                               \
     case m:                                                                                                   \
-        hipLaunchKernelGGL((k_modal_batch<T, m>), dim3(grid), dim3(modal_mb<T, m>() * 64), 0, s, args, start, \
-                           nruns, total);                                                                     \
+        hipLaunchKernelGGL((k_modal_batch<T, m>), dim3(grid), dim3(modal_mb<T, m>() * 64), 0, s, args, items, \
+                           total);                                                                            \
         break;
         SF_M(1) SF_M(2) SF_M(3) SF_M(4) SF_M(5) SF_M(6) SF_M(7) SF_M(8)
 #undef SF_M
@@ -898,13 +884,13 @@ hipError_t launch_xbase(const XBaseArgs<T>& a, int N1, int N2, bool threeD, hipS
 // 2D runs with the same N1 in one launch (grid-stride over the z-blocks of
 // all runs; see k_modal_batch)
 template <typename T, int N1>
-__global__ __launch_bounds__(BS) void k_xpass_batch(const XArgs<T>* __restrict__ args, const int* __restrict__ start,
-                                                    int nruns, int total) {
+__global__ __launch_bounds__(BS) void k_xpass_batch(const XArgs<T>* __restrict__ args, const int2* __restrict__ items,
+                                                    int total) {
     static_assert(xpass_bs<T, false, false>() == BS, "the batched 2D x-pass runs blocks of BS threads");
     __shared__ cx<T> lds[xpass_lds<N1, false>()];
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
-        const int r = find_run(start, nruns, item);
-        xpass_body<T, N1, false, false>(args[r], item - start[r], 0, lds);
+        const int2 it = items[item];  // run, item of the run
+        xpass_body<T, N1, false, false>(args[it.x], it.y, 0, lds);
     }
 }
 
@@ -923,16 +909,16 @@ constexpr int xpass_mixed_lds() {
 }
 
 template <typename T, int NMAX, int R1F>
-__global__ __launch_bounds__(BS) void k_xpass_mixed(const XArgs<T>* __restrict__ args, const int* __restrict__ start,
-                                                    int nruns, int total) {
+__global__ __launch_bounds__(BS) void k_xpass_mixed(const XArgs<T>* __restrict__ args, const int2* __restrict__ items,
+                                                    int total) {
     __shared__ cx<T> lds[xpass_mixed_lds<NMAX, R1F>()];
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
-        const int r = find_run(start, nruns, item);
-        const XArgs<T>& a = args[r];
+        const int2 it = items[item];  // run, item of the run
+        const XArgs<T>& a = args[it.x];
         switch (a.N1) {
 #define SF_CASE(n)                                                                              \
     case n:                                                                                     \
-        if constexpr (n <= NMAX) xpass_body<T, n, false, false, R1F>(a, item - start[r], 0, lds); \
+        if constexpr (n <= NMAX) xpass_body<T, n, false, false, R1F>(a, it.y, 0, lds); \
         break;
             SF_SIZES(SF_CASE)
 #undef SF_CASE
@@ -943,34 +929,34 @@ __global__ __launch_bounds__(BS) void k_xpass_mixed(const XArgs<T>* __restrict__
 }
 
 template <typename T, int R1F>
-static void launch_xpass_mixed_r(const XArgs<T>* args, const int* start, int nruns, int total, int nmax, int grid,
+static void launch_xpass_mixed_r(const XArgs<T>* args, const int2* items, int total, int nmax, int grid,
                                  hipStream_t s) {
-    if (nmax <= 128) hipLaunchKernelGGL((k_xpass_mixed<T, 128, R1F>), dim3(grid), dim3(BS), 0, s, args, start, nruns, total);
-    else if (nmax <= 256) hipLaunchKernelGGL((k_xpass_mixed<T, 256, R1F>), dim3(grid), dim3(BS), 0, s, args, start, nruns, total);
-    else hipLaunchKernelGGL((k_xpass_mixed<T, 512, R1F>), dim3(grid), dim3(BS), 0, s, args, start, nruns, total);
+    if (nmax <= 128) hipLaunchKernelGGL((k_xpass_mixed<T, 128, R1F>), dim3(grid), dim3(BS), 0, s, args, items, total);
+    else if (nmax <= 256) hipLaunchKernelGGL((k_xpass_mixed<T, 256, R1F>), dim3(grid), dim3(BS), 0, s, args, items, total);
+    else hipLaunchKernelGGL((k_xpass_mixed<T, 512, R1F>), dim3(grid), dim3(BS), 0, s, args, items, total);
 }
 
 // the variant compiled for N1 up to 128, 256 or 512 that covers nmax, with
 // the default FFT plans (r1f = 0) or first radix r1f = 8 where possible
 template <typename T>
-hipError_t launch_xpass_mixed(const XArgs<T>* args, const int* start, int nruns, int total, int nmax, int r1f,
+hipError_t launch_xpass_mixed(const XArgs<T>* args, const int2* items, int total, int nmax, int r1f,
                               int grid, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     if (nmax > 512) return hipErrorInvalidValue;
-    if (r1f == 0) launch_xpass_mixed_r<T, 0>(args, start, nruns, total, nmax, grid, s);
-    else if (r1f == 8) launch_xpass_mixed_r<T, 8>(args, start, nruns, total, nmax, grid, s);
+    if (r1f == 0) launch_xpass_mixed_r<T, 0>(args, items, total, nmax, grid, s);
+    else if (r1f == 8) launch_xpass_mixed_r<T, 8>(args, items, total, nmax, grid, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_xpass_batch(const XArgs<T>* args, const int* start, int nruns, int total, int N1, int grid,
+hipError_t launch_xpass_batch(const XArgs<T>* args, const int2* items, int total, int N1, int grid,
                               hipStream_t s) {
     if (total <= 0) return hipSuccess;
     switch (N1) {
 #define SF_CASE(n)                                                                                        \
     case n:                                                                                               \
-        hipLaunchKernelGGL((k_xpass_batch<T, n>), dim3(grid), dim3(BS), 0, s, args, start, nruns, total); \
+        hipLaunchKernelGGL((k_xpass_batch<T, n>), dim3(grid), dim3(BS), 0, s, args, items, total);        \
         return hipGetLastError();
         SF_SIZES(SF_CASE)
 #undef SF_CASE
@@ -1745,9 +1731,9 @@ hipError_t launch_diffprec(const DiffPrecArgs<T>& p, hipStream_t s) {
     template int xpass_slots<T>(int, bool, bool, int);
 
 #define SF_INST_BATCH(T) \
-    template hipError_t launch_modal_batch<T>(const ModalArgs<T>*, const int*, int, int, int, int, hipStream_t); \
-    template hipError_t launch_xpass_batch<T>(const XArgs<T>*, const int*, int, int, int, int, hipStream_t); \
-    template hipError_t launch_xpass_mixed<T>(const XArgs<T>*, const int*, int, int, int, int, int, hipStream_t); \
-    template hipError_t launch_modal_mixed<T>(const ModalArgs<T>*, const int*, int, int, int, int, int, hipStream_t);
+    template hipError_t launch_modal_batch<T>(const ModalArgs<T>*, const int2*, int, int, int, hipStream_t); \
+    template hipError_t launch_xpass_batch<T>(const XArgs<T>*, const int2*, int, int, int, hipStream_t); \
+    template hipError_t launch_xpass_mixed<T>(const XArgs<T>*, const int2*, int, int, int, int, hipStream_t); \
+    template hipError_t launch_modal_mixed<T>(const ModalArgs<T>*, const int2*, int, int, int, int, hipStream_t);
 
 }  // namespace sf

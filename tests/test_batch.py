@@ -145,3 +145,23 @@ def test_radix8_plans_of_larger_grids_fp64():
             print(runs[i][:2], f, "%.2e" % err, flush=True)
             assert err <= (1e-11 if f == "p" else 1e-12), (i, f, err)
     b.close()
+
+
+@pytest.mark.parametrize("runs", [12, 13, 26])
+def test_items_of_many_runs_fp64(runs):
+    """The item table puts every 64 work items in another order and leaves the
+    rest as it is: 60, 65 and 130 tiles of four modes (A1 = 17), bit for bit."""
+    import stratiflow_amd as sf
+    sizes = [(32, 48 + 16 * (i % 3), 500.0 + 100 * i, 0.1, 0.01) for i in range(runs)]
+    batched = [_make(*r, seed=400 + i, prec=8) for i, r in enumerate(sizes)]
+    twins = [_make(*r, seed=400 + i, prec=8) for i, r in enumerate(sizes)]
+    b = sf.Batch(batched)
+    for m in (sf.BATCH_MIXED, sf.BATCH_GROUPED):
+        b.select(sf.BATCH_MIXED, m)
+        b.step(2)
+        for t in twins:
+            t.TimeStep(2)
+    for i, (s, t) in enumerate(zip(batched, twins)):
+        for f in ("u1", "u3", "b", "p"):
+            assert np.array_equal(s.get(f), t.get(f)), (i, f)
+    b.close()
