@@ -527,10 +527,16 @@ constexpr int xpass_waves() {
     return (std::is_same<T, float>::value && THREED && !LIN) ? 4 : 1;
 }
 
-// threads per x-pass block (a multiple of 64)
-template <typename T, bool THREED, bool LIN>
+// threads per x-pass block (a multiple of 64).  A level of a short line is a
+// chain of phases with 32..128 items each, which a block of four waves leaves
+// mostly idle while its waves keep other blocks off the CU: with fewer
+// waves a block, more blocks are resident, each with fewer levels.  Per launch, 256
+// -> 128 -> 64 threads: 96x48x100 FP32 23.6 -> 22.1 -> 20.5 us, FP64 32.2 -> 27.1 ->
+// 25.2; 64x32x64 FP64 17.9 -> 15.3 -> 13.2; 128x64x128 FP32 30.5 -> 25.8 -> 27.1, FP64
+// 54.0 -> 40.5 -> 42.0; 192x96x192 FP32 66.9 -> 68.9.
+template <typename T, int N1, bool THREED, bool LIN>
 constexpr int xpass_bs() {
-    return BS;
+    return !THREED || N1 > 128 ? BS : N1 > 96 ? 128 : 64;
 }
 
 // LDS values of one x-pass block: NP product lines and a ring of 3 x 2 input
@@ -562,7 +568,7 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
     constexpr int NP = THREED ? 6 : 3;     // product pair lines per level
     constexpr int NB = NP + NI;            // lines per batched FFT
     constexpr int AMAX = N1 / 3;           // A1 <= N1/3
-    constexpr int XB = xpass_bs<T, THREED, LIN>();
+    constexpr int XB = xpass_bs<T, N1, THREED, LIN>();
     constexpr int FI = (NI * AMAX + XB - 1) / XB;
     constexpr int WI = LIN ? (N1 + XB - 1) / XB : 1;  // x points per thread
     // lds: [NP product lines][ring slot 0: NI lines][slot 1][slot 2]
@@ -809,7 +815,7 @@ __device__ __forceinline__ void xpass_body(const XArgs<T>& A, const int bx, cons
 }
 
 template <typename T, int N1, bool THREED, bool LIN>
-__global__ __launch_bounds__((xpass_bs<T, THREED, LIN>())) __attribute__((amdgpu_waves_per_eu(xpass_waves<T, THREED, LIN>()))) void k_xpass(
+__global__ __launch_bounds__((xpass_bs<T, N1, THREED, LIN>())) __attribute__((amdgpu_waves_per_eu(xpass_waves<T, THREED, LIN>()))) void k_xpass(
     XArgs<T> A) {
     __shared__ cx<T> lds[xpass_lds<N1, THREED>()];
     xpass_body<T, N1, THREED, LIN>(A, blockIdx.x, blockIdx.y, lds);
@@ -886,7 +892,7 @@ hipError_t launch_xbase(const XBaseArgs<T>& a, int N1, int N2, bool threeD, hipS
 template <typename T, int N1>
 __global__ __launch_bounds__(BS) void k_xpass_batch(const XArgs<T>* __restrict__ args, const int2* __restrict__ items,
                                                     int total) {
-    static_assert(xpass_bs<T, false, false>() == BS, "the batched 2D x-pass runs blocks of BS threads");
+    static_assert(xpass_bs<T, N1, false, false>() == BS, "the batched 2D x-pass runs blocks of BS threads");
     __shared__ cx<T> lds[xpass_lds<N1, false>()];
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         const int2 it = items[item];  // run, item of the run
@@ -974,7 +980,7 @@ static hipError_t launch_xpass_v(const XArgs<T>& a, int N2, hipStream_t s) {
         if (a.zch < 1 || a.A1 > N1 / 3) return hipErrorInvalidValue;
         const int nblk = (a.N3 + a.zch - 1) / a.zch;
         dim3 grid(nblk, THREED ? N2 : 1);
-        hipLaunchKernelGGL((k_xpass<T, N1, THREED, LIN>), grid, dim3(xpass_bs<T, THREED, LIN>()), 0, s, a);
+        hipLaunchKernelGGL((k_xpass<T, N1, THREED, LIN>), grid, dim3(xpass_bs<T, N1, THREED, LIN>()), 0, s, a);
         return hipGetLastError();
     }
 }
@@ -1007,7 +1013,8 @@ static int xpass_resident(int ncu) {
         return 0;
     } else {
         int per = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_xpass<T, N1, THREED, LIN>, xpass_bs<T, THREED, LIN>(), 0) != hipSuccess)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_xpass<T, N1, THREED, LIN>,
+                                                         xpass_bs<T, N1, THREED, LIN>(), 0) != hipSuccess)
             per = 1;
         return (per < 1 ? 1 : per) * ncu;
     }

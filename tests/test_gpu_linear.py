@@ -83,3 +83,19 @@ def test_linear_base_of_every_point_split(shape, prec):
         print(shape, prec, f, "%.2e" % e, flush=True)
         assert e < (1e-9 if prec == 8 else 1e-4), f
     s.close()
+
+
+@pytest.mark.parametrize("linear", [False, True])
+@pytest.mark.parametrize("shape", [(6, 6, 8, 0), (64, 6, 20, 0), (96, 48, 36, 0), (128, 64, 92, 0), (192, 6, 20, 0)])
+def test_products_of_every_block_size(shape, linear):
+    """x-pass blocks of 64, 128 and 256 threads, with one and two points of a
+    line per thread and columns that end inside a block's levels."""
+    s, o, keep = _with_base(shape, 8)
+    for _ in range(2):
+        s.TimeStepLinear(1) if linear else s.TimeStep(1)
+        o.step_linear(1) if linear else o.step(1)
+    for f in fields(shape[3]):
+        e = rel_l2(s.get(f), o.get_modal(f))
+        print(shape, linear, f, "%.2e" % e, flush=True)
+        assert e < 1e-9, f  # as the steps above
+    s.close()
