@@ -101,7 +101,6 @@ struct Ctx {
     double* partial = nullptr;
     double* scal = nullptr;
     double* scal_host = nullptr;
-    unsigned* ticket = nullptr;       // of the inner products' blocks
     DotResult* dot_host = nullptr;    // pinned: what the inner products leave for the host
     unsigned dot_call = 0;            // number of the last inner-product launch
     std::vector<double> zc_host;  // double copy of the coefficient table
@@ -209,7 +208,6 @@ struct Ctx {
         tw2 = dalloc<V>(2 * N2);
         twx = dalloc<V>(3 * N1 / 2);
         partial = dalloc<double>(DOT_MAX * DOT_BLOCKS);
-        ticket = dalloc<unsigned>(1);
         scal = dalloc<double>(16);
 
         // solver fields
@@ -955,7 +953,6 @@ struct Ctx {
         d.A1 = unsigned(A1);
         d.N3 = unsigned(N3);
         d.partial = partial;
-        d.ticket = ticket;
         d.host = dot_host;
         d.call = ++dot_call;
         const int sums = dot_sums(nmodal);

@@ -19,14 +19,15 @@ __device__ __forceinline__ double wave_sum(double v) {
 //   sum_z w_z sum_modes c_m Re(a conj b),  c = 1 for mode (0,0), 2 otherwise,
 // of up to DOT_MAX field pairs (blockIdx.y) in one launch.
 //
-// A 2D field is 0.2-0.7 MB, so latency and launches bound this, not HBM: the
+// A 2D field is 0.2-0.7 MB, so latency and launches bound this, not HBM: a
 // separate finishing kernel, the copy of the result to the host and the wait
 // on the stream cost more than the sums.  Results go straight to pinned host
 // memory, which the host watches.  Up to DOT_HOST blocks each write their own sum
-// and the host adds them; beyond that every block draws a ticket and the one with
-// the last adds the partials (through agent-scope accesses: the blocks' XCDs have
-// separate L2s), which costs 2 us more.  Either way the sums are added in block
-// order: the same bits on every call.
+// and the host adds them; the partials of more blocks are added by a second launch.
+// (A ticket by which the last block adds them is one atomic per block on one
+// address: the four pairs of an energy of 384x192x384 FP32 took 168 us with it,
+// 49 without, one pair 47 and 23; 512x1x512 FP32 takes 13 and 11.)
+// Either way the sums are added in a fixed order: the same bits on every call.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void dot_send(DotWord* to, double v, unsigned call) {
     const unsigned long long b = __double_as_longlong(v);
@@ -37,7 +38,6 @@ __device__ __forceinline__ void dot_send(DotWord* to, double v, unsigned call) {
 template <typename T>
 __global__ __launch_bounds__(FB) void k_dot(DotArgs<T> A) {
     __shared__ double red[FB / 64];
-    __shared__ bool last;
     const int y = blockIdx.y;
     const cx<T>* __restrict__ a = A.a[y];
     const cx<T>* __restrict__ b = A.b[y];
@@ -77,27 +77,19 @@ __global__ __launch_bounds__(FB) void k_dot(DotArgs<T> A) {
         double s = 0;
 #pragma unroll
         for (int i = 0; i < FB / 64; ++i) s += red[i];
-        if (gridDim.x <= DOT_HOST) {
-            dot_send(&A.host->sum[y][blockIdx.x], s, A.call);
-            last = false;
-        } else {
-            __hip_atomic_store(A.partial + y * gridDim.x + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned t = __hip_atomic_fetch_add(A.ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-            last = t + 1 == gridDim.x * gridDim.y;
-        }
+        if (gridDim.x <= DOT_HOST) dot_send(&A.host->sum[y][blockIdx.x], s, A.call);
+        else A.partial[y * gridDim.x + blockIdx.x] = s;
     }
-    __syncthreads();
-    if (!last) return;  // block-uniform
-    // one wave per pair
-    if (wave < int(gridDim.y)) {
-        double s = 0;
-        for (unsigned i = lane; i < gridDim.x; i += 64)
-            s += __hip_atomic_load(A.partial + wave * gridDim.x + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s = wave_sum(s);
-        if (lane == 0) dot_send(&A.host->sum[wave][0], s, A.call);
-    }
-    if (threadIdx.x == 0)
-        __hip_atomic_store(A.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+}
+
+// one wave per pair adds its partials
+static __global__ __launch_bounds__(64) void k_dot_sum(const double* __restrict__ partial, int blocks, DotResult* host,
+                                                       unsigned call) {
+    const int y = blockIdx.x;
+    double s = 0;
+    for (int i = threadIdx.x; i < blocks; i += 64) s += partial[y * blocks + i];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) dot_send(&host->sum[y][0], s, call);
 }
 
 // Blocks per pair: four elements a thread, up to DOT_BLOCKS where HBM bandwidth
@@ -115,9 +107,11 @@ int dot_sums(size_t n) {
 
 template <typename T>
 hipError_t launch_dot(const DotArgs<T>& a, int pairs, hipStream_t s) {
-    static_assert(DOT_MAX <= FB / 64, "the last block adds one pair per wave");
     if (pairs < 1 || pairs > DOT_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_dot<T>), dim3(dot_blocks(a.n), pairs), dim3(FB), 0, s, a);
+    const unsigned blocks = dot_blocks(a.n);
+    hipLaunchKernelGGL((k_dot<T>), dim3(blocks, pairs), dim3(FB), 0, s, a);
+    if (blocks > DOT_HOST)
+        hipLaunchKernelGGL(k_dot_sum, dim3(pairs), dim3(64), 0, s, a.partial, int(blocks), a.host, a.call);
     return hipGetLastError();
 }
 

@@ -152,7 +152,7 @@ template <typename T>
 hipError_t launch_x_r2c(const XTArgs<T>& a, int N1, int N2, hipStream_t s);
 template <typename T>
 hipError_t launch_x_sum(const XSumArgs<T>& a, int N1, int N2, hipStream_t s);
-// FP64 inner products (sf_fields.hip): one launch for up to DOT_MAX pairs, the
+// FP64 inner products (sf_fields.hip): up to DOT_MAX pairs per call, the
 // results in pinned host memory
 constexpr int DOT_MAX = 4;
 constexpr int DOT_BLOCKS = 1024;  // blocks (partial sums) per pair
@@ -174,7 +174,6 @@ struct DotArgs {
     const T* w[DOT_MAX];  // vertical weights of each pair
     unsigned n, A1, N3;   // n = A1*A2*N3 values per field
     double* partial;      // DOT_MAX * DOT_BLOCKS values
-    unsigned* ticket;     // zero between launches
     DotResult* host;
     unsigned call;        // number of the call
 };
