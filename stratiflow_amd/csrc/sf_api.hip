@@ -733,15 +733,19 @@ struct Ctx {
     int adj_terms() const { return three ? 12 : 6; }
     bool has_field(int i) const { return three || i != 1; }
 
+    // takes the buffers that are not there yet: one allocation may have failed in
+    // an earlier call
     void adjoint_alloc() {
-        if (adjQ[0]) return;
+        auto take = [&](T*& p) {
+            if (!p) p = dalloc<T>(nnodal);
+        };
         for (int i = 0; i < 4; ++i) {
             if (!has_field(i)) continue;
-            adjT[i] = dalloc<T>(nnodal);
-            adjDX[i] = dalloc<T>(nnodal);
-            if (three) adjDY[i] = dalloc<T>(nnodal);
+            take(adjT[i]);
+            take(adjDX[i]);
+            if (three) take(adjDY[i]);
         }
-        for (int q = 0; q < adj_terms(); ++q) adjQ[q] = dalloc<T>(nnodal);
+        for (int q = 0; q < adj_terms(); ++q) take(adjQ[q]);
     }
 
     // nodal totals and their horizontal derivatives (UpdateAdjointVariables,

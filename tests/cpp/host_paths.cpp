@@ -1,0 +1,222 @@
+// Host paths of the library on a stand-in for the HIP runtime: device memory is
+// host memory, kernels are counted and not run, and allocations fail when the
+// scenario says so.  The definitions here come before the runtime's own in the
+// program's symbol lookup, so the library as built is what runs.
+//   host_paths <scenario>      prints what went wrong and exits 1, or "ok"
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "sfhip.h"
+
+struct dim3 {
+    unsigned x, y, z;
+};
+
+namespace {
+std::set<void*> live;           // device allocations
+long mallocs_left = -1;         // allocations until they fail (-1: never)
+std::vector<std::string> launched;
+int graph_launches = 0;
+int null_stream_ops = 0;        // copies and clears outside any stream
+struct Config {
+    dim3 g, b;
+    size_t lds;
+    void* stream;
+} config;
+std::map<const void*, std::string>& kernels() {
+    static std::map<const void*, std::string> m;  // filled before main
+    return m;
+}
+
+int failures = 0;
+#define EXPECT(c, ...)                    \
+    do {                                  \
+        if (!(c)) {                       \
+            ++failures;                   \
+            std::printf("FAILED: %s: ", #c); \
+            std::printf(__VA_ARGS__);     \
+            std::printf("\n");            \
+        }                                 \
+    } while (0)
+}  // namespace
+
+extern "C" {
+void** __hipRegisterFatBinary(const void*) {
+    static void* h;
+    return &h;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+    kernels()[host] = name;
+}
+void __hipRegisterVar(void**, void*, char*, const char*, int, size_t, int, int) {}
+int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void* s) {
+    config = {g, b, lds, s};
+    return 0;
+}
+int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, void** s) {
+    *g = config.g;
+    *b = config.b;
+    *lds = config.lds;
+    *s = config.stream;
+    return 0;
+}
+int hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, void*) {
+    launched.push_back(kernels()[f]);
+    return 0;
+}
+int hipMalloc(void** p, size_t n) {
+    *p = nullptr;
+    if (mallocs_left == 0) return 2;  // out of memory
+    if (mallocs_left > 0) --mallocs_left;
+    *p = std::calloc(n, 1);
+    live.insert(*p);
+    return 0;
+}
+int hipFree(void* p) {
+    if (p && !live.erase(p)) EXPECT(false, "free of %p, which is no allocation", p);
+    std::free(p);
+    return 0;
+}
+int hipHostMalloc(void** p, size_t n, unsigned) {
+    *p = std::calloc(n, 1);
+    return 0;
+}
+int hipHostFree(void* p) {
+    std::free(p);
+    return 0;
+}
+int hipMemcpyAsync(void* d, const void* s, size_t n, int, void* stream) {
+    null_stream_ops += stream == nullptr;
+    std::memmove(d, s, n);
+    return 0;
+}
+int hipMemsetAsync(void* d, int v, size_t n, void* stream) {
+    null_stream_ops += stream == nullptr;
+    std::memset(d, v, n);
+    return 0;
+}
+int hipMemcpy(void* d, const void* s, size_t n, int k) { return hipMemcpyAsync(d, s, n, k, nullptr); }
+int hipMemset(void* d, int v, size_t n) { return hipMemsetAsync(d, v, n, nullptr); }
+int hipStreamCreateWithFlags(void** s, unsigned) {
+    *s = std::malloc(1);
+    return 0;
+}
+int hipStreamDestroy(void* s) {
+    std::free(s);
+    return 0;
+}
+int hipStreamSynchronize(void*) { return 0; }
+int hipEventCreate(void** e) {
+    *e = std::malloc(1);
+    return 0;
+}
+int hipEventDestroy(void* e) {
+    std::free(e);
+    return 0;
+}
+int hipEventRecord(void*, void*) { return 0; }
+int hipEventSynchronize(void*) { return 0; }
+int hipEventElapsedTime(float* ms, void*, void*) {
+    *ms = 1.0f;
+    return 0;
+}
+int hipStreamBeginCapture(void*, int) { return 0; }
+int hipStreamEndCapture(void*, void** g) {
+    *g = std::malloc(1);
+    return 0;
+}
+int hipGraphInstantiate(void** e, void*, void*, char*, size_t) {
+    *e = std::malloc(1);
+    return 0;
+}
+int hipGraphDestroy(void* g) {
+    std::free(g);
+    return 0;
+}
+int hipGraphExecDestroy(void* e) {
+    std::free(e);
+    return 0;
+}
+int hipGraphLaunch(void*, void*) {
+    ++graph_launches;
+    return 0;
+}
+int hipGetDevice(int* d) {
+    *d = 0;
+    return 0;
+}
+int hipDeviceGetAttribute(int* v, int, int) {
+    *v = 256;
+    return 0;
+}
+int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
+    *n = 4;
+    return 0;
+}
+int hipFuncSetAttribute(const void*, int, int) { return 0; }
+int hipGetSymbolAddress(void** p, const void*) {
+    static double scratch[1024];
+    *p = scratch;
+    return 0;
+}
+int hipGetLastError() { return 0; }
+const char* hipGetErrorString(int) { return "stand-in error"; }
+}
+
+static sf_ctx* context(int N1, int N2, int N3, int precision) {
+    const sf_grid g = {N1, N2, N3, N2 > 1 ? SF_THREE_D : SF_TWO_D};
+    const sf_flow f = {14.28, 7.14, 10.0, 1000.0, 0.1, 1.0, 0};
+    sf_ctx* c = nullptr;
+    const int rc = sf_ctx_create(&g, &f, precision, &c);
+    EXPECT(rc == SF_OK, "context: %s", sf_last_error(nullptr));
+    if (rc != SF_OK) std::exit(1);
+    return c;
+}
+
+// An adjoint step whose n-th allocation fails reports it, and so does the next
+// one while memory is short, without a launch; with memory back it runs on the
+// buffers of a context that never failed.
+static void adjoint_memory() {
+    size_t whole = 0;
+    for (int fail = -1; fail < 24; ++fail) {
+        sf_ctx* c = context(24, 12, 16, 8);
+        sf_field* f[4];
+        for (int i = 0; i < 4; ++i) sf_field_alloc(c, SF_MODAL, i == 2 ? SF_DIRICHLET : SF_NEUMANN, &f[i]);
+        launched.clear();
+        if (fail >= 0) {
+            mallocs_left = fail;
+            for (int again = 0; again < 2; ++again) {
+                const int rc = sf_step_adjoint(c, f, f);
+                EXPECT(rc != SF_OK && launched.empty(), "allocation %d, attempt %d: rc %d, %zu launches", fail, again, rc,
+                       launched.size());
+            }
+            mallocs_left = -1;
+        }
+        const int rc = sf_step_adjoint(c, f, f);
+        EXPECT(rc == SF_OK && !launched.empty(), "allocation %d, memory back: rc %d", fail, rc);
+        if (fail < 0) whole = live.size();
+        EXPECT(live.size() == whole, "allocation %d: %zu buffers, %zu without a failure", fail, live.size(), whole);
+        for (sf_field* x : f) sf_field_free(x);
+        sf_ctx_destroy(c);
+        EXPECT(live.empty(), "allocation %d: %zu buffers left", fail, live.size());
+    }
+}
+
+int main(int argc, char** argv) {
+    const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory}};
+    const auto s = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
+    if (s == scenarios.end()) {
+        std::printf("unknown scenario\n");
+        return 2;
+    }
+    s->second();
+    if (failures) return 1;
+    std::printf("ok\n");
+    return 0;
+}
