@@ -102,7 +102,9 @@ struct Ctx {
     double* scal = nullptr;
     double* scal_host = nullptr;
     DotResult* dot_host = nullptr;    // pinned: what the inner products leave for the host
-    unsigned dot_call = 0;            // number of the last inner-product launch
+    // number of the last inner-product launch; it starts short of its overflow so
+    // that the wrap is met early
+    unsigned dot_call = 0xffffff00u;
     std::vector<double> zc_host;  // double copy of the coefficient table
 
     sf_field state[17];
@@ -958,7 +960,11 @@ struct Ctx {
         d.N3 = unsigned(N3);
         d.partial = partial;
         d.host = dot_host;
-        d.call = ++dot_call;
+        if (++dot_call == 0) {  // nothing is in flight: every call waits for its own results
+            std::memset(dot_host, 0, sizeof(DotResult));
+            dot_call = 1;
+        }
+        d.call = dot_call;
         const int sums = dot_sums(nmodal);
         check(launch_dot<T>(d, pairs, stream), "dot");
         auto word = [&](int i, int k, int h) {

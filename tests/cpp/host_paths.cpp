@@ -208,8 +208,22 @@ static void adjoint_memory() {
     }
 }
 
+// No kernel runs, so no inner product may return: every call says that its result
+// did not arrive, whatever its number (numbers wrap, and no word of the results
+// may be taken for one of a call that it does not belong to).
+static void inner_product_results() {
+    sf_ctx* c = context(24, 1, 16, 8);
+    for (int i = 0; i < 1000; ++i) {
+        double ke = -1, pe = -1;
+        const int rc = sf_energy(c, &ke, &pe);
+        EXPECT(rc == SF_ERR_STATE, "call %d: rc %d, energies %g %g", i, rc, ke, pe);
+    }
+    sf_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
-    const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory}};
+    const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory},
+                                                         {"inner_product_results", inner_product_results}};
     const auto s = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (s == scenarios.end()) {
         std::printf("unknown scenario\n");

@@ -196,3 +196,19 @@ def test_whole_field_transforms(shape, prec):
     assert e < tol and b < 2 * tol
     assert np.array_equal(got[..., 0], got[..., 1])
     s.close()
+
+
+@pytest.mark.parametrize("shape", [(24, 1, 64, 1), (192, 96, 192, 0)])
+def test_many_inner_products(shape):
+    """The number that the results of a call carry starts 256 calls before its
+    overflow: the results on both sides of it are those of the first calls (on
+    the blocks' own sums and on the total of a second launch)."""
+    s = solver(shape, 8)
+    for n in ("u1", "u3", "b"):
+        s.state(n).assign(random_field(s, sf.DIRICHLET if n == "u3" else sf.NEUMANN, 4)[0])
+    u, b = s.state("u1"), s.state("b")
+    first = s.energies() + (s.InnerProd(u, b),)
+    assert all(np.isfinite(first)) and first[0] > 0 and first[1] > 0
+    for i in range(300):
+        assert s.energies() + (s.InnerProd(u, b),) == first, i
+    s.close()
