@@ -1319,6 +1319,7 @@ struct Batch {
 
     void build() {
         release_graph();
+        dts.clear();  // until every table is there: the next step builds again
         if (xplan != SF_BATCH_GROUPED) {
             build_xgroup(xmix, xmix.zch, xmix.grid, xr1f());
         } else {
@@ -1332,7 +1333,6 @@ struct Batch {
                 build_mgroup(mmix[k], true, [&](int r) { return stage_args(r, k); });
             }
         }
-        dts.clear();
         for (auto* c : runs) dts.push_back(c->dt);
         launches_per_step = 3 * ((xplan != SF_BATCH_GROUPED ? 1 : int(xg.size())) +
                                  (mplan == SF_BATCH_GROUPED ? int(mg[0].size()) : 1));
@@ -1522,8 +1522,8 @@ struct Batch {
     void step(int n, double* ms_out = nullptr) {
         SF_REQUIRE(n >= 0, SF_ERR_ARG, "negative step count");
         sync_runs();
-        bool stale = false;
-        for (size_t i = 0; i < runs.size(); ++i) stale = stale || (runs[i]->dt != dts[i]);
+        bool stale = dts.size() != runs.size();
+        for (size_t i = 0; i < dts.size(); ++i) stale = stale || (runs[i]->dt != dts[i]);
         if (stale) build();
         int first = 0;
         bool snap = false;

@@ -221,9 +221,37 @@ static void inner_product_results() {
     sf_ctx_destroy(c);
 }
 
+// A plan whose tables cannot be allocated is reported, and so is every step until
+// they can be: no launch goes without its tables.
+static void batch_memory() {
+    for (int fail = 0; fail < 8; ++fail) {
+        sf_ctx* c[2] = {context(24, 1, 16, 8), context(32, 1, 16, 8)};
+        sf_batch* b = nullptr;
+        EXPECT(sf_batch_create(c, 2, &b) == SF_OK, "batch: %s", sf_batch_last_error(nullptr));
+        if (!b) std::exit(1);
+        EXPECT(sf_batch_step(b, 1) == SF_OK, "first step");
+        mallocs_left = fail;
+        EXPECT(sf_batch_select(b, SF_BATCH_MIXED, SF_BATCH_MIXED) != SF_OK, "allocation %d: select succeeded", fail);
+        mallocs_left = 0;
+        launched.clear();
+        graph_launches = 0;
+        for (int again = 0; again < 2; ++again) {
+            const int rc = sf_batch_step(b, 1);
+            EXPECT(rc != SF_OK && launched.empty() && graph_launches == 0, "allocation %d, step %d: rc %d, %zu launches", fail,
+                   again, rc, launched.size());
+        }
+        mallocs_left = -1;
+        EXPECT(sf_batch_step(b, 1) == SF_OK && graph_launches == 1, "allocation %d, memory back", fail);
+        sf_batch_destroy(b);
+        for (sf_ctx* x : c) sf_ctx_destroy(x);
+        EXPECT(live.empty(), "allocation %d: %zu buffers left", fail, live.size());
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory},
-                                                         {"inner_product_results", inner_product_results}};
+                                                         {"inner_product_results", inner_product_results},
+                                                         {"batch_memory", batch_memory}};
     const auto s = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (s == scenarios.end()) {
         std::printf("unknown scenario\n");
