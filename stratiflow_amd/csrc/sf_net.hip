@@ -530,14 +530,6 @@ static unsigned grid_for(size_t n, unsigned cap = 4096) {
     return unsigned(b < 1 ? 1 : b);
 }
 
-template <typename P>
-static P* dalloc(size_t n) {
-    void* p = nullptr;
-    SF_HIP(hipMalloc(&p, (n ? n : 1) * sizeof(P)));
-    SF_HIP(hipMemset(p, 0, (n ? n : 1) * sizeof(P)));
-    return static_cast<P*>(p);
-}
-
 struct Net {
     sf_ctx* ctx = nullptr;
     CtxInfo info{};
@@ -605,6 +597,24 @@ struct Net {
     }
 
     hipStream_t st() const { return info.stream; }
+
+    // Clears and copies take their turn on the context's stream: the default
+    // stream does not wait for it, so a copy there could overtake a queued apply
+    // or optimiser step that uses the same buffer.
+    template <typename P>
+    P* dalloc(size_t n) {
+        void* p = nullptr;
+        SF_HIP(hipMalloc(&p, (n ? n : 1) * sizeof(P)));
+        const hipError_t e = hipMemsetAsync(p, 0, (n ? n : 1) * sizeof(P), st());
+        if (e != hipSuccess) (void)hipFree(p);
+        SF_HIP(e);
+        return static_cast<P*>(p);
+    }
+    // between host and device; the host's buffer is free on return
+    void copy(void* to, const void* from, size_t bytes, hipMemcpyKind kind) {
+        SF_HIP(hipMemcpyAsync(to, from, bytes, kind, st()));
+        SF_HIP(hipStreamSynchronize(st()));
+    }
     size_t profiles() const { return size_t(info.A1) * info.A2; }
 
     void init(sf_ctx* c, int hidden, int layers, unsigned long long seed) {
@@ -655,8 +665,8 @@ struct Net {
         am = dalloc<float>(nparam);
         av = dalloc<float>(nparam);
         pmask = dalloc<unsigned char>(nparam);
-        SF_HIP(hipMemcpy(w, hw.data(), nparam * sizeof(float), hipMemcpyHostToDevice));
-        SF_HIP(hipMemcpy(pmask, hm.data(), nparam, hipMemcpyHostToDevice));
+        copy(w, hw.data(), nparam * sizeof(float), hipMemcpyHostToDevice);
+        copy(pmask, hm.data(), nparam, hipMemcpyHostToDevice);
         for (int l = 0; l < L; ++l) {
             Wb.push_back(dalloc<bf16>(size_t(KT) * C[l + 1] * C[l]));
             Wt.push_back(dalloc<bf16>(size_t(KT) * C[l + 1] * C[l]));
@@ -1005,17 +1015,14 @@ int sf_net_param_count(const sf_net* n, size_t* count) {
 
 int sf_net_get_params(sf_net* n, float* host) {
     if (!n || !host) return SF_ERR_ARG;
-    return net_call(n, [&](sf::net::Net& N) {
-        SF_HIP(hipMemcpy(host, N.w, N.nparam * sizeof(float), hipMemcpyDeviceToHost));
-    });
+    return net_call(n, [&](sf::net::Net& N) { N.copy(host, N.w, N.nparam * sizeof(float), hipMemcpyDeviceToHost); });
 }
 
 int sf_net_set_params(sf_net* n, const float* host) {
     if (!n || !host) return SF_ERR_ARG;
     return net_call(n, [&](sf::net::Net& N) {
-        SF_HIP(hipMemcpy(N.w, host, N.nparam * sizeof(float), hipMemcpyHostToDevice));
+        N.copy(N.w, host, N.nparam * sizeof(float), hipMemcpyHostToDevice);
         N.cast_weights();
-        SF_HIP(hipStreamSynchronize(N.st()));
     });
 }
 
@@ -1044,7 +1051,7 @@ int sf_net_forward_raw(sf_net* n, const float* in, int nprof, float* out) {
         N.ensure_work(P);
         std::vector<sf::net::bf16> h(P * N.C[0]);
         for (size_t i = 0; i < h.size(); ++i) h[i] = sf::net::bf16(in[i]);
-        SF_HIP(hipMemcpy(N.act[0], h.data(), h.size() * sizeof(sf::net::bf16), hipMemcpyHostToDevice));
+        N.copy(N.act[0], h.data(), h.size() * sizeof(sf::net::bf16), hipMemcpyHostToDevice);
         N.forward(int(P));
         SF_HIP(hipMemcpyAsync(out, N.pre[N.L - 1], P * N.C[N.L] * sizeof(float), hipMemcpyDeviceToHost, N.st()));
         SF_HIP(hipStreamSynchronize(N.st()));
@@ -1058,11 +1065,11 @@ int sf_net_grad_raw(sf_net* n, const float* in, const float* target, int nprof, 
         N.ensure_work(P);
         std::vector<sf::net::bf16> h(P * N.C[0]);
         for (size_t i = 0; i < h.size(); ++i) h[i] = sf::net::bf16(in[i]);
-        SF_HIP(hipMemcpy(N.act[0], h.data(), h.size() * sizeof(sf::net::bf16), hipMemcpyHostToDevice));
-        SF_HIP(hipMemcpy(N.tgt, target, P * N.C[N.L] * sizeof(float), hipMemcpyHostToDevice));
+        N.copy(N.act[0], h.data(), h.size() * sizeof(sf::net::bf16), hipMemcpyHostToDevice);
+        N.copy(N.tgt, target, P * N.C[N.L] * sizeof(float), hipMemcpyHostToDevice);
         N.forward(int(P));
         *loss = N.backward(int(P));
-        SF_HIP(hipMemcpy(grad, N.gr, N.nparam * sizeof(float), hipMemcpyDeviceToHost));
+        N.copy(grad, N.gr, N.nparam * sizeof(float), hipMemcpyDeviceToHost);
     });
 }
 

@@ -248,10 +248,48 @@ static void batch_memory() {
     }
 }
 
+// A network's copies and clears take their turn on its context's stream: what is
+// still queued there reads the weights, activations and training pairs that were
+// there when it was queued.
+static void net_stream() {
+    sf_ctx* c = context(24, 1, 16, 4);
+    sf_field* f[4];
+    for (int i = 0; i < 4; ++i) sf_field_alloc(c, SF_MODAL, i == 2 ? SF_DIRICHLET : SF_NEUMANN, &f[i]);
+    null_stream_ops = 0;
+    sf_net* n = nullptr;
+    EXPECT(sf_net_create(c, 32, 3, 1, &n) == SF_OK, "%s", sf_net_last_error(nullptr));
+    if (!n) std::exit(1);
+    auto expect = [&](const char* call) {
+        EXPECT(null_stream_ops == 0, "%s: %d outside the stream", call, null_stream_ops);
+        null_stream_ops = 0;
+    };
+    expect("create");
+    size_t count = 0;
+    sf_net_param_count(n, &count);
+    std::vector<float> p(count, 0.5f), q(count);
+    sf_net_set_params(n, p.data());
+    expect("set_params");
+    sf_net_get_params(n, q.data());
+    expect("get_params");
+    EXPECT(p == q, "parameters");
+    sf_net_apply(n, f, f);
+    expect("apply");
+    std::vector<float> x(2 * 16 * 32), y(2 * 16 * 32);
+    sf_net_forward_raw(n, x.data(), 2, y.data());
+    expect("forward_raw");
+    double loss = 0;
+    sf_net_grad_raw(n, x.data(), y.data(), 2, q.data(), &loss);
+    expect("grad_raw");
+    sf_net_destroy(n);
+    for (sf_field* g : f) sf_field_free(g);
+    sf_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory},
                                                          {"inner_product_results", inner_product_results},
-                                                         {"batch_memory", batch_memory}};
+                                                         {"batch_memory", batch_memory},
+                                                         {"net_stream", net_stream}};
     const auto s = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (s == scenarios.end()) {
         std::printf("unknown scenario\n");

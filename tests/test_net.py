@@ -185,3 +185,32 @@ def test_fused_application_matches_layers(shape, prec, hidden, layers):
         off = np.abs(got - want) > 16 * eps * (np.abs(act[n]) + np.abs(want)).max()
         assert off.mean() < 1e-3 and np.abs(got - want).max() <= 2.0 ** -7 * np.abs(want).max(), n
     s.close()
+
+
+@pytest.mark.gpu
+def test_parameters_take_their_turn():
+    """set_params and get_params after calls that are still queued: an apply uses
+    the parameters that it was called with, and the parameters read back are
+    those of the last optimiser step."""
+    import stratiflow_amd as sf
+    s = sf.IMEXRK(64, 1, 64, sf.TWO_D, 2 * np.pi / 0.44, np.pi / 0.44, 10.0, 1000.0, 0.1, 1.0, precision=8)
+    net = sf.Net(s, hidden=32, layers=3, seed=5)
+    rng = np.random.default_rng(6)
+    first, second = (_rand_params(rng, net.channels, 8, 6).astype(np.float32) for _ in range(2))
+    fin, quiet, queued = ([s.field(sf.MODAL, sf.DIRICHLET if i == 2 else sf.NEUMANN) if i != 1 else None for i in range(4)]
+                          for _ in range(3))
+    for f in fin:
+        if f is not None:
+            f.upload(rng.standard_normal(f.shape) + 1j * rng.standard_normal(f.shape))
+    net.set_params(first)
+    net.apply(fin, quiet)
+    s.synchronize()
+    for _ in range(3):
+        net.set_params(first)
+        s.TimeStep(200)  # milliseconds of work in front of the call
+        net.apply(fin, queued)
+        net.set_params(second)
+        for a, b in zip(quiet, queued):
+            assert a is None or np.array_equal(a.download(), b.download())
+    assert np.array_equal(net.get_params(), second)
+    s.close()
