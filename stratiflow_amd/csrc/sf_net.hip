@@ -690,13 +690,13 @@ struct Net {
     void ensure_work(size_t P) {
         if (P <= cap_pos) return;
         free_work();
-        cap_pos = P;
         for (int l = 0; l <= L; ++l) act.push_back(dalloc<bf16>(P * C[l]));
         for (int l = 0; l < L; ++l) pre.push_back(dalloc<float>(P * C[l + 1]));
         for (int l = 0; l < L; ++l) gbuf.push_back(dalloc<bf16>(P * C[l + 1]));
         tgt = dalloc<float>(P * C[L]);
         part_n = size_t(DW_BLOCKS) * KT * H * H;
         part = dalloc<float>(part_n);
+        cap_pos = P;  // every buffer is there
     }
 
     void conv(int NT, const bf16* in, int Cin, const bf16* W, const float* bias, int P, float* out_f, bf16* out_b,
@@ -889,6 +889,8 @@ struct Net {
         ensure_work(size_t(batch) * Z);
         if (didx_n < batch) {
             if (didx) (void)hipFree(didx);
+            didx = nullptr;
+            didx_n = 0;
             didx = dalloc<int>(batch);
             didx_n = batch;
         }

@@ -285,11 +285,37 @@ static void net_stream() {
     sf_ctx_destroy(c);
 }
 
+// A raw forward pass whose n-th allocation of twelve fails reports it, and so does
+// the next one while memory is short, without a launch; with memory back it runs.
+static void net_memory() {
+    for (int fail = 0; fail < 12; ++fail) {
+        sf_ctx* c = context(24, 1, 16, 4);
+        sf_net* n = nullptr;
+        EXPECT(sf_net_create(c, 32, 3, 1, &n) == SF_OK, "%s", sf_net_last_error(nullptr));
+        if (!n) std::exit(1);
+        std::vector<float> x(4 * 16 * 32), y(4 * 16 * 32);
+        EXPECT(sf_net_forward_raw(n, x.data(), 2, y.data()) == SF_OK, "two profiles");
+        launched.clear();
+        mallocs_left = fail;
+        for (int again = 0; again < 2; ++again) {
+            const int rc = sf_net_forward_raw(n, x.data(), 4, y.data());
+            EXPECT(rc != SF_OK && launched.empty(), "allocation %d, attempt %d: rc %d, %zu launches", fail, again, rc,
+                   launched.size());
+        }
+        mallocs_left = -1;
+        EXPECT(sf_net_forward_raw(n, x.data(), 4, y.data()) == SF_OK, "allocation %d, memory back", fail);
+        sf_net_destroy(n);
+        sf_ctx_destroy(c);
+        EXPECT(live.empty(), "allocation %d: %zu buffers left", fail, live.size());
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory},
                                                          {"inner_product_results", inner_product_results},
                                                          {"batch_memory", batch_memory},
-                                                         {"net_stream", net_stream}};
+                                                         {"net_stream", net_stream},
+                                                         {"net_memory", net_memory}};
     const auto s = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (s == scenarios.end()) {
         std::printf("unknown scenario\n");

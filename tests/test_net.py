@@ -190,8 +190,7 @@ def test_fused_application_matches_layers(shape, prec, hidden, layers):
 @pytest.mark.gpu
 def test_parameters_take_their_turn():
     """set_params and get_params after calls that are still queued: an apply uses
-    the parameters that it was called with, and the parameters read back are
-    those of the last optimiser step."""
+    the parameters that it was called with, and those read back are the last set."""
     import stratiflow_amd as sf
     s = sf.IMEXRK(64, 1, 64, sf.TWO_D, 2 * np.pi / 0.44, np.pi / 0.44, 10.0, 1000.0, 0.1, 1.0, precision=8)
     net = sf.Net(s, hidden=32, layers=3, seed=5)
