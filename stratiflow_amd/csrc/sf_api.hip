@@ -80,7 +80,7 @@ struct Ctx {
     sf_ctx* owner = nullptr;
     int N1 = 0, N2 = 0, N3 = 0, M1 = 0, A1 = 0, A2 = 0, dim = 0, N3p = 0;
     bool three = false;
-    int zch = 4, zch_lin = 4;  // z levels per x-pass block, nonlinear and linearised products
+    int zch = 4, zch_lin = 0;  // z levels per x-pass block, nonlinear and linearised products (0: not asked yet)
     int device = 0;  // the device current at creation
     double L1 = 0, L2 = 0, L3 = 0, Re = 0, Ri = 0, Pr = 0;
     bool evolve_bg = false;  // FlowParams::EvolveBackground
@@ -92,6 +92,10 @@ struct Ctx {
     hipStream_t stream = nullptr;
     std::vector<void*> allocs;
 
+    // Coefficients, wavenumbers and twiddles lie in one allocation, which starts
+    // at zc, with an image of it on the host, so that a change is one copy.
+    std::vector<T> table;
+    size_t level_values = 0;  // zc and zl together
     T* zc = nullptr;
     T* zl = nullptr;  // zc in the order of the modal kernels' lanes (ModalArgs)
     T *kx = nullptr, *ky = nullptr, *kx2 = nullptr, *ky2 = nullptr;
@@ -100,8 +104,8 @@ struct Ctx {
     V* tw1_r8 = nullptr;  // x twiddles of the plan with first radix 8 (made on first use)
     double* partial = nullptr;
     double* scal = nullptr;
-    double* scal_host = nullptr;
     DotResult* dot_host = nullptr;    // pinned: what the inner products leave for the host
+    double* scal_host = nullptr;      // behind it: what read_scalars fetches
     // number of the last inner-product launch; it starts short of its overflow so
     // that the wrap is met early
     unsigned dot_call = 0xffffff00u;
@@ -157,7 +161,6 @@ struct Ctx {
     ~Ctx() {
         if (stream) (void)hipStreamSynchronize(stream);
         for (void* p : allocs) (void)hipFree(p);
-        if (scal_host) (void)hipHostFree(scal_host);
         if (dot_host) (void)hipHostFree(dot_host);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
@@ -190,25 +193,16 @@ struct Ctx {
         A2 = three ? 2 * (N2 / 3) - 1 : 1;
         N3p = N3;
         zch = xpass_levels(N1, N2, N3, three, false, int(sizeof(T)));
-        zch_lin = xpass_levels(N1, N2, N3, three, true, int(sizeof(T)));
         nmodal = size_t(A1) * A2 * N3;
         nnodal = size_t(N1) * N2 * N3;
         SF_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         SF_HIP(hipEventCreate(&ev0));
         SF_HIP(hipEventCreate(&ev1));
-        SF_HIP(hipHostMalloc((void**)&scal_host, 16 * sizeof(double), hipHostMallocDefault));
-        SF_HIP(hipHostMalloc((void**)&dot_host, sizeof(DotResult), hipHostMallocCoherent));
+        SF_HIP(hipHostMalloc((void**)&dot_host, sizeof(DotResult) + 16 * sizeof(double), hipHostMallocCoherent));
         std::memset(dot_host, 0, sizeof(DotResult));
+        scal_host = reinterpret_cast<double*>(dot_host + 1);
 
-        zc = dalloc<T>(size_t(ZC_COUNT) * N3p);
-        zl = dalloc<T>(size_t(ZC_COUNT) * 64 * rows_per_lane());
-        kx = dalloc<T>(A1);
-        kx2 = dalloc<T>(A1);
-        ky = dalloc<T>(A2);
-        ky2 = dalloc<T>(A2);
-        tw1 = dalloc<V>(2 * N1);
-        tw2 = dalloc<V>(2 * N2);
-        twx = dalloc<V>(3 * N1 / 2);
+        make_tables();
         partial = dalloc<double>(DOT_MAX * DOT_BLOCKS);
         scal = dalloc<double>(16);
 
@@ -256,15 +250,58 @@ struct Ctx {
 
     int rows_per_lane() const { return (N3 + 63) / 64; }
 
-    void upload_coefficients() {
-        std::vector<T> h(zc_host.size());
-        for (size_t i = 0; i < h.size(); ++i) h[i] = T(zc_host[i]);
-        SF_HIP(hipMemcpyAsync(zc, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, stream));
+    void make_tables() {
+        size_t end = 0;
+        auto place = [&](size_t values) {
+            const size_t at = end;
+            end += (values + 63) / 64 * 64;
+            return at;
+        };
+        place(size_t(ZC_COUNT) * N3p);
+        const size_t lanes = place(size_t(ZC_COUNT) * 64 * rows_per_lane());
+        level_values = end;
+        const size_t k[4] = {place(A1), place(A1), place(A2), place(A2)};
+        const size_t w[3] = {place(4 * N1), place(4 * N2), place(3 * N1)};
+        zc = dalloc<T>(end);
+        zl = zc + lanes;
+        kx = zc + k[0];
+        kx2 = zc + k[1];
+        ky = zc + k[2];
+        ky2 = zc + k[3];
+        tw1 = reinterpret_cast<V*>(zc + w[0]);
+        tw2 = reinterpret_cast<V*>(zc + w[1]);
+        twx = reinterpret_cast<V*>(zc + w[2]);
+        table.assign(end, T(0));
+        // FFT twiddles, computed in double
+        auto tw = [&](void (*fill)(int, double*, double*), int n, int entries, const V* dst) {
+            std::vector<double> re(entries), im(entries);
+            fill(n, re.data(), im.data());
+            T* t = image(reinterpret_cast<const T*>(dst));
+            for (int i = 0; i < entries; ++i) {
+                t[2 * i] = T(re[i]);
+                t[2 * i + 1] = T(im[i]);
+            }
+        };
+        tw(fft_twiddles, N1, 2 * N1, tw1);
+        tw(fft_twiddles, N2, 2 * N2, tw2);
+        tw(xt_twiddles, N1, 3 * N1 / 2, twx);
+    }
+    T* image(const T* device) { return table.data() + (device - zc); }
+
+    // rows c0..c1 of zc_host into the image, in both orders
+    void put_levels(int c0, int c1) {
         const int M = rows_per_lane();
-        std::vector<T> l(size_t(ZC_COUNT) * 64 * M, T(0));
-        for (int c = 0; c < ZC_COUNT; ++c)
-            for (int j = 0; j < N3; ++j) l[(size_t(c) * M + j % M) * 64 + j / M] = h[size_t(c) * N3p + j];
-        SF_HIP(hipMemcpyAsync(zl, l.data(), l.size() * sizeof(T), hipMemcpyHostToDevice, stream));
+        for (int c = c0; c <= c1; ++c) {
+            const double* h = zc_host.data() + size_t(c) * N3p;
+            T* rows = image(zc) + size_t(c) * N3p;
+            T* lanes = image(zl) + size_t(c) * M * 64;
+            for (int j = 0, lane = 0; j < N3; ++lane)
+                for (int t = 0; t < M && j < N3; ++t, ++j) rows[j] = lanes[t * 64 + lane] = T(h[j]);
+        }
+    }
+    // the first n values of the image to the device
+    void upload_table(size_t n) {
+        SF_HIP(hipMemcpyAsync(zc, table.data(), n * sizeof(T), hipMemcpyHostToDevice, stream));
         SF_HIP(hipStreamSynchronize(stream));
     }
 
@@ -316,40 +353,20 @@ struct Ctx {
             Z(ZC_UBAR, j) = old.empty() ? 0.0 : old[size_t(ZC_UBAR) * N3p + j];
             Z(ZC_S, j) = old.empty() ? 1.0 : old[size_t(ZC_S) * N3p + j];
         }
-        upload_coefficients();
+        put_levels(0, ZC_COUNT - 1);
         // Fourier wavenumbers of the active modes (Differentiation.cpp:113-160)
-        std::vector<T> hkx(A1), hkx2(A1), hky(A2), hky2(A2);
         for (int j = 0; j < A1; ++j) {
             const double k = 2.0 * M_PI * kindex(N1, j) / L1;
-            hkx[j] = T(k);
-            hkx2[j] = T(-k * k);
+            image(kx)[j] = T(k);
+            image(kx2)[j] = T(-k * k);
         }
         for (int ja = 0; ja < A2; ++ja) {
             const int j2 = three ? ((ja < N2 / 3) ? ja : ja + N2 - 2 * (N2 / 3) + 1) : 0;
             const double k = 2.0 * M_PI * kindex(N2, j2) / L2;
-            hky[ja] = T(k);
-            hky2[ja] = T(-k * k);
+            image(ky)[ja] = T(k);
+            image(ky2)[ja] = T(-k * k);
         }
-        SF_HIP(hipMemcpyAsync(kx, hkx.data(), A1 * sizeof(T), hipMemcpyHostToDevice, stream));
-        SF_HIP(hipMemcpyAsync(kx2, hkx2.data(), A1 * sizeof(T), hipMemcpyHostToDevice, stream));
-        SF_HIP(hipMemcpyAsync(ky, hky.data(), A2 * sizeof(T), hipMemcpyHostToDevice, stream));
-        SF_HIP(hipMemcpyAsync(ky2, hky2.data(), A2 * sizeof(T), hipMemcpyHostToDevice, stream));
-        // FFT twiddles, computed in double
-        auto tw = [&](void (*table)(int, double*, double*), int n, int entries, V* dst) {
-            std::vector<double> re(entries), im(entries);
-            table(n, re.data(), im.data());
-            std::vector<V> w(entries);
-            for (int k = 0; k < entries; ++k) {
-                w[k].x = T(re[k]);
-                w[k].y = T(im[k]);
-            }
-            SF_HIP(hipMemcpyAsync(dst, w.data(), entries * sizeof(V), hipMemcpyHostToDevice, stream));
-            SF_HIP(hipStreamSynchronize(stream));
-        };
-        tw(fft_twiddles, N1, 2 * N1, tw1);
-        tw(fft_twiddles, N2, 2 * N2, tw2);
-        tw(xt_twiddles, N1, 3 * N1 / 2, twx);
-        SF_HIP(hipStreamSynchronize(stream));
+        upload_table(table.size());
     }
 
     // x-direction twiddles for the FFT plan with first radix r1f (0: default)
@@ -385,7 +402,9 @@ struct Ctx {
             zc_host[size_t(ZC_UBAR) * N3p + j] = U ? U[j] : 0.0;
             zc_host[size_t(ZC_S) * N3p + j] = S ? S[j] : 1.0;
         }
-        upload_coefficients();
+        static_assert(ZC_S == ZC_UBAR + 1, "the background's rows follow each other");
+        put_levels(ZC_UBAR, ZC_S);
+        upload_table(level_values);
     }
 
     // UpdateForTimestep (IMEXRK.h:506-508); the implicit matrices are rebuilt
@@ -412,6 +431,7 @@ struct Ctx {
     // stages add the U_ of their time), callers may between calls
     void linear_base() {
         if (!xbase) xbase = dalloc<XBase<T>>(nnodal);
+        if (zch_lin == 0) zch_lin = xpass_levels(N1, N2, N3, three, true, int(sizeof(T)));
         XBaseArgs<T> a{};
         a.N3 = N3;
         a.A1 = A1;

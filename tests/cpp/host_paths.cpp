@@ -23,6 +23,7 @@ long mallocs_left = -1;         // allocations until they fail (-1: never)
 std::vector<std::string> launched;
 int graph_launches = 0;
 int null_stream_ops = 0;        // copies and clears outside any stream
+int copies = 0;
 struct Config {
     dim3 g, b;
     size_t lds;
@@ -93,6 +94,7 @@ int hipHostFree(void* p) {
 }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int, void* stream) {
     null_stream_ops += stream == nullptr;
+    ++copies;
     std::memmove(d, s, n);
     return 0;
 }
@@ -310,12 +312,35 @@ static void net_memory() {
     }
 }
 
+// A new background or new flow parameters reach the device in one copy, and the
+// background is read back from there.
+static void table_copies() {
+    for (int precision = 4; precision <= 8; precision += 4) {
+        sf_ctx* c = context(24, 12, 100, precision);
+        std::vector<double> u(100), s(100), back(100);
+        for (int j = 0; j < 100; ++j) {
+            u[j] = j / 64.0;  // exact in either precision
+            s[j] = 1 + j / 128.0;
+        }
+        copies = 0;
+        EXPECT(sf_set_background(c, u.data(), s.data()) == SF_OK && copies == 1, "set_background: %d copies", copies);
+        const sf_flow f = {14.28, 7.14, 12.0, 500.0, 0.2, 2.0, 1};
+        copies = 0;
+        EXPECT(sf_set_flow(c, &f) == SF_OK && copies == 1, "set_flow: %d copies", copies);
+        EXPECT(sf_get_background(c, back.data()) == SF_OK && back == u, "the background that was set");
+        EXPECT(sf_set_flow(c, &f) == SF_OK && sf_get_background(c, back.data()) == SF_OK && back == u,
+               "the background after set_flow");
+        sf_ctx_destroy(c);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> scenarios = {{"adjoint_memory", adjoint_memory},
                                                          {"inner_product_results", inner_product_results},
                                                          {"batch_memory", batch_memory},
                                                          {"net_stream", net_stream},
-                                                         {"net_memory", net_memory}};
+                                                         {"net_memory", net_memory},
+                                                         {"table_copies", table_copies}};
     const auto s = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
     if (s == scenarios.end()) {
         std::printf("unknown scenario\n");

@@ -23,7 +23,8 @@ def host_paths(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["adjoint_memory", "inner_product_results", "batch_memory", "net_stream", "net_memory"])
+@pytest.mark.parametrize("scenario", ["adjoint_memory", "inner_product_results", "batch_memory", "net_stream",
+                                      "net_memory", "table_copies"])
 def test_host_path(host_paths, scenario):
     r = subprocess.run([host_paths, scenario], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout[-3000:]
