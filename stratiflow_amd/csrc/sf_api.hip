@@ -93,9 +93,9 @@ struct Ctx {
     std::vector<void*> allocs;
 
     // Coefficients, wavenumbers and twiddles lie in one allocation, which starts
-    // at zc, with an image of it on the host, so that a change is one copy.
-    std::vector<T> table;
-    size_t level_values = 0;  // zc and zl together
+    // at zc, with an image of it in pinned memory, so that a change is one copy.
+    T* table = nullptr;
+    size_t table_values = 0, level_values = 0;  // all; zc and zl, which come first
     T* zc = nullptr;
     T* zl = nullptr;  // zc in the order of the modal kernels' lanes (ModalArgs)
     T *kx = nullptr, *ky = nullptr, *kx2 = nullptr, *ky2 = nullptr;
@@ -105,7 +105,7 @@ struct Ctx {
     double* partial = nullptr;
     double* scal = nullptr;
     DotResult* dot_host = nullptr;    // pinned: what the inner products leave for the host
-    double* scal_host = nullptr;      // behind it: what read_scalars fetches
+    double* scal_host = nullptr;      // behind it: what read_scalars fetches, then table
     // number of the last inner-product launch; it starts short of its overflow so
     // that the wrap is met early
     unsigned dot_call = 0xffffff00u;
@@ -198,10 +198,6 @@ struct Ctx {
         SF_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         SF_HIP(hipEventCreate(&ev0));
         SF_HIP(hipEventCreate(&ev1));
-        SF_HIP(hipHostMalloc((void**)&dot_host, sizeof(DotResult) + 16 * sizeof(double), hipHostMallocCoherent));
-        std::memset(dot_host, 0, sizeof(DotResult));
-        scal_host = reinterpret_cast<double*>(dot_host + 1);
-
         make_tables();
         partial = dalloc<double>(DOT_MAX * DOT_BLOCKS);
         scal = dalloc<double>(16);
@@ -262,6 +258,13 @@ struct Ctx {
         level_values = end;
         const size_t k[4] = {place(A1), place(A1), place(A2), place(A2)};
         const size_t w[3] = {place(4 * N1), place(4 * N2), place(3 * N1)};
+        table_values = end;
+        SF_HIP(hipHostMalloc((void**)&dot_host, sizeof(DotResult) + 16 * sizeof(double) + end * sizeof(T),
+                             hipHostMallocCoherent));
+        std::memset(dot_host, 0, sizeof(DotResult));
+        scal_host = reinterpret_cast<double*>(dot_host + 1);
+        table = reinterpret_cast<T*>(scal_host + 16);
+        std::fill(table, table + end, T(0));
         zc = dalloc<T>(end);
         zl = zc + lanes;
         kx = zc + k[0];
@@ -271,7 +274,6 @@ struct Ctx {
         tw1 = reinterpret_cast<V*>(zc + w[0]);
         tw2 = reinterpret_cast<V*>(zc + w[1]);
         twx = reinterpret_cast<V*>(zc + w[2]);
-        table.assign(end, T(0));
         // FFT twiddles, computed in double
         auto tw = [&](void (*fill)(int, double*, double*), int n, int entries, const V* dst) {
             std::vector<double> re(entries), im(entries);
@@ -286,7 +288,7 @@ struct Ctx {
         tw(fft_twiddles, N2, 2 * N2, tw2);
         tw(xt_twiddles, N1, 3 * N1 / 2, twx);
     }
-    T* image(const T* device) { return table.data() + (device - zc); }
+    T* image(const T* device) { return table + (device - zc); }
 
     // rows c0..c1 of zc_host into the image, in both orders
     void put_levels(int c0, int c1) {
@@ -301,7 +303,7 @@ struct Ctx {
     }
     // the first n values of the image to the device
     void upload_table(size_t n) {
-        SF_HIP(hipMemcpyAsync(zc, table.data(), n * sizeof(T), hipMemcpyHostToDevice, stream));
+        SF_HIP(hipMemcpyAsync(zc, table, n * sizeof(T), hipMemcpyHostToDevice, stream));
         SF_HIP(hipStreamSynchronize(stream));
     }
 
@@ -366,7 +368,7 @@ struct Ctx {
             image(ky)[ja] = T(k);
             image(ky2)[ja] = T(-k * k);
         }
-        upload_table(table.size());
+        upload_table(table_values);
     }
 
     // x-direction twiddles for the FFT plan with first radix r1f (0: default)
