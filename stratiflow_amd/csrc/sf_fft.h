@@ -200,14 +200,16 @@ __device__ __forceinline__ void reg_dft(cx<T>* v) {
 // ---- plan ------------------------------------------------------------------
 // R1F = 0: the default first radix (16 where N/16 <= 32, else 8); R1F = 8
 // or 16 asks for that first radix where it gives R2 <= 32 (fft_plan_ok), the
-// default otherwise.
+// default otherwise.  Up to 32 points a line is one DFT of one lane; R1F = 4
+// splits lines of 24 and 32 points into two passes as well.
 template <int N, int R1F>
 constexpr bool fft_plan_ok() {
+    if (R1F == 4) return N == 24 || N == 32;
     return N > 32 && (R1F == 8 || R1F == 16) && N % R1F == 0 && N / R1F <= 32;
 }
 template <int N, int R1F = 0>
 struct FftPlan {
-    static constexpr bool two = N > 32;
+    static constexpr bool two = N > 32 || fft_plan_ok<N, R1F>();
     static constexpr int R1 = !two ? N
                               : fft_plan_ok<N, R1F>() ? R1F
                                                       : ((N % 16 == 0 && N / 16 <= 32) ? 16 : 8);
@@ -428,7 +430,7 @@ template <typename T, int N, int NLMAX, int BS, int SIGN, int ES = 1, bool IL = 
           bool PAIRS = false, typename LP>
 __device__ __forceinline__ void lds_fft_lines(int nl, LP lp, const cx<T>* __restrict__ tw,
                                               const int tid = int(threadIdx.x)) {
-    if constexpr (FftPlan<N>::two) {
+    if constexpr (FftPlan<N, R1F>::two) {
         fft_pass1<T, N, NLMAX, BS, SIGN, ES, IL, R1F>(nl, lp, tid);
         if constexpr (PAIRS && !IL && FftPlan<N, R1F>::R2 % 2 == 0)
             fft_pass2_pairs<T, N, NLMAX, BS, SIGN, ES, R1F>(nl, lp, tw, tid);
