@@ -1122,6 +1122,19 @@ constexpr int y_ldp() {
     return l;
 }
 
+// The pointers of the FR fields from f0 on.  They are read at a block-uniform
+// place, whether the fields exist or not: behind a condition, each load of a
+// pointer from the kernel's arguments waits for the load of the condition.
+template <typename V, int FR>
+struct FieldPair {
+    static_assert(FR <= 2, "one or two fields");
+    V *first, *second;
+    template <int N>
+    __device__ __forceinline__ FieldPair(V* const (&fields)[N], int f0)
+        : first(fields[min(f0, N - 1)]), second(FR == 1 ? nullptr : fields[min(f0 + 1, N - 1)]) {}
+    __device__ __forceinline__ V* operator[](int fl) const { return FR == 1 || fl == 0 ? first : second; }
+};
+
 // inverse: out_f(n2, z, j1) = sum_{j2 active} in_f(ja, z, j1) e^{+2 pi i j2 n2/N2}
 // The loads of the next field are issued before the FFT of the current one.
 template <typename T, int N2, int YJ, int FR>
@@ -1141,16 +1154,16 @@ __global__ __launch_bounds__(BS) void k_yinv(YArgs<T> A) {
     auto lp = [&](int line) { return buf + line * LDP; };
     V g[PG];
     auto issue = [&](int f0) {
+        const FieldPair<const V, FR> in(A.in, f0);
 #pragma unroll
         for (int i = 0; i < PG; ++i) {
             const int idx = int(threadIdx.x) + i * BS;
             const int jj = idx % YJ;
             const int rest = idx / YJ;
             const int ja = rest % A2;
-            const int fl = rest / A2;
-            const int f = f0 + fl;
+            const int fl = FR == 1 ? 0 : rest / A2;
             const int j1 = j10 + jj;
-            g[i] = (idx < FR * A2 * YJ && f < A.nf && j1 < A1) ? A.in[f][sidx(ja, z, j1, N3, A1)] : czero<V>();
+            g[i] = (idx < FR * A2 * YJ && f0 + fl < A.nf && j1 < A1) ? in[fl][sidx(ja, z, j1, N3, A1)] : czero<V>();
         }
     };
     const int step = FR * gridDim.z;  // launch_y_fields
@@ -1162,6 +1175,14 @@ __global__ __launch_bounds__(BS) void k_yinv(YArgs<T> A) {
             const int line = idx / nband;
             buf[line * LDP + h + (idx - line * nband)] = czero<V>();
         }
+        if ((A.iky >> f0) & ((1u << FR) - 1)) {  // block-uniform
+#pragma unroll
+            for (int i = 0; i < PG; ++i) {
+                const int rest = (int(threadIdx.x) + i * BS) / YJ;
+                const int fl = FR == 1 ? 0 : rest / A2;
+                if ((A.iky >> (f0 + fl)) & 1) g[i] = cik(A.ky[rest % A2], g[i]);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < PG; ++i) {
             const int idx = int(threadIdx.x) + i * BS;
@@ -1169,22 +1190,22 @@ __global__ __launch_bounds__(BS) void k_yinv(YArgs<T> A) {
                 const int jj = idx % YJ;
                 const int rest = idx / YJ;
                 const int ja = rest % A2;
-                const int fl = rest / A2;
+                const int fl = FR == 1 ? 0 : rest / A2;
                 const int j2 = (ja < h) ? ja : ja + N2 - 2 * h + 1;
-                buf[(fl * YJ + jj) * LDP + j2] = ((A.iky >> (f0 + fl)) & 1) ? cik(A.ky[ja], g[i]) : g[i];
+                buf[(fl * YJ + jj) * LDP + j2] = g[i];
             }
         }
         sync_lds();
         if (f0 + step < A.nf) issue(f0 + step);
         lds_fft_lines<T, N2, NL, BS, +1>(NL, lp, A.tw);
+        const FieldPair<V, FR> out(A.out, f0);
         for (int idx = threadIdx.x; idx < FR * N2 * YJ; idx += BS) {
             const int jj = idx % YJ;
             const int rest = idx / YJ;
             const int n2 = rest % N2;
-            const int fl = rest / N2;
-            const int f = f0 + fl;
+            const int fl = FR == 1 ? 0 : rest / N2;
             const int j1 = j10 + jj;
-            if (f < A.nf && j1 < A1) A.out[f][sidx(n2, z, j1, N3, A1)] = buf[(fl * YJ + jj) * LDP + n2];
+            if (f0 + fl < A.nf && j1 < A1) out[fl][sidx(n2, z, j1, N3, A1)] = buf[(fl * YJ + jj) * LDP + n2];
         }
         sync_lds();
     }
@@ -1208,16 +1229,16 @@ __global__ __launch_bounds__(BS) void k_yfwd(YArgs<T> A) {
     auto lp = [&](int line) { return buf + line * LDP; };
     V g[PG];
     auto issue = [&](int f0) {
+        const FieldPair<const V, FR> in(A.in, f0);
 #pragma unroll
         for (int i = 0; i < PG; ++i) {
             const int idx = int(threadIdx.x) + i * BS;
             const int jj = idx % YJ;
             const int rest = idx / YJ;
             const int n2 = rest % N2;
-            const int fl = rest / N2;
-            const int f = f0 + fl;
+            const int fl = FR == 1 ? 0 : rest / N2;
             const int j1 = j10 + jj;
-            g[i] = (idx < FR * N2 * YJ && f < nin && j1 < A1) ? A.in[f][sidx(n2, z, j1, N3, A1)] : czero<V>();
+            g[i] = (idx < FR * N2 * YJ && f0 + fl < nin && j1 < A1) ? in[fl][sidx(n2, z, j1, N3, A1)] : czero<V>();
         }
     };
     const int step = FR * gridDim.z;  // launch_y_fields
@@ -1230,7 +1251,7 @@ __global__ __launch_bounds__(BS) void k_yfwd(YArgs<T> A) {
                 const int jj = idx % YJ;
                 const int rest = idx / YJ;
                 const int n2 = rest % N2;
-                const int fl = rest / N2;
+                const int fl = FR == 1 ? 0 : rest / N2;
                 buf[(fl * YJ + jj) * LDP + n2] = g[i];
             }
         }
@@ -1242,7 +1263,7 @@ __global__ __launch_bounds__(BS) void k_yfwd(YArgs<T> A) {
                 const int jj = idx % YJ;
                 const int rest = idx / YJ;
                 const int ja = rest % A2;
-                const int pr = rest / A2;
+                const int pr = FR <= 2 ? 0 : rest / A2;
                 const int r = f0 / 2 + pr;
                 const int j1 = j10 + jj;
                 if (r >= A.nf || j1 >= A1) continue;
@@ -1252,16 +1273,16 @@ __global__ __launch_bounds__(BS) void k_yfwd(YArgs<T> A) {
                 A.out[r][sidx(ja, z, j1, N3, A1)] = cscale(A.scale, cadd(Fa, cik(A.ky[ja], Fb)));
             }
         } else {
+            const FieldPair<V, FR> out(A.out, f0);
             for (int idx = threadIdx.x; idx < FR * A2 * YJ; idx += BS) {
                 const int jj = idx % YJ;
                 const int rest = idx / YJ;
                 const int ja = rest % A2;
-                const int fl = rest / A2;
-                const int f = f0 + fl;
+                const int fl = FR == 1 ? 0 : rest / A2;
                 const int j1 = j10 + jj;
-                if (f >= nin || j1 >= A1) continue;
+                if (f0 + fl >= nin || j1 >= A1) continue;
                 const int j2 = (ja < h) ? ja : ja + N2 - 2 * h + 1;
-                A.out[f][sidx(ja, z, j1, N3, A1)] = cscale(A.scale, buf[(fl * YJ + jj) * LDP + j2]);
+                out[fl][sidx(ja, z, j1, N3, A1)] = cscale(A.scale, buf[(fl * YJ + jj) * LDP + j2]);
             }
         }
         sync_lds();
