@@ -588,6 +588,7 @@ struct Ctx {
         m.A2 = A2;
         m.nmodes = A1 * A2;
         m.threeD = three ? 1 : 0;
+        m.zc = zc;
         m.zl = zl;
         m.kx = kx;
         m.ky = ky;

@@ -9,9 +9,10 @@ namespace sf {
 template <typename T>
 struct ModalArgs {
     int N3, N3p, A1, A2, nmodes, threeD;
-    // the coefficient table in the order of the columns' lanes: row c of level
-    // lane*M + t at (c*M + t)*64 + lane, M = rows per lane (zero beyond N3)
-    const T* zl;
+    // the coefficient table by level, [ZC_COUNT][N3p], and in the order of the
+    // columns' lanes: row c of level lane*M + t at (c*M + t)*64 + lane, M = rows per
+    // lane (zero beyond N3)
+    const T *zc, *zl;
     const T *kx, *ky, *kx2, *ky2;
     cx<T> *u1, *u2, *u3, *b, *p;
     const cx<T> *ro1, *ro2, *ro3, *roB;  // explicit terms of the previous stage (null: not read)

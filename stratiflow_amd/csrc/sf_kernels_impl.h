@@ -44,6 +44,17 @@ constexpr int modal_mb() {
     return (std::is_same<T, float>::value ? M <= 6 : M <= 3) ? 8 : 4;
 }
 
+// Which order of the coefficient table a tile's waves read.  In the order of the
+// lanes a load is one contiguous run of 4 bytes per lane; by level, a lane's M rows
+// are neighbours, which the compiler reads in loads of up to 16 bytes.  FP32 gains
+// from the first (us per launch by level / by lane: 384x192x384 357 / 332, 192x96x512
+// 216 / 163) but for M = 7 (192x96x448: stage equal, projection 36.4 / 39.0), FP64 from
+// the second (192x96x384 186 / 198, 64x32x320 39.8 / 44.1, 192x96x100 57.4 / 58.1).
+template <typename T, int M>
+constexpr bool modal_by_lane() {
+    return std::is_same<T, float>::value && M != 7;
+}
+
 // One block owns MB modes (ja, j10 .. j10+MB-1), one wavefront each.  Every
 // field access goes through an LDS tile of N3 rows x MB modes so that global
 // memory sees runs of MB consecutive j1 ([ja][z][j1] layout); wave w then
@@ -52,7 +63,7 @@ constexpr int modal_mb() {
 // FULL (N3 == 64*M): every tile row exists, so a thread keeps one base offset
 // per table and reaches its row t through the scalar offset (fewer live
 // registers than an offset per row).
-template <typename T, int M, int MB, bool FULL = false>
+template <typename T, int M, int MB, bool FULL = false, bool BY_LANE = modal_by_lane<T, M>()>
 __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, const int j10, cx<T>* const tile) {
     using V = cx<T>;
     constexpr int TP = MB + 1;  // tile row pitch (tile: 64*M*TP values of LDS)
@@ -72,12 +83,23 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
     int row[M];
 #pragma unroll
     for (int t = 0; t < M; ++t) row[t] = lane * M + t;
-    // a wave reads a coefficient of its rows as one contiguous run; gathered from
-    // the table by level (a stride of M rows per lane) each load took a dozen cache
-    // lines (per launch: 357 -> 332 us at 384x192x384 FP32, 216 -> 163 us at
-    // 192x96x512 FP32)
-    const rsrc_t zr = make_rsrc(A.zl, size_t(ZC_COUNT) * M * 64 * sizeof(T));
-    auto coefz = [&](int c, int t) -> T { return bld<T>(zr, lane * int(sizeof(T)), (c * M + t) * 64 * int(sizeof(T))); };
+    // row c of the coefficients at the lane's row t; rows at or beyond N3 read zero
+    const rsrc_t zr = BY_LANE ? make_rsrc(A.zl, size_t(ZC_COUNT) * M * 64 * sizeof(T))
+                              : make_rsrc(A.zc, size_t(ZC_COUNT) * A.N3p * sizeof(T));
+    int zoff[BY_LANE || FULL ? 1 : M];
+    if constexpr (BY_LANE) {
+        zoff[0] = lane * int(sizeof(T));
+    } else if constexpr (FULL) {
+        zoff[0] = lane * M * int(sizeof(T));
+    } else {
+#pragma unroll
+        for (int t = 0; t < M; ++t) zoff[t] = row[t] < N ? row[t] * int(sizeof(T)) : BUF_OOB;
+    }
+    auto coefz = [&](int c, int t) -> T {
+        if constexpr (BY_LANE) return bld<T>(zr, zoff[0], (c * M + t) * 64 * int(sizeof(T)));
+        else if constexpr (FULL) return bld<T>(zr, zoff[0], (c * A.N3p + t) * int(sizeof(T)));
+        else return bld<T>(zr, zoff[t], c * A.N3p * int(sizeof(T)));
+    };
     auto dzzn = [&](int i, int t) -> T { return coefz(ZC_DZZN_LO + i, t); };
     auto dzzd = [&](int i, int t) -> T { return coefz(ZC_DZZD_LO + i, t); };
     // tile element owned by this thread in the cooperative (coalesced) phase:
@@ -393,7 +415,7 @@ __global__ __launch_bounds__(MB * 64) void k_modal_mixed(const ModalArgs<T>* __r
         switch ((a.N3 + 63) / 64) {
 #define SF_M(m)                                                       \
     case m:                                                           \
-        if constexpr (m <= MMAX) modal_body<T, m, MB>(a, ja, j10, tile); \
+        if constexpr (m <= MMAX) modal_body<T, m, MB, false, MB == 8 && modal_by_lane<T, m>()>(a, ja, j10, tile); \
         break;
             SF_M(1) SF_M(2) SF_M(3) SF_M(4) SF_M(5) SF_M(6) SF_M(7) SF_M(8)
 #undef SF_M
