@@ -116,7 +116,8 @@ hipError_t launch_modal(const ModalArgs<T>& a, hipStream_t s);
 // the same for grids of few modes (sf_modal_cols.hip): one block per mode
 template <typename T>
 hipError_t launch_modal_cols(const ModalArgs<T>& a, hipStream_t s);
-bool modal_cols_fit(int A1, int A2, int N3, int value_bytes);  // whether it is the faster one
+// whether it is the faster one, for a stage (step) or the projection alone
+bool modal_cols_fit(int A1, int A2, int N3, int value_bytes, bool step);
 template <typename T>
 hipError_t launch_xpass(const XArgs<T>& a, int N1, int N2, bool threeD, hipStream_t s);
 template <typename T>

@@ -489,7 +489,7 @@ static void launch_modal_mb(const ModalArgs<T>& a, hipStream_t s) {
 
 template <typename T>
 hipError_t launch_modal(const ModalArgs<T>& a, hipStream_t s) {
-    if (modal_cols_fit(a.A1, a.A2, a.N3, int(sizeof(cx<T>)))) return launch_modal_cols<T>(a, s);
+    if (modal_cols_fit(a.A1, a.A2, a.N3, int(sizeof(cx<T>)), a.mode == 0)) return launch_modal_cols<T>(a, s);
     const int M = (a.N3 + 63) / 64;
     switch (M) {
 #define SF_M(m)                                        \

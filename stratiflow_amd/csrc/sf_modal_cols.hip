@@ -20,7 +20,14 @@ namespace {
 // wave of each column
 enum ColWave { CW_U1 = 0, CW_U3, CW_B, CW_P, CW_U2 };
 
-template <typename T, int M>
+// PROJECT: the projection alone, in a kernel of its own for FP64: with the registers
+// of a stage, columns of more than 320 levels spill up to 182 of them (projection
+// of 256x1x512: 19.8 us in the stage's kernel, 12.7 in its own; 256x1x384: 12.8 and
+// 10.5).  In FP32 the kernel of its own is no faster, its registers are those of the
+// (0,0) mode's FP64 solve (96x32x100: 6.1 us in the stage's kernel, 7.4 in its own).
+// A stage asks the mode at run time: fixed at compile time its allocation spills
+// more at 384 levels (256x1x384 FP64: 21.1 -> 24.5 us).
+template <typename T, int M, bool PROJECT>
 __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int ja, const int j1,
                                                 cx<T> (*const col)[M][64]) {
     using V = cx<T>;
@@ -42,7 +49,8 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
         case CW_B: x_ = A.b, n_ = A.nB, ro_ = A.roB, rn_ = A.rnB; break;
         default: x_ = A.p, n_ = nullptr, ro_ = nullptr, rn_ = nullptr; break;
     }
-    const bool step = A.mode == 0;
+
+    const bool step = !PROJECT && A.mode == 0;
 
     int row[M], foff[M];
 #pragma unroll
@@ -275,37 +283,61 @@ __device__ __forceinline__ void modal_cols_body(const ModalArgs<T>& A, const int
 }  // namespace
 
 // threads: four waves in 2D, five in 3D
-template <typename T, int M>
+template <typename T, int M, bool PROJECT>
 __global__ __launch_bounds__(320) void k_modal_cols(ModalArgs<T> A) {
     __shared__ cx<T> col[5][M][64];
     // modes of one cache line on one XCD
     const int m = xcd_tile(blockIdx.x, gridDim.x);
-    modal_cols_body<T, M>(A, m / A.A1, m % A.A1, col);
+    modal_cols_body<T, M, PROJECT>(A, m / A.A1, m % A.A1, col);
 }
 
-// Up to 256 modes, or 1024 where a field is at most 1.5 MB: four or five waves
-// per mode then fill the GPU in one round, and the columns, which are read a
-// cache line per row, stay cheap.  Against tiles of eight modes (us per stage by
-// events, tiles / columns):
-//   256x1x256 FP64 (85 modes) 28.1 / 15.7      64x32x512 FP32 (399, 1.6 MB) 59.1 / 55.1
-//   512x1x512 FP32 (170) 48.6 / 24.2           64x32x256 FP64 (399, 1.6 MB) 34.4 / 38.9
-//   96x32x256 FP32 (608, 1.2 MB) 35.0 / 25.5   96x48x192 FP32 (992, 1.5 MB) 27.0 / 28.9
-//   96x48x100 FP32 (992, 0.8 MB) 21.7 / 16.2   128x48x100 FP32 (1302, 1.0 MB) 24.4 / 31.7
-// and one wave per mode for all fields, one mode per block: 21.4 us at 256x1x256
-// FP64 and 8.3 us at 64x1x64 FP32, where these waves take 13.1 and 5.9 us (by
-// kernel trace).
-bool modal_cols_fit(int A1, int A2, int N3, int value_bytes) {
+// Up to one mode per CU the columns are the faster kernel by far (us per stage by
+// events, tiles of eight modes / columns: 256x1x256 FP64, 85 modes, 28.5 / 15.4;
+// 512x1x512 FP32, 170 modes, 35.8 / 21.0; one wave per mode for all fields took
+// 21.4 us at 256x1x256 FP64 where these take 13.1 by kernel trace).  With more modes a
+// CU runs two, three or four blocks at once, which compete for its LDS and
+// registers the more the longer the columns are, and tiles read whole cache lines
+// where columns read a value of a line each.  Rows of whole groups of eight modes
+// keep the modes of a line on one XCD (xcd_tile needs their number to divide by
+// eight), ragged rows do not and reach the crossover earlier; of rows of two
+// modes a tile uses only two of its eight places.  Stage, tiles / columns:
+//   2 modes per CU, whole              48x48x512 FP32 45.1 / 34.1   48x48x384 FP64 47.0 / 40.3, x512 77.2 / 82.3
+//              2, ragged              64x32x256 FP32 31.9 / 23.8, x384 36.9 / 39.0    x192 FP64 37.8 / 32.8, x256 36.0 / 38.7
+//              3, whole               96x32x256 FP32 30.3 / 23.3, x384 35.9 / 37.7    x192 FP64 35.9 / 29.9, x256 33.0 / 34.7
+//              3, ragged              64x48x128 FP32 23.0 / 20.8, x192 26.4 / 32.1    x100 FP64 30.7 / 28.2, x128 31.8 / 33.1
+//              4, whole               96x48x128 FP32 22.5 / 17.4, x192 25.9 / 27.3    x128 FP64 30.5 / 28.7, x192 37.5 / 39.5
+//              4, ragged              64x64x100 FP32 23.4 / 22.0, x128 23.6 / 26.7    x64 FP64 25.7 / 22.0, x100 31.6 / 37.9
+// (128x48x64, 1302 modes: FP32 19.9 / 21.4, FP64 26.7 / 30.1.)  The projection alone has
+// one solve to spread over the waves and crosses over at shorter columns: whole
+// 48x48x256 FP32 10.5 / 8.9, x384 12.7 / 14.4, x192 FP64 9.9 / 8.5, x384 15.5 / 17.3;
+// 96x48x192 FP32 9.8 / 14.5, x100 FP64 8.7 / 10.2; ragged 64x48x100 FP32 8.4 / 10.2.
+bool modal_cols_fit(int A1, int A2, int N3, int value_bytes, bool step) {
+    // levels up to which the columns are taken, by modes per CU (2, 3, 4)
+    static const int levels[2][2][2][3] = {
+        {{{0, 0, 0}, {0, 0, 0}}, {{256, 100, 48}, {192, 128, 64}}},              // projection: ragged, whole; FP32, FP64
+        {{{256, 128, 100}, {192, 100, 64}}, {{512, 256, 128}, {384, 192, 128}}}  // step
+    };
     const long modes = long(A1) * A2;
-    return modes <= 256 || (modes <= 1024 && modes * N3 * value_bytes <= 1536 * 1000L);
+    if (modes <= 256) return true;
+    if (modes > 1024) return false;
+    const bool whole = A1 % 8 == 0 || A1 < 4;
+    const int per_cu = A1 < 4 ? 2 : int((modes + 255) / 256);
+    return N3 <= levels[step][whole][value_bytes == 16][per_cu - 2];
 }
 
 template <typename T>
 hipError_t launch_modal_cols(const ModalArgs<T>& a, hipStream_t s) {
     const dim3 grid(a.A1 * a.A2), block(a.threeD ? 320 : 256);
     switch ((a.N3 + 63) / 64) {
-#define SF_M(m)                                                            \
-    case m:                                                                \
-        hipLaunchKernelGGL((k_modal_cols<T, m>), grid, block, 0, s, a);    \
+#define SF_M(m)                                                                        \
+    case m:                                                                            \
+        if constexpr (std::is_same<T, double>::value) {                                \
+            if (a.mode != 0) {                                                         \
+                hipLaunchKernelGGL((k_modal_cols<T, m, true>), grid, block, 0, s, a);  \
+                break;                                                                 \
+            }                                                                          \
+        }                                                                              \
+        hipLaunchKernelGGL((k_modal_cols<T, m, false>), grid, block, 0, s, a);         \
         break;
         SF_M(1) SF_M(2) SF_M(3) SF_M(4) SF_M(5) SF_M(6) SF_M(7) SF_M(8)
 #undef SF_M
