@@ -212,3 +212,29 @@ def test_many_inner_products(shape):
     for i in range(300):
         assert s.energies() + (s.InnerProd(u, b),) == first, i
     s.close()
+
+
+@pytest.mark.parametrize("shape,prec", [((48, 1, 36, 1), 4), ((64, 1, 68, 1), 8), ((48, 12, 20, 0), 8), ((64, 6, 16, 0), 8),
+                                        ((32, 16, 48, 0), 8), ((64, 12, 64, 0), 4)])
+def test_transforms_of_short_lines(shape, prec):
+    """Lines of 24 and 32 points (N1 = 48, 64) in two passes, with blocks that fill
+    or do not fill their levels, and FP64 blocks of whole lines in their own
+    order: a random nodal field against numpy, there and back."""
+    s = solver(shape, prec)
+    N1, N2, N3, dim = shape
+    n, m, back = s.field(sf.NODAL, sf.NEUMANN), s.field(sf.MODAL, sf.NEUMANN), s.field(sf.NODAL, sf.NEUMANN)
+    n.upload(np.random.default_rng(8).standard_normal(n.shape))
+    v = n.download()
+    n.ToModal(m)
+    m.ToNodal(back)
+    want = np.fft.rfft2(v, axes=(0, 1)) / (N1 * N2)
+    want[:, N1 // 3:] = 0
+    if dim == 0:
+        want[N2 // 3:N2 - N2 // 3 + 1] = 0
+    tol = 8 * np.finfo(np.float32 if prec == 4 else np.float64).eps * np.log2(N1 * N2)
+    e = np.linalg.norm(m.download() - want) / np.linalg.norm(want)
+    back_want = np.fft.irfft2(want, s=(N2, N1), axes=(0, 1)) * (N1 * N2)
+    b = np.linalg.norm(back.download() - back_want) / np.linalg.norm(back_want)
+    print(shape, prec, "%.2e %.2e" % (e / tol, b / tol), flush=True)
+    assert e < tol and b < 2 * tol
+    s.close()
