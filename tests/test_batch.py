@@ -165,3 +165,27 @@ def test_items_of_many_runs_fp64(runs):
         for f in ("u1", "u3", "b", "p"):
             assert np.array_equal(s.get(f), t.get(f)), (i, f)
     b.close()
+
+
+@pytest.mark.parametrize("runs,odd,tiles", [(15, 0, 60), (16, 0, 64), (16, 1, 65), (31, 0, 124), (32, 0, 128), (32, 1, 129),
+                                            (33, 0, 132)])
+def test_whole_windows_of_items_fp64(runs, odd, tiles):
+    """Every whole 64 work items are put in another order: stage launches of just
+    under one window, of one and two whole ones, and of one tile more, bit for
+    bit.  A run of N1 = 48 has 16 modes, four tiles of four; one of N1 = 12 has
+    four, one tile."""
+    import stratiflow_amd as sf
+    sizes = [(48, 32 + 4 * (i % 8), 500.0 + 100 * i, 0.1, 0.01) for i in range(runs)]
+    sizes += [(12, 36, 700.0, 0.1, 0.01)] * odd
+    assert sum(-(-(n[0] // 3) // 4) for n in sizes) == tiles
+    batched = [_make(*r, seed=500 + i, prec=8) for i, r in enumerate(sizes)]
+    twins = [_make(*r, seed=500 + i, prec=8) for i, r in enumerate(sizes)]
+    b = sf.Batch(batched)
+    b.select(sf.BATCH_MIXED, sf.BATCH_MIXED)
+    b.step(2)
+    for t in twins:
+        t.TimeStep(2)
+    for i, (s, t) in enumerate(zip(batched, twins)):
+        for f in ("u1", "u3", "b", "p"):
+            assert np.array_equal(s.get(f), t.get(f)), (i, f)
+    b.close()
