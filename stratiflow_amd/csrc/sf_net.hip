@@ -556,9 +556,9 @@ struct Net {
     float* tgt = nullptr;
     float* part = nullptr;
     size_t part_n = 0;
-    double* dpart = nullptr;
-    unsigned* ticket = nullptr;  // of k_rms's blocks
-    double* scale = nullptr;     // its results, for two inputs
+    double* dpart = nullptr;  // partial sums; in the same allocation:
+    double* scale = nullptr;     // k_rms's results, for two inputs
+    unsigned* ticket = nullptr;  // of its blocks
     int* didx = nullptr;
     int didx_n = 0;
     static constexpr int DW_BLOCKS = 240;
@@ -578,8 +578,6 @@ struct Net {
         F(set_t);
         free_work();
         F(dpart);
-        F(ticket);
-        F(scale);
         F(didx);
     }
     void free_work() {
@@ -671,9 +669,9 @@ struct Net {
             Wb.push_back(dalloc<bf16>(size_t(KT) * C[l + 1] * C[l]));
             Wt.push_back(dalloc<bf16>(size_t(KT) * C[l + 1] * C[l]));
         }
-        dpart = dalloc<double>(4096);
-        ticket = dalloc<unsigned>(1);
-        scale = dalloc<double>(4);
+        dpart = dalloc<double>(4096);  // partial sums of at most 1024 blocks
+        scale = dpart + 4088;
+        ticket = reinterpret_cast<unsigned*>(dpart + 4095);
         cast_weights();
         SF_HIP(hipStreamSynchronize(st()));
     }

@@ -258,9 +258,12 @@ static void net_stream() {
     sf_field* f[4];
     for (int i = 0; i < 4; ++i) sf_field_alloc(c, SF_MODAL, i == 2 ? SF_DIRICHLET : SF_NEUMANN, &f[i]);
     null_stream_ops = 0;
+    const size_t before = live.size();
     sf_net* n = nullptr;
     EXPECT(sf_net_create(c, 32, 3, 1, &n) == SF_OK, "%s", sf_net_last_error(nullptr));
     if (!n) std::exit(1);
+    // parameters, gradient, two moments and mask, two layouts of three layers, partial sums
+    EXPECT(live.size() - before == 12, "%zu buffers", live.size() - before);
     auto expect = [&](const char* call) {
         EXPECT(null_stream_ops == 0, "%s: %d outside the stream", call, null_stream_ops);
         null_stream_ops = 0;
