@@ -586,7 +586,6 @@ struct Ctx {
         m.N3p = N3p;
         m.A1 = A1;
         m.A2 = A2;
-        m.nmodes = A1 * A2;
         m.threeD = three ? 1 : 0;
         m.zc = zc;
         m.zl = zl;

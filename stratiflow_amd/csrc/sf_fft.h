@@ -442,13 +442,6 @@ __device__ __forceinline__ void lds_fft_lines(int nl, LP lp, const cx<T>* __rest
     }
 }
 
-// NL contiguous lines at stride fft_ldp<N>()
-template <typename T, int N, int NL, int BS, int SIGN>
-__device__ __forceinline__ void lds_fft(cx<T>* buf, const cx<T>* __restrict__ tw, const int tid = int(threadIdx.x)) {
-    constexpr int LDP = fft_ldp<N>();
-    lds_fft_lines<T, N, NL, BS, SIGN>(NL, [buf](int line) { return buf + line * LDP; }, tw, tid);
-}
-
 // host: twiddle table of 2N entries for the plan FftPlan<N, R1F>: the layout
 // fft_pass2 reads, then the same values in the order fft_pass2_pairs reads
 template <int N, int R1F = 0>

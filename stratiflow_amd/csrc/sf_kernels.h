@@ -8,7 +8,7 @@ namespace sf {
 // Fused per-mode stage kernel (one wavefront per Fourier mode).
 template <typename T>
 struct ModalArgs {
-    int N3, N3p, A1, A2, nmodes, threeD;
+    int N3, N3p, A1, A2, threeD;
     // the coefficient table by level, [ZC_COUNT][N3p], and in the order of the
     // columns' lanes: row c of level lane*M + t at (c*M + t)*64 + lane, M = rows per
     // lane (zero beyond N3)

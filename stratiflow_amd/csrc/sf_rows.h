@@ -6,11 +6,11 @@
 
 namespace sf {
 
-// the rows before and after each row of the lane (V complex or one part)
+// the rows before and after each row of the lane
 template <int M, typename V>
 __device__ __forceinline__ void nb_prev(const V (&x)[M], V (&xm)[M], int lane) {
     V s = shfl_idx(x[M - 1], (lane - 1) & 63);
-    if (lane == 0) set_zero(s);
+    if (lane == 0) s = czero<V>();
     xm[0] = s;
 #pragma unroll
     for (int t = 1; t < M; ++t) xm[t] = x[t - 1];
@@ -18,7 +18,7 @@ __device__ __forceinline__ void nb_prev(const V (&x)[M], V (&xm)[M], int lane) {
 template <int M, typename V>
 __device__ __forceinline__ void nb_next(const V (&x)[M], V (&xp)[M], int lane) {
     V s = shfl_idx(x[0], (lane + 1) & 63);
-    if (lane == 63) set_zero(s);
+    if (lane == 63) s = czero<V>();
 #pragma unroll
     for (int t = 0; t < M - 1; ++t) xp[t] = x[t + 1];
     xp[M - 1] = s;

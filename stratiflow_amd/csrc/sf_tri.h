@@ -43,15 +43,6 @@ __device__ __forceinline__ cx<T> tmadc(T a, cx<T> v, cx<T> c) {  // a*v + c
     return mkc<T>(tmad(a, v.x, c.x), tmad(a, v.y, c.y));
 }
 
-template <typename T>
-__device__ __forceinline__ T tscale(T a, T v) {
-    return tmul(a, v);
-}
-template <typename T>
-__device__ __forceinline__ T tmadc(T a, T v, T c) {
-    return tmad(a, v, c);
-}
-
 __device__ __forceinline__ float shfl_idx(float v, int src) { return __shfl(v, src, 64); }
 __device__ __forceinline__ double shfl_idx(double v, int src) { return __shfl(v, src, 64); }
 template <typename V>
@@ -60,12 +51,6 @@ __device__ __forceinline__ V shfl_idx(V v, int src) {
     r.x = __shfl(v.x, src, 64);
     r.y = __shfl(v.y, src, 64);
     return r;
-}
-__device__ __forceinline__ void set_zero(float& v) { v = 0; }
-__device__ __forceinline__ void set_zero(double& v) { v = 0; }
-template <typename V>
-__device__ __forceinline__ void set_zero(V& v) {
-    v = czero<V>();
 }
 
 template <typename T, int M>
@@ -165,11 +150,12 @@ __device__ __forceinline__ void tri_factor(TriFactor<T, M>& F, const T (&a)[M], 
 }
 
 // Solve in place: d holds the lane's M right-hand-side rows on entry and the
-// solution on exit.  D is complex, or T for one part of it.
-template <typename T, int M, typename D>
-__device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, D (&d)[M], int lane) {
-    D Ds;
-    D g[M];
+// solution on exit.
+template <typename T, int M>
+__device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, cx<T> (&d)[M], int lane) {
+    using V = cx<T>;
+    V Ds;
+    V g[M];
     if constexpr (M == 1) {
         Ds = d[0];
     } else {
@@ -179,24 +165,24 @@ __device__ __forceinline__ void tri_apply(const TriFactor<T, M>& F, D (&d)[M], i
         for (int t = 1; t <= M - 2; ++t) g[t] = tscale(F.rden[t], tmadc(-F.a[t], g[t - 1], d[t]));
 #pragma unroll
         for (int t = M - 3; t >= 0; --t) g[t] = tmadc(-F.cc[t], g[t + 1], g[t]);
-        D gn0 = shfl_idx(g[0], (lane + 1) & 63);
-        if (lane == 63) set_zero(gn0);
+        V gn0 = shfl_idx(g[0], (lane + 1) & 63);
+        if (lane == 63) gn0 = czero<V>();
         Ds = tmadc(-F.cI, gn0, tmadc(-F.aI, g[M - 2], d[M - 1]));
     }
 #pragma unroll
     for (int lev = 0; lev < 6; ++lev) {
         const int s = 1 << lev;
-        D Dm = shfl_idx(Ds, (lane - s) & 63), Dp = shfl_idx(Ds, (lane + s) & 63);
-        if (lane - s < 0) set_zero(Dm);
-        if (lane + s > 63) set_zero(Dp);
+        V Dm = shfl_idx(Ds, (lane - s) & 63), Dp = shfl_idx(Ds, (lane + s) & 63);
+        if (lane - s < 0) Dm = czero<V>();
+        if (lane + s > 63) Dp = czero<V>();
         Ds = tmadc(F.gamma[lev], Dp, tmadc(F.alpha[lev], Dm, Ds));
     }
-    const D sl = tscale(F.rB, Ds);
+    const V sl = tscale(F.rB, Ds);
     if constexpr (M == 1) {
         d[0] = sl;
     } else {
-        D sm = shfl_idx(sl, (lane - 1) & 63);
-        if (lane == 0) set_zero(sm);
+        V sm = shfl_idx(sl, (lane - 1) & 63);
+        if (lane == 0) sm = czero<V>();
 #pragma unroll
         for (int t = 0; t <= M - 2; ++t) d[t] = tmadc(-F.w[t], sl, tmadc(-F.v[t], sm, g[t]));
         d[M - 1] = sl;
