@@ -375,12 +375,12 @@ __device__ __forceinline__ void modal_body(const ModalArgs<T>& A, const int ja, 
     store(A.p, pp);
 }
 
-template <typename T, int M, bool FULL, int MB>
+template <typename T, int M, bool FULL, int MB, bool BY_LANE>
 __global__ __launch_bounds__(MB * 64) void k_modal(ModalArgs<T> A) {
     __shared__ cx<T> tile[64 * M * (MB + 1)];
     const int nt = gridDim.x;  // j1 tiles per ja
     const int t = xcd_tile(blockIdx.x + nt * blockIdx.y, nt * gridDim.y);
-    modal_body<T, M, MB, FULL>(A, t / nt, (t % nt) * MB, tile);
+    modal_body<T, M, MB, FULL, BY_LANE>(A, t / nt, (t % nt) * MB, tile);
 }
 
 // Many independent runs in one launch: a grid-stride (persistent) loop over
@@ -480,11 +480,22 @@ hipError_t launch_modal_batch(const ModalArgs<T>* args, const int2* items, int t
     return hipGetLastError();
 }
 
-template <typename T, int M, int MB>
+template <typename T, int M, int MB, bool BY_LANE>
 static void launch_modal_mb(const ModalArgs<T>& a, hipStream_t s) {
     const dim3 grid((a.A1 + MB - 1) / MB, a.A2);
-    if (a.N3 == 64 * M) hipLaunchKernelGGL((k_modal<T, M, true, MB>), grid, dim3(MB * 64), 0, s, a);
-    else hipLaunchKernelGGL((k_modal<T, M, false, MB>), grid, dim3(MB * 64), 0, s, a);
+    if (a.N3 == 64 * M) hipLaunchKernelGGL((k_modal<T, M, true, MB, BY_LANE>), grid, dim3(MB * 64), 0, s, a);
+    else hipLaunchKernelGGL((k_modal<T, M, false, MB, BY_LANE>), grid, dim3(MB * 64), 0, s, a);
+}
+// the projection alone of five and six rows per lane reads by level in FP32 too
+// (384x192x384 93.5 us by level, 99.3 by lane; x320 79.9, 85.5; up to four rows and
+// with eight it is by lane that is faster or equal: x512 219.6, 202.3)
+template <typename T, int M>
+static void launch_modal_m(const ModalArgs<T>& a, hipStream_t s) {
+    constexpr int MB = modal_mb<T, M>();
+    if constexpr (modal_by_lane<T, M>() && (M == 5 || M == 6)) {
+        if (a.mode != 0) return launch_modal_mb<T, M, MB, false>(a, s);
+    }
+    launch_modal_mb<T, M, MB, modal_by_lane<T, M>()>(a, s);
 }
 
 template <typename T>
@@ -494,7 +505,7 @@ hipError_t launch_modal(const ModalArgs<T>& a, hipStream_t s) {
     switch (M) {
 #define SF_M(m)                                        \
     case m:                                            \
-        launch_modal_mb<T, m, modal_mb<T, m>()>(a, s); \
+        launch_modal_m<T, m>(a, s);                    \
         break;
         SF_M(1) SF_M(2) SF_M(3) SF_M(4) SF_M(5) SF_M(6) SF_M(7) SF_M(8)
 #undef SF_M

@@ -61,3 +61,23 @@ def test_both_sides_of_the_lines(shape):
         print(shape, f, "%.2e" % e, flush=True)
         assert e < (1e-9 if f == "p" else 1e-11), f
     s.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N3", [260, 320, 324, 384])
+def test_projection_of_long_columns_fp32(N3):
+    """Tiles of five and six rows per lane, whole and ragged, read their
+    coefficients by level in the projection and by lane in a stage: FP32 within
+    three times the FP32 oracle's own error."""
+    from helpers import fields, make_pair, rel_l2
+    shape = (96, 64, N3, 0)
+    s, o64 = make_pair(*shape, gpu_prec=4, amplitude=0.05, seed=12, project=False)
+    _, o32 = make_pair(*shape, gpu_prec=4, oracle_prec=4, amplitude=0.05, seed=12, project=False)
+    s.RemoveDivergence(0.5)
+    o64.remove_divergence(0.5)
+    o32.remove_divergence(0.5)
+    for f in fields(shape[3]):
+        eg, er = rel_l2(s.get(f), o64.get_modal(f)), rel_l2(o32.get_modal(f), o64.get_modal(f))
+        print(shape, f, "%.2e %.2e" % (eg, er), flush=True)
+        assert eg <= max(3 * er, 1e-6), f
+    s.close()
