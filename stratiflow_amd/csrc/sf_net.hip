@@ -244,24 +244,39 @@ __global__ __launch_bounds__(NB) void k_wcast(const float* __restrict__ w, int C
     Wt[(size_t(KT - 1 - t) * Cin + ci) * Cout + co] = x;
 }
 
+__device__ __forceinline__ void block_sum(double (&red)[NB], double s) {
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int k = NB / 2; k > 0; k >>= 1) {
+        if (int(threadIdx.x) < k) red[threadIdx.x] += red[threadIdx.x + k];
+        __syncthreads();
+    }
+}
+// s = RMS and 1/s (0 for a zero field) into scale[0..1] from the blocks' sums, added
+// in block order by the NB threads of one block
+__device__ __forceinline__ void rms_total(double (&red)[NB], const double* part, unsigned blocks, double count,
+                                          double* scale) {
+    double s = 0;
+    for (unsigned b = threadIdx.x; b < blocks; b += NB)
+        s += __hip_atomic_load(part + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    block_sum(red, s);
+    if (threadIdx.x == 0) {
+        const double rms = sqrt(red[0] / count);
+        scale[0] = rms;
+        scale[1] = rms > 0 ? 1.0 / rms : 0.0;
+    }
+}
+
 // RMS of up to 4 complex fields over the active modes: FP64 partial sums of
-// |f|^2, added in block order by the block that draws the last ticket (agent
-// scope: the blocks' XCDs have separate L2s), which leaves s = RMS and 1/s (0
-// for a zero field) in scale[0..1].  The host does not wait for it.
+// |f|^2, added by the block that draws the last ticket (agent scope: the
+// blocks' XCDs have separate L2s) or, without a ticket, by k_rms_total.  The host
+// does not wait for it.
 template <typename T>
 __global__ __launch_bounds__(NB) void k_rms(const cx<T>* f0, const cx<T>* f1, const cx<T>* f2, const cx<T>* f3, size_t n,
                                             double count, double* __restrict__ part, unsigned* __restrict__ ticket,
                                             double* __restrict__ scale) {
     __shared__ double red[NB];
     __shared__ bool last;
-    auto block_sum = [&](double s) {
-        red[threadIdx.x] = s;
-        __syncthreads();
-        for (int k = NB / 2; k > 0; k >>= 1) {
-            if (int(threadIdx.x) < k) red[threadIdx.x] += red[threadIdx.x + k];
-            __syncthreads();
-        }
-    };
     double s = 0;
     const cx<T>* fs[4] = {f0, f1, f2, f3};
     for (int k = 0; k < 4; ++k) {
@@ -271,24 +286,25 @@ __global__ __launch_bounds__(NB) void k_rms(const cx<T>* f0, const cx<T>* f1, co
             s += double(v.x) * double(v.x) + double(v.y) * double(v.y);
         }
     }
-    block_sum(s);
+    block_sum(red, s);
     if (threadIdx.x == 0) {
         __hip_atomic_store(part + blockIdx.x, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
+        last = ticket != nullptr &&
+               __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
     }
     __syncthreads();
     if (!last) return;  // block-uniform
-    s = 0;
-    for (unsigned b = threadIdx.x; b < gridDim.x; b += NB)
-        s += __hip_atomic_load(part + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    block_sum(s);
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-        const double rms = sqrt(red[0] / count);
-        scale[0] = rms;
-        scale[1] = rms > 0 ? 1.0 / rms : 0.0;
-    }
+    rms_total(red, part, gridDim.x, count, scale);
+    if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
 }
+static __global__ __launch_bounds__(NB) void k_rms_total(const double* part, unsigned blocks, double count, double* scale) {
+    __shared__ double red[NB];
+    rms_total(red, part, blocks, count, scale);
+}
+// Blocks up to which the last one adds the sums: a ticket is one atomic per block
+// on one address, which a second launch outweighs (an application, us, ticket / second
+// launch: 34 blocks 21.9 / 22.5, 85 blocks 28.7 / 27.9, 340 48.7 / 43.8, 1024 275 / 256)
+constexpr unsigned RMS_TICKET = 64;
 
 struct PackArgs {
     const void* f[4];  // present fields (null: absent), modal layout [ja][z][j1]
@@ -806,8 +822,12 @@ struct Net {
                 p[i] = static_cast<const cx<T>*>(f[i]->d);
                 ++nf_;
             }
-        hipLaunchKernelGGL((k_rms<T>), dim3(grid_for(n, 1024)), dim3(NB), 0, st(), p[0], p[1], p[2], p[3], n,
-                           double(n * size_t(nf_)), dpart, ticket, sc);
+        const unsigned blocks = grid_for(n, 1024);
+        const double count = double(n * size_t(nf_));
+        const bool one = blocks <= RMS_TICKET;
+        hipLaunchKernelGGL((k_rms<T>), dim3(blocks), dim3(NB), 0, st(), p[0], p[1], p[2], p[3], n, count, dpart,
+                           one ? ticket : nullptr, sc);
+        if (!one) hipLaunchKernelGGL(k_rms_total, dim3(1), dim3(NB), 0, st(), dpart, blocks, count, sc);
         SF_HIP(hipGetLastError());
     }
 

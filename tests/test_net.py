@@ -213,3 +213,12 @@ def test_parameters_take_their_turn():
             assert a is None or np.array_equal(a.download(), b.download())
     assert np.array_equal(net.get_params(), second)
     s.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,prec,hidden,layers", [((96, 1, 512, 1), 8, 64, 2), ((128, 1, 400, 1), 4, 32, 2),
+                                                      ((48, 24, 72, 0), 8, 32, 3)])
+def test_rms_on_both_sides_of_the_second_launch(shape, prec, hidden, layers):
+    """Up to 64 blocks the last one adds the sums of the RMS, of more (64, 66 and
+    68 blocks here) a second launch does."""
+    test_fused_application_matches_layers(shape, prec, hidden, layers)
