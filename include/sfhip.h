@@ -18,7 +18,11 @@
  *    modes (ModalField::ParallelPerStack, Field.h:1129-1166); uploading a
  *    modal array therefore applies ModalField::Filter (Field.h:996-1021).
  *  - One context owns one HIP stream; calls are stream-ordered and
- *    asynchronous except downloads, reductions and sf_synchronize.
+ *    asynchronous except downloads, sf_synchronize and calls that return a
+ *    number.  sf_inner_prod and sf_energy return when their result has arrived:
+ *    everything queued on the context before them has run, but the stream is
+ *    not waited for, so that a failure of an earlier asynchronous call may be
+ *    reported by a later one.
  */
 #ifndef SFHIP_H
 #define SFHIP_H
