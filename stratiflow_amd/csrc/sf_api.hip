@@ -1276,11 +1276,11 @@ struct Batch {
     // Arguments of the members and the table of their work items, count[m] of each.
     // Blocks go to the eight XCDs in turn: of every 64 items each XCD takes eight
     // consecutive ones, which are of one run as a rule and share its coefficients
-    // and the cache lines that two neighbouring tiles of modes have in common.  Per
-    // stage of 16 runs of 64..256 x 100..384 FP32 the modal launch (4 modes) takes
-    // 32 us with 1 item in turn, 27 with 4, 24 with 8, 25 with 12, and that of 64
-    // runs (8 modes) 59, 54, 55, 54; whole runs on an XCD are as good for 16
-    // runs and 10 us worse for 64, by their unequal lengths.  The x-pass is within 3%.
+    // and the cache lines that two neighbouring tiles of modes have in common.  The
+    // modal launch takes, us per stage with 1, 4, 8 and 12 items in turn: 16 runs of
+    // 64..256 x 96..384 FP32, 4 modes per block, 26.5, 23.7, 23.6, 22.8; 64 runs, 4 modes, 64,
+    // 55, 55, 55, and 8 modes, 52, 47, 45, 46.  Whole runs on an XCD are as good for 16 runs
+    // and 10 us worse for 64, by their unequal lengths.  The x-pass is within 3%.
     template <typename A>
     void upload_group(Group& g, const std::vector<A>& a, const std::vector<int>& count, int grid) {
         g.total = 0;
