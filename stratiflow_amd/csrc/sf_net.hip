@@ -302,9 +302,11 @@ static __global__ __launch_bounds__(NB) void k_rms_total(const double* part, uns
     rms_total(red, part, blocks, count, scale);
 }
 // Blocks up to which the last one adds the sums: a ticket is one atomic per block
-// on one address, which a second launch outweighs (an application, us, ticket / second
-// launch: 34 blocks 21.9 / 22.5, 85 blocks 28.7 / 27.9, 340 48.7 / 43.8, 1024 275 / 256)
-constexpr unsigned RMS_TICKET = 64;
+// on one address, a second launch is work for the host too.  An application, us,
+// ticket / second launch: one context, 34 blocks 21.9 / 22.5, 85 blocks 28.4 / 27.7,
+// 94 blocks 24.2 / 23.4, 340 48.5 / 43.6, 1024 275 / 256; two contexts in turn, 85 blocks
+// 17.8 / 18.1, 94 blocks 15.1 / 14.4, 170 22.2 / 19.7.  Above 90 both uses gain.
+constexpr unsigned RMS_TICKET = 90;
 
 struct PackArgs {
     const void* f[4];  // present fields (null: absent), modal layout [ja][z][j1]

@@ -216,9 +216,9 @@ def test_parameters_take_their_turn():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape,prec,hidden,layers", [((96, 1, 512, 1), 8, 64, 2), ((128, 1, 400, 1), 4, 32, 2),
-                                                      ((48, 24, 72, 0), 8, 32, 3)])
+@pytest.mark.parametrize("shape,prec,hidden,layers", [((192, 1, 360, 1), 8, 64, 2), ((192, 1, 364, 1), 4, 32, 2),
+                                                      ((48, 24, 100, 0), 8, 32, 3)])
 def test_rms_on_both_sides_of_the_second_launch(shape, prec, hidden, layers):
-    """Up to 64 blocks the last one adds the sums of the RMS, of more (64, 66 and
-    68 blocks here) a second launch does."""
+    """Up to 90 blocks the last one adds the sums of the RMS, of more (90, 91 and
+    94 blocks here) a second launch does."""
     test_fused_application_matches_layers(shape, prec, hidden, layers)
